@@ -88,7 +88,7 @@ typedef struct rt_tensor_desc {
                               NULL with row_len set (rt_step_multi only): the update kernel takes the row means
                               itself -- same summation, same bits as rt_row_means -- which saves the separate pass
                               over g; for whole tensors (elem_offset 0, numel a multiple of row_len) of 16-bit
-                              arrays, 16-byte aligned, Philox noise, no debug outputs, row_len a multiple of 8
+                              arrays, Philox noise, no debug outputs, row_len a multiple of 8
                               in [512, 32768]; RT_EINVAL otherwise */
     uint64_t numel;
     uint64_t elem_offset;  /* index of element 0 inside the logical tensor; multiple of 8 */

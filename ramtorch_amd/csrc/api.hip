@@ -250,9 +250,9 @@ static int dtype_size(int dt) { return dt == RT_DT_F32 ? 4 : dt == RT_DT_F64 ? 8
 using MultiKernel = void (*)(const LaunchArgs);
 
 struct KernelPair {
-    MultiKernel fast;     // whole fast units of aligned tensors, plus (16-bit layouts, Philox) their pieces
-    MultiKernel generic;  // unaligned tensors, debug outputs, leftovers without a piece path, rows shorter than 8
-    MultiKernel fast_cen; // whole fast units of aligned tensors with centralization (16-bit layouts, Philox), or NULL
+    MultiKernel fast;     // whole fast units, plus (16-bit layouts, Philox) their pieces
+    MultiKernel generic;  // debug outputs, leftovers without a piece path, rows shorter than 8
+    MultiKernel fast_cen; // whole fast units of tensors with centralization (16-bit layouts, Philox), or NULL
     MultiKernel rowwise;  // whole tensors with centralization whose row means the kernel takes itself (same layouts), or NULL
     MultiKernel rowwise_short;  // the same for rows of at most kRowwiseShortMax elements
 };
@@ -321,10 +321,9 @@ static inline uint32_t combo_of(const rt_tensor_desc& d) { return compiled_combo
 // Centralization with row_mean == NULL: whether the row-wise kernel can take this tensor
 // (see sr_adamw_rowwise_kernel).
 static inline bool rowwise_ok(const rt_tensor_desc& d, int noise_mode, bool allow_host) {
-    const uintptr_t all = (uintptr_t)d.p | (uintptr_t)d.g | (uintptr_t)d.m | (uintptr_t)d.v;
     return !allow_host && noise_mode == RT_NOISE_PHILOX && compiled_combo(d) && d.p_dtype != RT_DT_F32 &&
-           d.g_dtype != RT_DT_F32 && d.m_dtype != RT_DT_F32 && d.v_dtype != RT_DT_F32 && (all & 15u) == 0 &&
-           !d.dbg_p && !d.dbg_m && !d.dbg_v && d.elem_offset == 0 && d.row_len % kVec == 0 &&
+           d.g_dtype != RT_DT_F32 && d.m_dtype != RT_DT_F32 && d.v_dtype != RT_DT_F32 && !d.dbg_p && !d.dbg_m &&
+           !d.dbg_v && d.elem_offset == 0 && d.row_len % kVec == 0 &&
            d.row_len >= kRowwiseMinLen && d.row_len <= kWaveRowMax && d.numel % d.row_len == 0 &&
            d.numel / d.row_len <= kMaxGrid;
 }
@@ -374,7 +373,7 @@ static int validate(const rt_tensor_desc* descs, uint32_t n, const rt_scalars* s
             if (!d.row_mean && !rowwise_ok(d, noise_mode, allow_host))
                 return fail(RT_EINVAL,
                             "tensor %u: centralization without row_mean (the update takes the row means itself only "
-                            "for whole 16-byte-aligned device tensors of 16-bit arrays with Philox noise, rows a "
+                            "for whole device tensors of 16-bit arrays with Philox noise, rows a "
                             "multiple of 8 and %u .. %u elements long, no debug outputs)",
                             i, kRowwiseMinLen, kWaveRowMax);
         }
@@ -389,7 +388,7 @@ static int validate(const rt_tensor_desc* descs, uint32_t n, const rt_scalars* s
 // Lays out [DevScalars sets][DevTensor records][first units][their DevTensor records][PieceRef pieces][ChunkRef list]
 // in h->image.  Tensors are grouped by dtype combination so that each combination
 // is one contiguous range of every list = at most two launches.
-// Whole fast units of plain tensors (16-byte aligned, no debug output, no centralization) become
+// Whole fast units of plain tensors (no debug output, no centralization) become
 // ranges; what such a tensor leaves over becomes pieces where the layout has a piece path (all
 // arrays 16 bit, Philox noise), chunks of the generic kernel otherwise; every other tensor goes to
 // the generic kernel chunk by chunk.
@@ -435,8 +434,6 @@ static void build_image(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, c
         t.tensor_id4 = d.tensor_id * 4u;
         t.set_idx = it->second;
         t.dtypes = dtypes_of(d);
-        const uint64_t all = t.p | t.g | t.m | t.v | t.np | t.nm | t.nv;
-        t.flags = (all & 15u) == 0 ? kFlagAligned : 0u;
         if (sets[it->second].s.centralization != 0.0f && !d.row_mean) t.flags |= kFlagRowwise;   // validated: rowwise_ok
     }
 
@@ -462,7 +459,7 @@ static void build_image(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, c
         b.first_piece = (uint32_t)pieces.size();
         const bool has_pieces = !want_explicit && narrow_combo(combo);
         auto plain = [&](const DevTensor& t) {
-            return combo != kComboAny && (t.flags & kFlagAligned) && !(t.flags & kFlagRowwise) &&
+            return combo != kComboAny && !(t.flags & kFlagRowwise) &&
                    (t.dp | t.dm | t.dv | t.row_mean) == 0;
         };
         uint32_t units = 0;
@@ -497,7 +494,7 @@ static void build_image(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, c
         // kernel's centralizing variant (16-bit layouts with Philox noise have one), the rest of them
         // to the generic kernel.  A lane's 8 elements must lie in at most two rows.
         auto cen_plain = [&](const DevTensor& t) {
-            return has_pieces && (t.flags & kFlagAligned) && (t.dp | t.dm | t.dv) == 0 && t.row_mean != 0 &&
+            return has_pieces && (t.dp | t.dm | t.dv) == 0 && t.row_mean != 0 &&
                    t.row_len >= (uint64_t)kVec && t.row_len < (1ull << 31);
         };
         b.first_cen_range = (uint32_t)ranges.size();
@@ -915,8 +912,8 @@ int rt_step_multi(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, const r
 }
 
 // The gradient table of the norm pass: one NormEntry per non-empty gradient.  Chunks of 8192
-// elements are numbered in two sequences -- every whole chunk of the 16-byte aligned gradients
-// first, then all other chunks, each in tensor order -- and chunk c belongs to workgroup c mod grid.
+// elements are numbered in two sequences -- every whole chunk of the gradients
+// first, then the partial ones, each in tensor order -- and chunk c belongs to workgroup c mod grid.
 static int build_norm_table(const rt_tensor_desc* descs, uint32_t n, size_t max_entries, std::vector<NormEntry>& tab,
                             uint64_t& n_whole, uint64_t& n_rest) {
     tab.clear();
@@ -935,7 +932,7 @@ static int build_norm_table(const rt_tensor_desc* descs, uint32_t n, size_t max_
                         "rt_grad_norm_static takes at most %zu non-empty gradients per call (its table is a fixed "
                         "device array); use rt_grad_norm", max_entries);
         const uint64_t chunks = (d.numel + kChunkElems - 1) / kChunkElems;
-        const uint64_t whole = ((uintptr_t)d.g & 15u) == 0 ? d.numel / kChunkElems : 0;
+        const uint64_t whole = d.numel / kChunkElems;
         NormEntry e;
         e.g = (uint64_t)d.g;
         e.numel = d.numel;
@@ -1136,18 +1133,17 @@ int rt_sr_copy(void* target_bf16, const float* source, uint64_t numel, const voi
     if (((uintptr_t)target_bf16 & 1u) || ((uintptr_t)source & 3u) || ((uintptr_t)noise & 1u))
         return fail(RT_EINVAL, "pointer not aligned to its element size");
     hipStream_t stream = (hipStream_t)stream_;
-    const int aligned = ((((uintptr_t)target_bf16) | ((uintptr_t)source) | ((uintptr_t)noise)) & 15u) == 0;
     const uint64_t blocks = (numel + (uint64_t)kThreads * kVec - 1) / ((uint64_t)kThreads * kVec);
     // one block of 2048 elements per workgroup: a capped grid with a grid-stride loop ran 25 % slower
     const uint32_t grid = (uint32_t)std::min<uint64_t>(blocks, kMaxGrid);
     if (noise)
         hipLaunchKernelGGL(sr_copy_kernel<RT_NOISE_EXPLICIT>, dim3(grid), dim3(kThreads), 0, stream,
                            (uint64_t)target_bf16, (uint64_t)source, numel, (uint64_t)noise, (uint32_t)seed,
-                           (uint32_t)(seed >> 32), aligned);
+                           (uint32_t)(seed >> 32));
     else
         hipLaunchKernelGGL(sr_copy_kernel<RT_NOISE_PHILOX>, dim3(grid), dim3(kThreads), 0, stream,
                            (uint64_t)target_bf16, (uint64_t)source, numel, (uint64_t)0, (uint32_t)seed,
-                           (uint32_t)(seed >> 32), aligned);
+                           (uint32_t)(seed >> 32));
     HIP_TRY(hipGetLastError());
     return RT_OK;
 }

@@ -13,7 +13,6 @@ constexpr int kItersPerChunk = 4;                   // vectors per lane per chun
 constexpr uint32_t kChunkElems = kThreads * kVec * kItersPerChunk;  // 8192
 
 // DevTensor.flags
-constexpr uint32_t kFlagAligned = 1u;  // every array pointer of the tensor is 16-byte aligned
 constexpr uint32_t kFlagRowwise = 2u;  // centralization with the row means taken inside the update kernel (row_mean == 0)
 
 // One tensor (or contiguous piece) as the kernels see it; 128 bytes so that a

@@ -50,11 +50,20 @@ __device__ __forceinline__ uint32_t f2u(float f) { return __builtin_bit_cast(uin
 // nontemporal hint: lines are not kept in L2 (4 MB per XCD, far smaller than
 // what 256 CUs have in flight), which removed re-fetches of evicted lines and
 // measured ~10 % faster than plain accesses on the 8B-element set.
+//
+// Vectors need no alignment beyond that of one element (2 bytes): gfx950 runs in unaligned-access
+// mode, and the compiler emits the same single 128-bit instruction for a 2-byte-aligned vector as for
+// an aligned one.  Gradients that are views of a communication bucket, or parameters of a flat
+// buffer, lie at any element; a wave's 1 KB access then touches nine lines instead of eight.
+// Loading such tensors element by element instead cost a factor of three: 122 M bf16 elements whose
+// gradients lie one element off took 868 us (1.96 TB/s), as vectors 296 us (5.75 TB/s, the rate of the
+// same set with aligned gradients).
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
 __device__ __forceinline__ u32x4 ldg128(uint64_t addr) {
-    return __builtin_nontemporal_load((const RT_GLOBAL u32x4*)addr);
+    return __builtin_nontemporal_load((const RT_GLOBAL u32x4_any*)addr);
 }
 __device__ __forceinline__ void stg128(uint64_t addr, u32x4 v) {
-    __builtin_nontemporal_store(v, (RT_GLOBAL u32x4*)addr);
+    __builtin_nontemporal_store(v, (RT_GLOBAL u32x4_any*)addr);
 }
 __device__ __forceinline__ uint32_t ldg16(uint64_t addr) { return *(const RT_GLOBAL uint16_t*)addr; }
 __device__ __forceinline__ void stg16(uint64_t addr, uint32_t v) { *(RT_GLOBAL uint16_t*)addr = (uint16_t)v; }
@@ -115,7 +124,7 @@ __device__ __forceinline__ Raw8<DT> load_raw(uint64_t base, uint64_t i) {
     return r;
 }
 
-// Per-element load for tails and unaligned tensors: elements at or past n read as 0.
+// Per-element load for tails: elements at or past n read as 0.
 template <int DT>
 __device__ __forceinline__ Raw8<DT> load_raw_guarded(uint64_t base, uint64_t i, uint64_t n) {
     Raw8<DT> r;
@@ -438,7 +447,7 @@ __device__ __forceinline__ void piece_body(const LaunchArgs& a, uint32_t q) {
 
 // ---------------------------------------------------------------------------
 // Fast kernel, all arrays 16 bit wide.  One launch covers everything that needs
-// no special care in 16-byte aligned tensors:
+// no special care:
 //  * n_piece_wgs workgroups serve four pieces each, one per wavefront (Philox
 //    mode only);
 //  * the other workgroups serve one unit of kFastUnitElems elements each, lying
@@ -588,11 +597,12 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_fast_kernel(const LaunchArg
 // neighbour swap (DPP quad_perm), so the Philox count per element is unchanged.
 // ---------------------------------------------------------------------------
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef u32x2 u32x2_any __attribute__((aligned(2)));
 __device__ __forceinline__ u32x2 ldg64(uint64_t addr) {
-    return __builtin_nontemporal_load((const RT_GLOBAL u32x2*)addr);
+    return __builtin_nontemporal_load((const RT_GLOBAL u32x2_any*)addr);
 }
 __device__ __forceinline__ void stg64(uint64_t addr, u32x2 v) {
-    __builtin_nontemporal_store(v, (RT_GLOBAL u32x2*)addr);
+    __builtin_nontemporal_store(v, (RT_GLOBAL u32x2_any*)addr);
 }
 __device__ __forceinline__ uint32_t swap_neighbour(uint32_t x) {  // value of lane ^ 1
     return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xB1 /* quad_perm [1,0,3,2] */, 0xF, 0xF, false);
@@ -738,10 +748,9 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_fast_wide_kernel(const Laun
 }
 
 // ---------------------------------------------------------------------------
-// Generic kernel: the last (partial) chunk of a tensor, tensors whose pointers
-// are not 16-byte aligned, debug outputs, gradient centralization.  Full
-// aligned vectors still move as 128-bit accesses; everything else element by
-// element under an index guard.
+// Generic kernel: the last (partial) chunk of a tensor, debug outputs, gradient
+// centralization.  Full vectors still move as 128-bit accesses; everything else
+// element by element under an index guard.
 // ---------------------------------------------------------------------------
 template <int PDT, int GDT, int MDT, int VDT, int NOISE>
 __global__ __launch_bounds__(kThreads) void sr_adamw_generic_kernel(const LaunchArgs a) {
@@ -753,12 +762,11 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_generic_kernel(const Launch
 
     const uint64_t n = t.numel;
     const uint64_t chunk_base = (uint64_t)cr.chunk * kChunkElems;
-    const bool aligned = (t.flags & kFlagAligned) != 0u;
 #pragma unroll 1
     for (int it = 0; it < kItersPerChunk; ++it) {
         const uint64_t i = chunk_base + (uint64_t)(it * kThreads + (int)threadIdx.x) * kVec;
         if (i >= n) break;
-        const bool full = aligned && (i + kVec <= n);
+        const bool full = i + kVec <= n;
         Raw8<PDT> rp; Raw8<GDT> rg; Raw8<MDT> rm; Raw8<VDT> rv;
         u32x4 zp = 0, zm = 0, zv = 0;
         if (full) {
@@ -827,8 +835,8 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_generic_kernel(const Launch
 // fp64 input is rounded to nearest even on the way in.  Such layouts are rare,
 // so this is one kernel with a per-tensor dtype switch instead of another 200
 // instantiations: a lane owns one Philox block of 8 elements, as in the
-// kernels above, and moves them as 128-bit accesses where the tensor is plain
-// and aligned, element by element otherwise.  The four accesses a lane makes
+// kernels above, and moves them as 128-bit accesses where the tensor is plain,
+// element by element otherwise.  The four accesses a lane makes
 // to an fp64 array are ordinary cached ones: with the nontemporal hint every
 // one of them fetched its 128-byte line from the L2 again (1.5 TB/s instead of
 // 4.9 TB/s for an all-fp64 layout).
@@ -856,7 +864,7 @@ __device__ __forceinline__ uint32_t noise_field(const u32x4& z, int j) {
     return (j & 1) ? (w >> 16) : (w & 0xFFFFu);
 }
 
-// Eight consecutive elements of a 16-byte-aligned array as fp32, by 128-bit accesses, with the
+// Eight consecutive elements of an array as fp32, by 128-bit accesses, with the
 // dtype known only at run time (it is the same for the whole wave, so the switch is a scalar
 // branch).  fp64 takes four accesses of two doubles each; the conversions are the ones load_any /
 // store_any make element by element.
@@ -868,7 +876,7 @@ __device__ __forceinline__ void load8_any(uint64_t base, uint32_t dt, uint64_t i
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 // ordinary (cached) accesses: a lane's four accesses fall into one 64-byte half line
-                const u32x4 w = *(const RT_GLOBAL u32x4*)(base + i * 8 + (uint64_t)k * 16);
+                const u32x4 w = *(const RT_GLOBAL u32x4_any*)(base + i * 8 + (uint64_t)k * 16);
                 x[2 * k] = (float)__builtin_bit_cast(double, (uint64_t)w.x | ((uint64_t)w.y << 32));
                 x[2 * k + 1] = (float)__builtin_bit_cast(double, (uint64_t)w.z | ((uint64_t)w.w << 32));
             }
@@ -888,7 +896,7 @@ __device__ __forceinline__ void store8_any(uint64_t base, uint32_t dt, uint64_t 
                 const uint64_t hi = __builtin_bit_cast(uint64_t, (double)x[2 * k + 1]);
                 u32x4 w;
                 w.x = (uint32_t)lo; w.y = (uint32_t)(lo >> 32); w.z = (uint32_t)hi; w.w = (uint32_t)(hi >> 32);
-                *(RT_GLOBAL u32x4*)(base + i * 8 + (uint64_t)k * 16) = w;
+                *(RT_GLOBAL u32x4_any*)(base + i * 8 + (uint64_t)k * 16) = w;
             }
             break;
         default: store_out<RT_DT_F32>(base, i, x, noise); break;
@@ -896,7 +904,7 @@ __device__ __forceinline__ void store8_any(uint64_t base, uint32_t dt, uint64_t 
 }
 
 // The same for a whole wavefront at once, for the two wide dtypes: the wave's 512 consecutive
-// elements start at element w0 of a 16-byte-aligned array, and every instruction moves one contiguous
+// elements start at element w0 of the array, and every instruction moves one contiguous
 // kilobyte (lane l takes the 16 bytes at l * 16 of the k-th kilobyte) instead of 16 bytes out of
 // every 32 (fp32) or 64 (fp64) per lane.  The values change hands through `stage`, 512 floats of
 // shared memory that belong to this wave alone: written in array order, read back as each lane's own
@@ -976,7 +984,7 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_any_kernel(const LaunchArgs
                    vdt = (t.dtypes >> 6) & 3u;
     const uint64_t n = t.numel;
     const uint64_t chunk_base = (uint64_t)cr.chunk * kChunkElems;
-    const bool plain = (t.flags & kFlagAligned) != 0u && (t.dp | t.dm | t.dv | t.row_mean) == 0;
+    const bool plain = (t.dp | t.dm | t.dv | t.row_mean) == 0;
     __shared__ __attribute__((aligned(16))) float stage_all[kThreads / 64][64 * kVec];
 #pragma unroll 1
     for (int it = 0; it < kItersPerChunk; ++it) {
@@ -1024,8 +1032,8 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_any_kernel(const LaunchArgs
             store8(t.v, vdt, v, zv);
             continue;
         }
-        // Whole vectors of plain aligned tensors move as 128-bit accesses, like everywhere else;
-        // tails, unaligned views, debug outputs and centralization go element by element below.
+        // Whole vectors of plain tensors move as 128-bit accesses, like everywhere else; tails, debug
+        // outputs and centralization go element by element below.
         if (plain && i + kVec <= n) {
             if constexpr (NOISE == RT_NOISE_EXPLICIT) {
                 if (pdt == RT_DT_BF16) zp = ldg128(t.np + i * 2);
@@ -1143,12 +1151,11 @@ __global__ __launch_bounds__(kThreads) void stream_probe_kernel(uint64_t p, uint
 // ---------------------------------------------------------------------------
 template <int NOISE>
 __global__ __launch_bounds__(kThreads) void sr_copy_kernel(uint64_t target, uint64_t source, uint64_t n,
-                                                           uint64_t noise, uint32_t seed_lo, uint32_t seed_hi,
-                                                           int aligned) {
-    // Whole blocks of 2048 elements of aligned arrays use the lane mapping of the wide update
+                                                           uint64_t noise, uint32_t seed_lo, uint32_t seed_hi) {
+    // Whole blocks of 2048 elements use the lane mapping of the wide update
     // kernel (a lane owns 4 + 4 elements of its wave's 512-element block, so the fp32 loads are
     // contiguous kilobytes across the wave) and the same neighbour swap of Philox halves; the last
-    // partial block and unaligned arrays go element by element under an index guard.
+    // partial block goes element by element under an index guard.
     constexpr uint64_t kBlock = (uint64_t)kThreads * kVec;
     constexpr uint32_t kHalf = 64 * kVec / 2;
     const uint64_t n_blocks = (n + kBlock - 1) / kBlock;
@@ -1156,7 +1163,7 @@ __global__ __launch_bounds__(kThreads) void sr_copy_kernel(uint64_t target, uint
     const bool odd = (lane & 1u) != 0u;
     for (uint64_t b = blockIdx.x; b < n_blocks; b += gridDim.x) {
         const uint64_t base = b * kBlock;
-        if (aligned && base + kBlock <= n) {
+        if (base + kBlock <= n) {
             const uint64_t blk = base + (uint64_t)wave * (64 * kVec);
             u32x4 raw[2];
             u32x2 z[2];
@@ -1242,7 +1249,7 @@ __device__ __forceinline__ float block_sum(float x, float* lds) {
 }
 
 // Sum of squares of one chunk of one gradient tensor (per-lane partial).
-// Whole chunk of an aligned gradient: every load is 16 bytes per lane and contiguous across the
+// Whole chunk: every load is 16 bytes per lane and contiguous across the
 // wave whatever the element type (a sum does not care which lane gets which element), all loads
 // of the chunk are in flight together.
 template <int GDT>
@@ -1280,14 +1287,13 @@ __device__ __forceinline__ float chunk_sumsq_full(uint64_t g_addr, uint32_t chun
 template <int GDT>
 __device__ __forceinline__ float chunk_sumsq(uint64_t g_addr, uint64_t n, uint32_t chunk, float inv_loss_scale) {
     const uint64_t chunk_base = (uint64_t)chunk * kChunkElems;
-    const bool aligned = (g_addr & 15u) == 0;
-    if (aligned && chunk_base + kChunkElems <= n) return chunk_sumsq_full<GDT>(g_addr, chunk, inv_loss_scale);
+    if (chunk_base + kChunkElems <= n) return chunk_sumsq_full<GDT>(g_addr, chunk, inv_loss_scale);
     float acc = 0.0f;
 #pragma unroll 1
     for (int it = 0; it < kItersPerChunk; ++it) {
         const uint64_t i = chunk_base + (uint64_t)(it * kThreads + (int)threadIdx.x) * kVec;
         if (i >= n) break;
-        const bool full = aligned && (i + kVec <= n);
+        const bool full = i + kVec <= n;
         const Raw8<GDT> r = full ? load_raw<GDT>(g_addr, i) : load_raw_guarded<GDT>(g_addr, i, n);
         float g[8];
         decode<GDT>(r, g);
@@ -1313,7 +1319,7 @@ __device__ __forceinline__ float chunk_sumsq_dt(int dt, uint64_t g_addr, uint64_
 // is one NormEntry per gradient (small enough to live in a fixed device array
 // for the entry point that allocates nothing); a chunk finds its gradient by
 // binary search.  Chunks are numbered in two sequences -- first every whole
-// chunk of the 16-byte aligned gradients, then everything else, each in tensor
+// chunk of the gradients, then the partial ones, each in tensor
 // order -- so that most workgroups see nothing but whole chunks.
 // ---------------------------------------------------------------------------
 struct alignas(16) NormEntry {
@@ -1420,17 +1426,16 @@ __device__ __forceinline__ float load_elem(uint64_t base, uint64_t idx) {
 }
 
 // Sum of row [base, base + row_len) of g by the calling wavefront; the result is in every lane.
-// A row that starts on a 16-byte boundary (every row of a matrix whose rows are a multiple of 8
-// elements long) moves as whole vectors, 32 registers of them in flight per lane, and at most 7
-// single elements at its end; any other row goes element by element.
+// A row moves as whole vectors, 32 registers of them in flight per lane, and at most 7 single
+// elements at its end.
 // KEEP: the row is read again right away (by the update that takes its own row means), so its
 // lines are loaded the ordinary way and stay in the L2; the values and their order are the same.
 template <int DT>
 __device__ __forceinline__ Raw8<DT> load_raw_cached(uint64_t base, uint64_t i) {
     Raw8<DT> r;
     const uint64_t addr = base + i * esize<DT>();
-    r.a = *(const RT_GLOBAL u32x4*)addr;
-    if constexpr (DT == RT_DT_F32) r.b = *(const RT_GLOBAL u32x4*)(addr + 16);
+    r.a = *(const RT_GLOBAL u32x4_any*)addr;
+    if constexpr (DT == RT_DT_F32) r.b = *(const RT_GLOBAL u32x4_any*)(addr + 16);
     return r;
 }
 
@@ -1439,27 +1444,23 @@ __device__ __forceinline__ float row_sum_wave(uint64_t g, uint64_t base, uint32_
     constexpr int kB = GDT == RT_DT_F32 ? kRowVecs / 2 : kRowVecs;   // an fp32 vector of 8 elements is two loads
     const uint32_t lane = threadIdx.x & 63u;
     float acc = 0.0f;
-    if (((g + base * esize<GDT>()) & 15u) == 0) {
-        const uint32_t n_vec = row_len / kVec;
-        for (uint32_t v0 = 0; v0 < n_vec; v0 += 64u * kB) {
-            Raw8<GDT> r[kB];
+    const uint32_t n_vec = row_len / kVec;
+    for (uint32_t v0 = 0; v0 < n_vec; v0 += 64u * kB) {
+        Raw8<GDT> r[kB];
 #pragma unroll
-            for (int k = 0; k < kB; ++k) {
-                const uint32_t v = v0 + (uint32_t)k * 64u + lane;
-                if (v < n_vec)
-                    r[k] = KEEP ? load_raw_cached<GDT>(g, base + (uint64_t)v * kVec) : load_raw<GDT>(g, base + (uint64_t)v * kVec);
-            }
-#pragma unroll
-            for (int k = 0; k < kB; ++k) {
-                const uint32_t v = v0 + (uint32_t)k * 64u + lane;
-                if (v < n_vec) acc = add_vec<GDT>(acc, r[k], inv_loss_scale);
-            }
+        for (int k = 0; k < kB; ++k) {
+            const uint32_t v = v0 + (uint32_t)k * 64u + lane;
+            if (v < n_vec)
+                r[k] = KEEP ? load_raw_cached<GDT>(g, base + (uint64_t)v * kVec) : load_raw<GDT>(g, base + (uint64_t)v * kVec);
         }
-        const uint32_t t = n_vec * kVec + lane;
-        if (t < row_len) acc = acc + load_elem<GDT>(g, base + t) * inv_loss_scale;
-    } else {
-        for (uint32_t e = lane; e < row_len; e += 64u) acc = acc + load_elem<GDT>(g, base + e) * inv_loss_scale;
+#pragma unroll
+        for (int k = 0; k < kB; ++k) {
+            const uint32_t v = v0 + (uint32_t)k * 64u + lane;
+            if (v < n_vec) acc = add_vec<GDT>(acc, r[k], inv_loss_scale);
+        }
     }
+    const uint32_t t = n_vec * kVec + lane;
+    if (t < row_len) acc = acc + load_elem<GDT>(g, base + t) * inv_loss_scale;
     return wave_sum(acc);
 }
 
@@ -1468,7 +1469,6 @@ template <int GDT>
 __device__ __forceinline__ float row_sum_block(uint64_t g, uint64_t base, uint64_t row_len, float inv_loss_scale,
                                                float* lds) {
     constexpr int kInFlight = 4;
-    const bool aligned = ((g + base * esize<GDT>()) & 15u) == 0;
     float acc = 0.0f;
     for (uint64_t c0 = 0; c0 < row_len; c0 += (uint64_t)kThreads * kVec * kInFlight) {
         Raw8<GDT> r[kInFlight];
@@ -1476,7 +1476,7 @@ __device__ __forceinline__ float row_sum_block(uint64_t g, uint64_t base, uint64
         for (int k = 0; k < kInFlight; ++k) {
             const uint64_t e = c0 + ((uint64_t)k * kThreads + threadIdx.x) * kVec;
             if (e < row_len)
-                r[k] = (aligned && e + kVec <= row_len) ? load_raw<GDT>(g, base + e)
+                r[k] = (e + kVec <= row_len) ? load_raw<GDT>(g, base + e)
                                                         : load_raw_guarded<GDT>(g, base + e, base + row_len);
         }
 #pragma unroll
@@ -1566,7 +1566,7 @@ __global__ __launch_bounds__(kThreads) void row_mean_table_long_kernel(const uin
 // at a time with all their loads issued first, as the fast kernel does.  The gradient is read twice,
 // but the second time out of the L2 it was loaded into a few microseconds before: the separate
 // row-mean pass (2 bytes per element more from HBM, one launch more) is not needed for such tensors.
-// For whole 16-byte-aligned tensors of 16-bit arrays with Philox noise whose rows are a multiple of 8
+// For whole tensors of 16-bit arrays with Philox noise whose rows are a multiple of 8
 // and between 512 and kWaveRowMax elements long -- every matrix of a transformer; the host sends
 // everything else through precomputed means.  `first` lists every tensor's first row number in the
 // launch (ascending), `fast_tensors` its record at the same index; workgroup b takes rows 4b .. 4b+3.

@@ -1,0 +1,84 @@
+"""The update kernels at the edges of their work split: arrays that begin at any element, lengths around
+units, pieces and rows.  Everything bit for bit against the oracle, and nothing outside the arrays may change.
+Needs an MI355X: run with ``-m gpu``.
+"""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from ramtorch_amd import _native as N
+from ramtorch_amd import functional as F
+
+pytestmark = pytest.mark.gpu
+
+HP0 = dict(lr=1e-4, betas=(0.9, 0.999), eps=1e-8, weight_decay=0.01)
+_TORCH = {oracle.DT_BF16: torch.bfloat16, oracle.DT_F16: torch.float16, oracle.DT_F32: torch.float32,
+          oracle.DT_F64: torch.float64}
+_GUARD = 37   # elements of 0xA5 bytes on either side of every array
+
+
+@pytest.fixture(scope="module")
+def handle():
+    assert torch.cuda.is_available(), "these tests need the GPU"
+    h = N.Handle(0)
+    yield h
+    torch.cuda.synchronize()
+    h.close()
+
+
+def bits(t):
+    t = t.detach().cpu().contiguous()
+    return t.view({2: torch.int16, 4: torch.int32, 8: torch.int64}[t.element_size()]).numpy().ravel()
+
+
+def guarded(a, code, shift):
+    """``a`` on the GPU, ``shift`` elements past a 512-byte boundary, between guard bytes."""
+    dt = _TORCH[code]
+    values = torch.from_numpy((a.view(np.int16) if a.dtype == np.uint16 else a).copy())
+    values = values.view(dt) if values.dtype == torch.int16 else values
+    whole = torch.empty(256 + shift + a.size + _GUARD, dtype=dt, device="cuda")
+    whole.view(torch.uint8).fill_(0xA5)
+    view = whole[256 + shift:256 + shift + a.size]
+    view.copy_(values)
+    return view, whole
+
+
+def check_guards(whole, shift, n):
+    b = whole.view(torch.uint8)
+    es = whole.element_size()
+    assert bool((b[:(256 + shift) * es] == 0xA5).all()) and bool((b[(256 + shift + n) * es:] == 0xA5).all())
+
+
+_MIX = {"bf16": (0, 0, 0, 0), "f16": (2, 2, 2, 2), "bf16_f32grad_f32v": (0, 1, 0, 1), "f32_bf16states": (1, 1, 0, 0),
+        "f64states": (0, 0, 3, 3)}
+
+
+@pytest.mark.parametrize("mix", list(_MIX))
+@pytest.mark.parametrize("shifts", [(0, 1, 0, 0), (3, 7, 5, 1), (4, 4, 4, 4)])
+def test_arrays_may_begin_at_any_element(handle, mix, shifts):
+    """Views of a bucket or of a flat buffer: p, g, m and v each begin at an element of their own.  Lengths
+    around one and several units of 8192 elements, around pieces of 512 and vectors of 8."""
+    codes = _MIX[mix]
+    lengths = [1, 7, 8, 9, 511, 513, 2048, 8191, 8192, 8193, 3 * 8192 + 515]
+    tensors = []
+    for k, n in enumerate(lengths):
+        arrays = oracle.synth_inputs(n, 50 + k)
+        as_code = [a if c == 0 else oracle.bf16_to_f32(a).astype(
+            {1: np.float32, 2: np.float16, 3: np.float64}[c]) for a, c in zip(arrays, codes)]
+        as_code = [a.view(np.uint16) if a.dtype == np.float16 else a for a in as_code]
+        tensors.append((n, as_code, [guarded(a, c, s) for a, c, s in zip(as_code, codes, shifts)]))
+    entries = [F.Entry(p=v[0][0], g=v[1][0], m=v[2][0], v=v[3][0], step=10, scalars_idx=0, tensor_id=k)
+               for k, (_, _, v) in enumerate(tensors)]
+    F.step_resident(handle, entries, [F.make_scalars(step=10, **HP0)], seed=77, explicit_noise=False)
+    torch.cuda.synchronize()
+    sc = oracle.scalars_from_hparams(step=10, **HP0)
+    for k, (n, a, views) in enumerate(tensors):
+        po, mo, vo = a[0].copy(), a[2].copy(), a[3].copy()
+        oracle.step_tensor(po, a[1], mo, vo, sc, p_dtype=codes[0], g_dtype=codes[1], m_dtype=codes[2], v_dtype=codes[3],
+                           seed=77, step=10, tensor_id=k)
+        for name, got, want in zip("pmv", (views[0], views[2], views[3]), (po, mo, vo)):
+            w = want.view({2: np.int16, 4: np.int32, 8: np.int64}[want.dtype.itemsize])
+            np.testing.assert_array_equal(bits(got[0]), w, err_msg=f"{mix} n={n} {name}")
+        for (view, whole), s in zip(views, shifts):
+            check_guards(whole, s, n)
