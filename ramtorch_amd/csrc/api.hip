@@ -134,21 +134,27 @@ struct Streamed {
 // ---------------------------------------------------------------------------
 namespace {
 
+// Tensors that one launch of one kernel serves: consecutive records of the image, those with whole units
+// (row-wise kernel: all of them) first.
+struct Group {
+    uint32_t first_tensor, n_ranges;     // records from `first_tensor` on; the first n_ranges have an entry in the list of first units / rows
+    uint32_t n_units;                    // units (row-wise kernel: rows)
+    uint32_t first_piece, n_pieces;
+};
+
 struct Batch {            // tensors of one dtype combination inside a table image
     uint32_t combo;
-    uint32_t first_range, n_ranges, n_units;   // fast kernel: entries of the range list, fast units
-    uint32_t first_piece, n_pieces;            // pieces served by the fast kernel's first workgroups
-    uint32_t first_generic, n_generic;         // chunk range of the generic kernel
-    uint32_t first_cen_range, n_cen_ranges, n_cen_units;  // the same lists for tensors with centralization
-    // tensors whose row means the kernel takes itself, as lists of first rows: [0] rows longer than
-    // kRowwiseShortMax elements, [1] the others
-    uint32_t first_rw_range[2], n_rw_ranges[2], n_rw_rows[2];
+    Group plain;          // fast kernel
+    Group cen;            // fast kernel, gradients centralized by row means that were computed before
+    Group rowwise[2];     // centralization with the row means taken inside: [0] rows longer than kRowwiseShortMax, [1] the others
+    uint32_t first_tensor;
+    uint32_t first_generic, n_generic;   // chunk range of the generic (or runtime-typed) kernel
 };
 
 struct Plan {
-    size_t off_sets = 0, off_tensors = 0, off_ranges = 0, off_fast_tensors = 0, off_pieces = 0, off_chunks = 0,
-           bytes = 0;
-    uint32_t n_sets = 0, n_tensors = 0, n_chunks = 0;
+    size_t off_sets = 0, off_tensors = 0, off_extras = 0, off_first = 0, off_piece_tensor = 0, off_chunks = 0, bytes = 0;
+    uint32_t n_sets = 0, n_tensors = 0;
+    bool has_extras = false;
     DevScalars first_set;   // passed by value when n_sets == 1
     std::vector<Batch> batches;
     std::vector<std::pair<uint32_t, uint32_t>> set_keys;  // set index -> (scalars_idx, step)
@@ -156,7 +162,7 @@ struct Plan {
 
 inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
-// All arrays 16 bit wide: the layouts whose fast kernel has a piece path.
+// All arrays 16 bit wide.
 inline bool narrow_combo(uint32_t combo) {
     if (combo & 0x100u) return false;
     for (int k = 0; k < 4; ++k)
@@ -210,11 +216,9 @@ struct rt_handle {
         Plan plan;
     } layout;
     uint64_t layout_gen = 0;
-    std::vector<uint8_t> image;  // scratch for building a table image
-    std::vector<DevTensor> tens;
-    std::vector<uint32_t> ranges;       // first unit of each tensor of the fast kernel
-    std::vector<DevTensor> fast_tens;   // their records
-    std::vector<PieceRef> pieces;
+    std::vector<uint8_t> image;      // scratch for building a table image
+    std::vector<uint32_t> order, set_of;   // build_image: tensors in the order of the image's records, their sets
+    std::vector<uint8_t> kind;
     std::vector<ChunkRef> chunks;
     bool timing = false;
     // Timing: a ring of event pairs, one pair per timed launch, so that the launches of a whole
@@ -250,9 +254,9 @@ static int dtype_size(int dt) { return dt == RT_DT_F32 ? 4 : dt == RT_DT_F64 ? 8
 using MultiKernel = void (*)(const LaunchArgs);
 
 struct KernelPair {
-    MultiKernel fast;     // whole fast units, plus (16-bit layouts, Philox) their pieces
-    MultiKernel generic;  // debug outputs, leftovers without a piece path, rows shorter than 8
-    MultiKernel fast_cen; // whole fast units of tensors with centralization (16-bit layouts, Philox), or NULL
+    MultiKernel fast;     // whole fast units, plus (Philox) pieces
+    MultiKernel generic;  // debug outputs, leftovers of explicit-noise tensors, rows shorter than 8
+    MultiKernel fast_cen; // the same with centralization (16-bit layouts, Philox), or NULL
     MultiKernel rowwise;  // whole tensors with centralization whose row means the kernel takes itself (same layouts), or NULL
     MultiKernel rowwise_short;  // the same for rows of at most kRowwiseShortMax elements
 };
@@ -385,180 +389,188 @@ static int validate(const rt_tensor_desc* descs, uint32_t n, const rt_scalars* s
 // table building and launch
 // ---------------------------------------------------------------------------
 
-// Lays out [DevScalars sets][DevTensor records][first units][their DevTensor records][PieceRef pieces][ChunkRef list]
-// in h->image.  Tensors are grouped by dtype combination so that each combination
-// is one contiguous range of every list = at most two launches.
-// Whole fast units of plain tensors (no debug output, no centralization) become
-// ranges; what such a tensor leaves over becomes pieces where the layout has a piece path (all
-// arrays 16 bit, Philox noise), chunks of the generic kernel otherwise; every other tensor goes to
-// the generic kernel chunk by chunk.
+// Lays out [DevScalars sets][TensorRec records][TensorExtra records][first units / rows][tensor of each
+// piece][ChunkRef list] in `image`.  Tensors are grouped by dtype combination, and within a combination by
+// the kernel that serves them, so that every launch works on consecutive records.
+// Whole fast units of tensors without debug output become units, what such a tensor leaves over becomes
+// pieces (Philox noise; with explicit noise chunks of the generic kernel); tensors whose row means the
+// update takes itself go to the row-wise kernel; everything else goes to the generic kernel chunk by chunk.
+// One pass classifies the tensors, one writes the records where they belong.
 static void build_image(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, const rt_scalars* scalars,
-                        bool want_explicit, Plan& plan) {
-    // (scalars_idx, step) -> set index
-    std::map<std::pair<uint32_t, uint32_t>, uint32_t> set_of;
+                        bool want_explicit, Plan& plan, std::vector<uint8_t>& image) {
+    enum Kind : uint8_t { kUnits, kPieces, kCenUnits, kCenPieces, kRowLong, kRowShort, kGeneric, kKinds };
+    constexpr uint64_t unit = kFastUnitElems;
+    static_assert(kFastUnitElems == kChunkElems, "what a tensor's units leave over is its last chunk");
+    std::map<std::pair<uint32_t, uint32_t>, uint32_t> set_index;   // (scalars_idx, step) -> set index
     std::vector<DevScalars> sets;
-    std::vector<uint32_t> order;
-    order.reserve(n);
+    std::vector<uint32_t>& order = h->order;
+    order.clear();
     for (uint32_t i = 0; i < n; ++i)
         if (descs[i].numel != 0) order.push_back(i);
-    const auto by_combo = [&](uint32_t a, uint32_t b) { return combo_of(descs[a]) < combo_of(descs[b]); };
+    const auto by_combo = [&](uint32_t x, uint32_t y) { return combo_of(descs[x]) < combo_of(descs[y]); };
     if (!std::is_sorted(order.begin(), order.end(), by_combo))  // one combination is the common case
         std::stable_sort(order.begin(), order.end(), by_combo);
+    const size_t count = order.size();
 
-    std::vector<DevTensor>& tens = h->tens;
-    tens.resize(order.size());
-    auto it = set_of.end();
-    for (size_t k = 0; k < order.size(); ++k) {
-        const rt_tensor_desc& d = descs[order[k]];
-        auto key = std::make_pair(d.scalars_idx, d.step);
-        if (it == set_of.end() || it->first != key) it = set_of.find(key);  // neighbours mostly share a set
-        if (it == set_of.end()) {
-            DevScalars ds;
-            memset(&ds, 0, sizeof(ds));
-            ds.s = scalars[d.scalars_idx];
-            ds.step = d.step;
-            it = set_of.emplace(key, (uint32_t)sets.size()).first;
-            sets.push_back(ds);
-        }
-        DevTensor& t = tens[k];
-        memset(&t, 0, sizeof(t));
-        t.p = (uint64_t)d.p; t.g = (uint64_t)d.g; t.m = (uint64_t)d.m; t.v = (uint64_t)d.v;
-        if (want_explicit) {
-            t.np = (uint64_t)d.noise_p; t.nm = (uint64_t)d.noise_m; t.nv = (uint64_t)d.noise_v;
-        }
-        t.dp = (uint64_t)d.dbg_p; t.dm = (uint64_t)d.dbg_m; t.dv = (uint64_t)d.dbg_v;
-        t.row_mean = sets[it->second].s.centralization != 0.0f ? (uint64_t)d.row_mean : 0;
-        t.numel = d.numel;
-        t.block_base = d.elem_offset >> 3;
-        t.row_len = d.row_len ? d.row_len : 1;
-        t.tensor_id4 = d.tensor_id * 4u;
-        t.set_idx = it->second;
-        t.dtypes = dtypes_of(d);
-        if (sets[it->second].s.centralization != 0.0f && !d.row_mean) t.flags |= kFlagRowwise;   // validated: rowwise_ok
-    }
-
-    // ---- work lists, combination by combination
-    std::vector<uint32_t>& ranges = h->ranges;
-    std::vector<DevTensor>& fast_tens = h->fast_tens;
-    std::vector<PieceRef>& pieces = h->pieces;
+    std::vector<uint32_t>& set_of = h->set_of;
+    std::vector<uint8_t>& kind = h->kind;
     std::vector<ChunkRef>& chunks = h->chunks;
-    ranges.clear();
-    fast_tens.clear();
-    pieces.clear();
+    set_of.resize(count);
+    kind.resize(count);
     chunks.clear();
     plan.batches.clear();
-    constexpr uint64_t unit = kFastUnitElems;
-    size_t k0 = 0;
-    while (k0 < order.size()) {
+    plan.has_extras = false;
+    uint64_t pieces_total = 0;
+    auto it = set_index.end();
+    for (size_t k0 = 0; k0 < count;) {
         const uint32_t combo = combo_of(descs[order[k0]]);
+        const bool templated = combo != kComboAny, cen_kernel = narrow_combo(combo) && !want_explicit;
+        uint32_t in_kind[kKinds] = {};
         size_t k1 = k0;
-        while (k1 < order.size() && combo_of(descs[order[k1]]) == combo) ++k1;
+        for (; k1 < count && combo_of(descs[order[k1]]) == combo; ++k1) {
+            const rt_tensor_desc& d = descs[order[k1]];
+            const auto key = std::make_pair(d.scalars_idx, d.step);
+            if (it == set_index.end() || it->first != key) it = set_index.find(key);  // neighbours mostly share a set
+            if (it == set_index.end()) {
+                DevScalars ds;
+                memset(&ds, 0, sizeof(ds));
+                ds.s = scalars[d.scalars_idx];
+                ds.step = d.step;
+                it = set_index.emplace(key, (uint32_t)sets.size()).first;
+                sets.push_back(ds);
+            }
+            set_of[k1] = it->second;
+            const bool cen = sets[it->second].s.centralization != 0.0f, debug = d.dbg_p || d.dbg_m || d.dbg_v;
+            uint8_t what = kGeneric;
+            if (cen && !d.row_mean) what = d.row_len <= kRowwiseShortMax ? kRowShort : kRowLong;   // validated: rowwise_ok
+            else if (templated && !debug && !cen) what = d.numel >= unit ? kUnits : want_explicit ? kGeneric : kPieces;
+            else if (cen_kernel && !debug && cen && d.row_len >= (uint64_t)kVec && d.row_len < (1ull << 31))
+                what = d.numel >= unit ? kCenUnits : kCenPieces;   // a lane's 8 elements lie in at most two rows
+            kind[k1] = what;
+            ++in_kind[what];
+            plan.has_extras |= cen || debug || want_explicit || !templated;
+        }
+        // ---- where each kind's records begin
         Batch b{};
         b.combo = combo;
-        b.first_range = (uint32_t)ranges.size();
-        b.first_piece = (uint32_t)pieces.size();
-        const bool has_pieces = !want_explicit && narrow_combo(combo);
-        auto plain = [&](const DevTensor& t) {
-            return combo != kComboAny && !(t.flags & kFlagRowwise) &&
-                   (t.dp | t.dm | t.dv | t.row_mean) == 0;
-        };
-        uint32_t units = 0;
-        for (size_t k = k0; k < k1; ++k) {
-            const DevTensor& t = tens[k];
-            if (!plain(t)) continue;
-            const uint32_t nu = (uint32_t)(t.numel / unit);
-            if (nu) {
-                ranges.push_back(units);
-                fast_tens.push_back(t);
-                units += nu;
-            }
-            if (has_pieces) {
-                for (uint64_t e = (uint64_t)nu * unit; e < t.numel; e += kPieceElems) {
-                    PieceRef r;
-                    memset(&r, 0, sizeof(r));
-                    const int ep = dtype_size(t.dtypes & 3u), eg = dtype_size((t.dtypes >> 2) & 3u),
-                              em = dtype_size((t.dtypes >> 4) & 3u), ev = dtype_size((t.dtypes >> 6) & 3u);
-                    r.p = t.p + e * ep; r.g = t.g + e * eg; r.m = t.m + e * em; r.v = t.v + e * ev;
-                    r.block = t.block_base + (e >> 3);
-                    r.count = (uint32_t)std::min<uint64_t>(kPieceElems, t.numel - e);
-                    r.tensor_id4 = t.tensor_id4;
-                    r.set_idx = t.set_idx;
-                    pieces.push_back(r);
-                }
-            }
+        b.first_tensor = (uint32_t)k0;
+        uint32_t at[kKinds];
+        for (uint32_t t = 0, pos = (uint32_t)k0; t < kKinds; ++t) {
+            at[t] = pos;
+            pos += in_kind[t];
         }
-        b.n_ranges = (uint32_t)ranges.size() - b.first_range;
-        b.n_units = units;
-        b.n_pieces = (uint32_t)pieces.size() - b.first_piece;
-        // Tensors with centralization that are otherwise plain: their whole units go to the fast
-        // kernel's centralizing variant (16-bit layouts with Philox noise have one), the rest of them
-        // to the generic kernel.  A lane's 8 elements must lie in at most two rows.
-        auto cen_plain = [&](const DevTensor& t) {
-            return has_pieces && (t.dp | t.dm | t.dv) == 0 && t.row_mean != 0 &&
-                   t.row_len >= (uint64_t)kVec && t.row_len < (1ull << 31);
-        };
-        b.first_cen_range = (uint32_t)ranges.size();
-        uint32_t cen_units = 0;
-        for (size_t k = k0; k < k1; ++k) {
-            const DevTensor& t = tens[k];
-            if (!cen_plain(t) || t.numel < unit) continue;
-            ranges.push_back(cen_units);
-            fast_tens.push_back(t);
-            cen_units += (uint32_t)(t.numel / unit);
+        b.plain.first_tensor = at[kUnits];
+        b.plain.n_ranges = in_kind[kUnits];
+        b.cen.first_tensor = at[kCenUnits];
+        b.cen.n_ranges = in_kind[kCenUnits];
+        for (int s = 0; s < 2; ++s) {
+            b.rowwise[s].first_tensor = at[s ? kRowShort : kRowLong];
+            b.rowwise[s].n_ranges = in_kind[s ? kRowShort : kRowLong];
         }
-        b.n_cen_ranges = (uint32_t)ranges.size() - b.first_cen_range;
-        b.n_cen_units = cen_units;
-        // Tensors whose row means the update takes itself: whole tensors, a wavefront per row.
-        for (int kind = 0; kind < 2; ++kind) {
-            b.first_rw_range[kind] = (uint32_t)ranges.size();
-            uint64_t rw_rows = 0;
-            for (size_t k = k0; k < k1; ++k) {
-                const DevTensor& t = tens[k];
-                if (!(t.flags & kFlagRowwise) || (int)(t.row_len <= kRowwiseShortMax) != kind) continue;
-                ranges.push_back((uint32_t)rw_rows);
-                fast_tens.push_back(t);
-                rw_rows += t.numel / t.row_len;
-            }
-            b.n_rw_ranges[kind] = (uint32_t)ranges.size() - b.first_rw_range[kind];
-            b.n_rw_rows[kind] = (uint32_t)std::min<uint64_t>(rw_rows, 0xFFFFFFFFull);   // checked against the grid limit at launch
-        }
-        b.first_generic = (uint32_t)chunks.size();
-        for (size_t k = k0; k < k1; ++k) {
-            const DevTensor& t = tens[k];
-            const uint32_t nc = (uint32_t)((t.numel + kChunkElems - 1) / kChunkElems);
-            uint32_t j0 = 0;
-            if (plain(t)) j0 = has_pieces ? nc : (uint32_t)((t.numel / unit) * unit / kChunkElems);
-            if (cen_plain(t)) j0 = (uint32_t)((t.numel / unit) * unit / kChunkElems);
-            if (t.flags & kFlagRowwise) j0 = nc;
-            for (uint32_t j = j0; j < nc; ++j) chunks.push_back(ChunkRef{(uint32_t)k, j});
-        }
-        b.n_generic = (uint32_t)chunks.size() - b.first_generic;
         plan.batches.push_back(b);
+        if (in_kind[kUnits] + in_kind[kPieces] + in_kind[kRowLong] + in_kind[kRowShort] == k1 - k0 &&
+            std::max({in_kind[kUnits], in_kind[kPieces], in_kind[kRowLong], in_kind[kRowShort]}) == k1 - k0) {
+            // all of one kind: in place already
+        } else {   // stable by kind
+            std::vector<uint32_t> o(order.begin() + k0, order.begin() + k1), s(set_of.begin() + k0, set_of.begin() + k1);
+            std::vector<uint8_t> w(kind.begin() + k0, kind.begin() + k1);
+            for (size_t k = 0; k < o.size(); ++k) {
+                const uint32_t to = at[w[k]]++;
+                order[to] = o[k];
+                set_of[to] = s[k];
+                kind[to] = w[k];
+            }
+        }
+        // ---- units, pieces and chunks in the order of the records
+        Batch& bb = plan.batches.back();
+        bb.first_generic = (uint32_t)chunks.size();
+        uint64_t n_rows[2] = {0, 0};
+        for (int c = 0; c < 2; ++c) {
+            Group& grp = c ? bb.cen : bb.plain;
+            grp.first_piece = (uint32_t)pieces_total;
+            for (size_t k = k0; k < k1; ++k) {
+                if (kind[k] != (c ? kCenUnits : kUnits) && kind[k] != (c ? kCenPieces : kPieces)) continue;
+                const uint64_t numel = descs[order[k]].numel;
+                grp.n_units += (uint32_t)(numel / unit);
+                const uint64_t rest = numel % unit;
+                if (!rest) continue;
+                if (want_explicit) chunks.push_back(ChunkRef{(uint32_t)(k - k0), (uint32_t)(numel / unit)});
+                else pieces_total += (rest + kPieceElems - 1) / kPieceElems;
+            }
+            grp.n_pieces = (uint32_t)(pieces_total - grp.first_piece);
+        }
+        for (size_t k = k0; k < k1; ++k) {
+            const rt_tensor_desc& d = descs[order[k]];
+            if (kind[k] == kRowLong || kind[k] == kRowShort) n_rows[kind[k] == kRowShort] += d.numel / d.row_len;
+            if (kind[k] != kGeneric) continue;
+            const uint32_t nc = (uint32_t)((d.numel + kChunkElems - 1) / kChunkElems);
+            for (uint32_t j = 0; j < nc; ++j) chunks.push_back(ChunkRef{(uint32_t)(k - k0), j});
+        }
+        for (int s = 0; s < 2; ++s)
+            bb.rowwise[s].n_units = (uint32_t)std::min<uint64_t>(n_rows[s], 0xFFFFFFFFull);   // checked against the grid limit at launch
+        bb.n_generic = (uint32_t)chunks.size() - bb.first_generic;
         k0 = k1;
     }
 
     plan.set_keys.assign(sets.size(), {0u, 0u});
-    for (const auto& kv : set_of) plan.set_keys[kv.second] = kv.first;
+    for (const auto& kv : set_index) plan.set_keys[kv.second] = kv.first;
     plan.n_sets = (uint32_t)sets.size();
-    plan.n_tensors = (uint32_t)tens.size();
-    plan.n_chunks = (uint32_t)chunks.size();
+    plan.n_tensors = (uint32_t)count;
     if (!sets.empty()) plan.first_set = sets[0];
     plan.off_sets = 0;
     plan.off_tensors = align_up(sets.size() * sizeof(DevScalars), 256);
-    plan.off_ranges = plan.off_tensors + align_up(tens.size() * sizeof(DevTensor), 128);
-    plan.off_fast_tensors = plan.off_ranges + align_up(ranges.size() * sizeof(uint32_t), 128);
-    plan.off_pieces = plan.off_fast_tensors + align_up(fast_tens.size() * sizeof(DevTensor), 128);
-    plan.off_chunks = plan.off_pieces + align_up(pieces.size() * sizeof(PieceRef), 128);
+    plan.off_extras = plan.off_tensors + align_up(count * sizeof(TensorRec), 128);
+    plan.off_first = plan.off_extras + (plan.has_extras ? align_up(count * sizeof(TensorExtra), 128) : 0);
+    plan.off_piece_tensor = plan.off_first + align_up(count * sizeof(uint32_t), 128);
+    plan.off_chunks = plan.off_piece_tensor + align_up(pieces_total * sizeof(uint32_t), 128);
     plan.bytes = plan.off_chunks + align_up(chunks.size() * sizeof(ChunkRef), 128);
-    h->image.assign(plan.bytes, 0);
-    uint8_t* img = h->image.data();
+    image.resize(plan.bytes);
+    uint8_t* img = image.data();
     if (!sets.empty()) memcpy(img + plan.off_sets, sets.data(), sets.size() * sizeof(DevScalars));
-    if (!tens.empty()) memcpy(img + plan.off_tensors, tens.data(), tens.size() * sizeof(DevTensor));
-    if (!ranges.empty()) memcpy(img + plan.off_ranges, ranges.data(), ranges.size() * sizeof(uint32_t));
-    if (!fast_tens.empty())
-        memcpy(img + plan.off_fast_tensors, fast_tens.data(), fast_tens.size() * sizeof(DevTensor));
-    if (!pieces.empty()) memcpy(img + plan.off_pieces, pieces.data(), pieces.size() * sizeof(PieceRef));
     if (!chunks.empty()) memcpy(img + plan.off_chunks, chunks.data(), chunks.size() * sizeof(ChunkRef));
+    TensorRec* recs = (TensorRec*)(img + plan.off_tensors);
+    TensorExtra* extras = (TensorExtra*)(img + plan.off_extras);
+    uint32_t* first = (uint32_t*)(img + plan.off_first);
+    uint32_t* piece_tensor = (uint32_t*)(img + plan.off_piece_tensor);
+    for (const Batch& b : plan.batches) {
+        const size_t k1 = &b == &plan.batches.back() ? count : (&b + 1)->first_tensor;
+        uint32_t units[2] = {0, 0}, rows[2] = {0, 0}, piece[2] = {0, 0};   // running numbers per launch
+        for (size_t k = b.first_tensor; k < k1; ++k) {
+            const rt_tensor_desc& d = descs[order[k]];
+            TensorRec& t = recs[k];
+            t.p = (uint64_t)d.p; t.g = (uint64_t)d.g; t.m = (uint64_t)d.m; t.v = (uint64_t)d.v;
+            t.numel = d.numel;
+            t.block_base = d.elem_offset >> 3;
+            t.tensor_id4 = d.tensor_id * 4u;
+            t.set_idx = set_of[k];
+            t.first_piece = 0;
+            t.dtypes = dtypes_of(d);
+            first[k] = 0;
+            if (kind[k] <= kCenPieces) {
+                const int c = kind[k] >= kCenUnits;
+                const Group& grp = c ? b.cen : b.plain;
+                first[k] = units[c];
+                units[c] += (uint32_t)(d.numel / unit);
+                t.first_piece = piece[c];
+                if (!want_explicit)
+                    for (uint64_t e = d.numel / unit * unit; e < d.numel; e += kPieceElems)
+                        piece_tensor[grp.first_piece + piece[c]++] = (uint32_t)k - grp.first_tensor;
+            } else if (kind[k] != kGeneric) {
+                const int s = kind[k] == kRowShort;
+                first[k] = rows[s];
+                rows[s] += (uint32_t)(d.numel / d.row_len);
+            }
+            if (!plan.has_extras) continue;
+            TensorExtra& x = extras[k];
+            memset(&x, 0, sizeof(x));
+            if (want_explicit) {
+                x.np = (uint64_t)d.noise_p; x.nm = (uint64_t)d.noise_m; x.nv = (uint64_t)d.noise_v;
+            }
+            x.dp = (uint64_t)d.dbg_p; x.dm = (uint64_t)d.dbg_m; x.dv = (uint64_t)d.dbg_v;
+            x.row_mean = sets[set_of[k]].s.centralization != 0.0f ? (uint64_t)d.row_mean : 0;
+            x.row_len = d.row_len ? d.row_len : 1;
+        }
+    }
 }
 
 // Puts a table image into a free table slot (skipping what the slot's device memory already
@@ -616,7 +628,6 @@ static int enqueue_kernels(const Plan& plan, const uint8_t* base, uint64_t seed,
                            hipEvent_t t_begin = nullptr, hipEvent_t t_end = nullptr) {
     LaunchArgs a;
     memset(&a, 0, sizeof(a));
-    a.tensors = (const DevTensor*)(base + plan.off_tensors);
     a.sets = (const DevScalars*)(base + plan.off_sets);
     a.clip_coef = d_clip_coef;
     a.skip = d_skip;
@@ -630,52 +641,58 @@ static int enqueue_kernels(const Plan& plan, const uint8_t* base, uint64_t seed,
         LaunchArgs args;
     };
     std::vector<Launch> launches;
+    auto records_from = [&](LaunchArgs& x, uint32_t first_tensor) {
+        x.tensors = (const TensorRec*)(base + plan.off_tensors) + first_tensor;
+        x.extras = plan.has_extras ? (const TensorExtra*)(base + plan.off_extras) + first_tensor : nullptr;
+        x.first = (const uint32_t*)(base + plan.off_first) + first_tensor;
+    };
     for (const Batch& b : plan.batches) {
         KernelPair k{};
         if (b.combo == kComboAny) {
-            k.fast = nullptr;  // no ranges and no pieces for this group
+            k.fast = nullptr;  // no units and no pieces for this group
             k.generic = noise_mode == RT_NOISE_EXPLICIT ? sr_adamw_any_kernel<RT_NOISE_EXPLICIT>
                                                         : sr_adamw_any_kernel<RT_NOISE_PHILOX>;
         } else {
             k = pick_kernel(b.combo & 3, (b.combo >> 2) & 3, (b.combo >> 4) & 3, (b.combo >> 6) & 3, noise_mode);
         }
-        a.first = (const uint32_t*)(base + plan.off_ranges) + b.first_range;
-        a.fast_tensors = (const DevTensor*)(base + plan.off_fast_tensors) + b.first_range;
-        a.n_ranges = b.n_ranges;
-        a.pieces = (const PieceRef*)(base + plan.off_pieces) + b.first_piece;
-        a.n_pieces = b.n_pieces;
-        a.n_piece_wgs = (b.n_pieces + 3u) / 4u;
-        a.chunks = (const ChunkRef*)(base + plan.off_chunks) + b.first_generic;
-        const uint64_t grid = (uint64_t)a.n_piece_wgs + b.n_units;
-        a.piece_rate = 0;  // only pieces, or none
-        if (a.n_piece_wgs != 0 && b.n_units != 0)
-            a.piece_rate = (uint32_t)((((uint64_t)a.n_piece_wgs << 32) + grid - 1) / grid);  // < 2^32: n_piece_wgs < grid
-        if (grid > kMaxGrid || b.n_generic > kMaxGrid) return fail(RT_EUNSUPPORTED, "too many workgroups in one launch");
-        if (grid) launches.push_back(Launch{k.fast, (uint32_t)grid, a});
-        if (b.n_generic) launches.push_back(Launch{k.generic, b.n_generic, a});
-        if (b.n_cen_units) {
-            if (!k.fast_cen) return fail(RT_EHIP, "internal: centralized units without a kernel for them");
-            LaunchArgs c = a;
-            c.first = (const uint32_t*)(base + plan.off_ranges) + b.first_cen_range;
-            c.fast_tensors = (const DevTensor*)(base + plan.off_fast_tensors) + b.first_cen_range;
-            c.n_ranges = b.n_cen_ranges;
-            c.n_pieces = c.n_piece_wgs = c.piece_rate = 0;
-            launches.push_back(Launch{k.fast_cen, b.n_cen_units, c});
+        for (int c = 0; c < 2; ++c) {
+            const Group& grp = c ? b.cen : b.plain;
+            const uint32_t piece_wgs = (grp.n_pieces + 3u) / 4u;
+            const uint64_t grid = (uint64_t)piece_wgs + grp.n_units;
+            if (!grid) continue;
+            if (grid > kMaxGrid) return fail(RT_EUNSUPPORTED, "too many workgroups in one launch");
+            const MultiKernel kern = c ? k.fast_cen : k.fast;
+            if (!kern) return fail(RT_EHIP, "internal: units without a kernel for them");
+            launches.push_back(Launch{kern, (uint32_t)grid, a});
+            LaunchArgs& x = launches.back().args;
+            records_from(x, grp.first_tensor);
+            x.n_ranges = grp.n_ranges;
+            x.piece_tensor = (const uint32_t*)(base + plan.off_piece_tensor) + grp.first_piece;
+            x.n_pieces = grp.n_pieces;
+            x.n_piece_wgs = piece_wgs;
+            x.piece_rate = 0;  // only pieces, or none
+            if (piece_wgs != 0 && grp.n_units != 0)
+                x.piece_rate = (uint32_t)((((uint64_t)piece_wgs << 32) + grid - 1) / grid);  // < 2^32: piece_wgs < grid
         }
-        for (int kind = 0; kind < 2; ++kind) {
-            if (!b.n_rw_rows[kind]) continue;
-            const MultiKernel kern = kind ? k.rowwise_short : k.rowwise;
+        if (b.n_generic) {
+            if (b.n_generic > kMaxGrid) return fail(RT_EUNSUPPORTED, "too many workgroups in one launch");
+            launches.push_back(Launch{k.generic, b.n_generic, a});
+            records_from(launches.back().args, b.first_tensor);
+            launches.back().args.chunks = (const ChunkRef*)(base + plan.off_chunks) + b.first_generic;
+        }
+        for (int s = 0; s < 2; ++s) {
+            const Group& grp = b.rowwise[s];
+            if (!grp.n_units) continue;
+            const MultiKernel kern = s ? k.rowwise_short : k.rowwise;
             if (!kern) return fail(RT_EHIP, "internal: row-wise tensors without a kernel for them");
-            const uint64_t rw_grid = ((uint64_t)b.n_rw_rows[kind] + kThreads / 64 - 1) / (kThreads / 64);
-            if (b.n_rw_rows[kind] == 0xFFFFFFFFu || rw_grid > kMaxGrid)
+            const uint64_t rw_grid = ((uint64_t)grp.n_units + kThreads / 64 - 1) / (kThreads / 64);
+            if (grp.n_units == 0xFFFFFFFFu || rw_grid > kMaxGrid)
                 return fail(RT_EUNSUPPORTED, "too many rows in one launch");
-            LaunchArgs c = a;
-            c.first = (const uint32_t*)(base + plan.off_ranges) + b.first_rw_range[kind];
-            c.fast_tensors = (const DevTensor*)(base + plan.off_fast_tensors) + b.first_rw_range[kind];
-            c.n_ranges = b.n_rw_ranges[kind];
-            c.n_rows = b.n_rw_rows[kind];
-            c.n_pieces = c.n_piece_wgs = c.piece_rate = 0;
-            launches.push_back(Launch{kern, (uint32_t)rw_grid, c});
+            launches.push_back(Launch{kern, (uint32_t)rw_grid, a});
+            LaunchArgs& x = launches.back().args;
+            records_from(x, grp.first_tensor);
+            x.n_ranges = grp.n_ranges;
+            x.n_rows = grp.n_units;
         }
     }
     for (size_t i = 0; i < launches.size(); ++i) {
@@ -734,8 +751,7 @@ static int launch_update(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, 
         lc.valid = false;
         int rc = validate(descs, n, scalars, n_scalars, noise_mode, /*allow_host=*/false);
         if (rc != RT_OK) return rc;
-        build_image(h, descs, n, scalars, noise_mode == RT_NOISE_EXPLICIT, lc.plan);
-        lc.image = h->image;
+        build_image(h, descs, n, scalars, noise_mode == RT_NOISE_EXPLICIT, lc.plan, lc.image);
         lc.descs.assign(descs, descs + n);
         lc.cen.resize(lc.plan.set_keys.size());
         for (size_t j = 0; j < lc.plan.set_keys.size(); ++j)
@@ -1565,7 +1581,7 @@ static int streamed_enqueue_impl(rt_handle* h, const rt_tensor_desc* descs, uint
             pieces[c].push_back(q);
         }
         build_image(h, pieces[c].data(), (uint32_t)pieces[c].size(), scalars, noise_mode == RT_NOISE_EXPLICIT,
-                    plans[c]);
+                    plans[c], h->image);
         plan_off[c] = align_up(blob.size(), 256);
         blob.resize(plan_off[c] + plans[c].bytes);
         if (plans[c].bytes) memcpy(blob.data() + plan_off[c], h->image.data(), plans[c].bytes);

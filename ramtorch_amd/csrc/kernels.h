@@ -330,7 +330,7 @@ __device__ __forceinline__ void update_n(float (&p)[N], const float (&g)[N], flo
 
 // Noise for the block of 8 elements starting at element i of tensor t.
 template <int PDT, int MDT, int VDT>
-__device__ __forceinline__ void philox_noise3(const DevTensor& t, const UpdateCtx& c, uint64_t i, u32x4& zp,
+__device__ __forceinline__ void philox_noise3(const TensorRec& t, const UpdateCtx& c, uint64_t i, u32x4& zp,
                                               u32x4& zm, u32x4& zv) {
     const uint64_t blk = t.block_base + (i >> 3);
     const uint32_t b0 = (uint32_t)blk, b1 = (uint32_t)(blk >> 32);
@@ -400,17 +400,55 @@ __device__ __forceinline__ uint32_t find_range(const uint32_t* __restrict__ firs
 }
 
 // ---------------------------------------------------------------------------
-// Piece: at most 512 consecutive elements handled by one wavefront, one 128-bit
+// Which part of a launch a workgroup serves.  Piece workgroups (four pieces each, one per wavefront)
+// are spread evenly among the unit workgroups: of the first b workgroups, min(n_piece_wgs,
+// floor(b * piece_rate / 2^32)) serve pieces (piece_rate = ceil(n_piece_wgs * 2^32 / gridDim.x), or 0 when the
+// launch has only pieces).  Pieces are bound by instruction issue and by the latency of their short
+// dependent chains, units by memory: resident side by side they overlap.
+// Returns true for units and then the unit's number, false for pieces and then the wavefront's piece.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ bool unit_or_pieces(const LaunchArgs& a, uint32_t& which) {
+    const uint32_t b = blockIdx.x;
+    uint32_t pieces_before = b, pieces_after = b + 1u;
+    if (a.piece_rate != 0u) {
+        pieces_before = min(a.n_piece_wgs, __umulhi(b, a.piece_rate));
+        pieces_after = min(a.n_piece_wgs, __umulhi(b + 1u, a.piece_rate));
+    } else if (a.n_piece_wgs == 0u) {
+        pieces_before = pieces_after = 0u;
+    }
+    if (pieces_after == pieces_before) {
+        which = b - pieces_before;
+        return true;
+    }
+    which = (uint32_t)__builtin_amdgcn_readfirstlane((int)(pieces_before * 4u + (threadIdx.x >> 6)));
+    return false;
+}
+
+// Centralization: what to subtract from each of a lane's 8 elements, which lie in at most two rows
+// (row_len >= 8): fl(mean(row) * c), the product rounded before it is subtracted (adamw.py:179-184,
+// grad.sub_(mean.mul_(c))).  `rem`: position of the first element inside its row.
+__device__ __forceinline__ void subtract_means(float (&g)[8], float mean0, float mean1, uint32_t rem, uint32_t row_len,
+                                               const UpdateCtx& c) {
+    const float mc0 = cen_term(mean0, c.s, c.do_clip, c.coef), mc1 = cen_term(mean1, c.s, c.do_clip, c.coef);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) g[j] = g[j] - (rem + (uint32_t)j < row_len ? mc0 : mc1);
+}
+
+// ---------------------------------------------------------------------------
+// Piece: at most 512 consecutive elements handled by one wavefront, one 8-element
 // vector per lane (the last lane with elements may hold fewer than 8 and then
 // moves them one by one).  Short tensors and the leftovers of long ones.
 // ---------------------------------------------------------------------------
-template <int PDT, int GDT, int MDT, int VDT>
+template <int PDT, int GDT, int MDT, int VDT, bool CEN>
 __device__ __forceinline__ void piece_body(const LaunchArgs& a, uint32_t q) {
-    // (the piece records stream through: read with vector loads they stay out of the small scalar
+    // (the records stream through: read with vector loads they stay out of the small scalar
     // cache that the unit workgroups' tables live in -- 2.7 % faster on the 20 064-tensor set)
-    const PieceRef& r = a.pieces[q];
-    const uint64_t rp = r.p, rg = r.g, rm = r.m, rv = r.v;
-    const uint32_t count = r.count;
+    const uint32_t ti = a.piece_tensor[q];
+    const TensorRec& r = a.tensors[ti];
+    const uint64_t start = (r.numel & ~(uint64_t)(kFastUnitElems - 1u)) + (uint64_t)(q - r.first_piece) * kPieceElems;
+    const uint64_t rp = r.p + start * esize<PDT>(), rg = r.g + start * esize<GDT>(), rm = r.m + start * esize<MDT>(),
+                   rv = r.v + start * esize<VDT>();
+    const uint32_t count = (uint32_t)min((uint64_t)kPieceElems, r.numel - start);
     const uint64_t i = (uint64_t)(threadIdx.x & 63u) * kVec;
     if (i >= count) return;
     const bool full = i + kVec <= count;
@@ -424,7 +462,20 @@ __device__ __forceinline__ void piece_body(const LaunchArgs& a, uint32_t q) {
     }
     UpdateCtx c;
     make_ctx(a, r.set_idx, c);
-    const uint64_t blk = r.block + (i >> 3);
+    float mean0 = 0.0f, mean1 = 0.0f;
+    uint32_t rem = 0, row_len = 0;
+    if constexpr (CEN) {
+        const TensorExtra& x = a.extras[ti];
+        row_len = (uint32_t)x.row_len;
+        const uint64_t e0 = (r.block_base << 3) + start + i;
+        const uint64_t row = e0 / row_len;
+        rem = (uint32_t)(e0 - row * row_len);
+        mean0 = ldg32f(x.row_mean + row * 4);
+        // (a row that begins behind the tensor's last element has no mean)
+        const bool next_row = rem + (kVec - 1) >= row_len && start + i + (row_len - rem) < r.numel;
+        mean1 = next_row ? ldg32f(x.row_mean + row * 4 + 4) : 0.0f;
+    }
+    const uint64_t blk = r.block_base + ((start + i) >> 3);
     const uint32_t b0 = (uint32_t)blk, b1 = (uint32_t)(blk >> 32);
     u32x4 zp = 0, zm = 0, zv = 0;
     if constexpr (PDT == RT_DT_BF16) zp = philox4x32_10(b0, b1, r.tensor_id4 + 0u, c.step, c.seed_lo, c.seed_hi);
@@ -433,6 +484,7 @@ __device__ __forceinline__ void piece_body(const LaunchArgs& a, uint32_t q) {
     float p[8], g[8], m[8], v[8];
     decode<PDT>(xp, p); decode<GDT>(xg, g); decode<MDT>(xm, m); decode<VDT>(xv, v);
     scale_grads(g, c);
+    if constexpr (CEN) subtract_means(g, mean0, mean1, rem, row_len, c);
     update_n<8>(p, g, m, v, c.s);
     if (full) {
         store_out<PDT>(rp, i, p, zp);
@@ -447,48 +499,34 @@ __device__ __forceinline__ void piece_body(const LaunchArgs& a, uint32_t q) {
 
 // ---------------------------------------------------------------------------
 // Fast kernel, all arrays 16 bit wide.  One launch covers everything that needs
-// no special care:
-//  * n_piece_wgs workgroups serve four pieces each, one per wavefront (Philox
-//    mode only);
-//  * the other workgroups serve one unit of kFastUnitElems elements each, lying
-//    wholly inside one tensor.  Every access is a 128-bit global load or store;
-//    all loads of the unit are issued before the math of its first vector so that
-//    memory latency hides behind the VALU work (Philox, sqrt, division).
+// no special care: workgroups with pieces (Philox mode only), and workgroups
+// with one unit of kFastUnitElems elements each, lying wholly inside one tensor.
+// Every access to a unit is a 128-bit global load or store; all loads of the
+// unit are issued before the math of its first vector so that memory latency
+// hides behind the VALU work (Philox, sqrt, division).
 // Everything is inlined and lives in registers: a stack frame here would turn
 // into scratch-memory traffic on every workgroup.
 // ---------------------------------------------------------------------------
-// CEN: the tensors of the launch have their gradients centralized (adamw.py:179-184): fl(mean(row) * c)
-// is subtracted from every gradient element before the update.  Rows are at least 8 elements long
-// (shorter ones take the generic kernel), so a lane's 8 elements lie in at most two rows.
+// CEN: the tensors of the launch have their gradients centralized by row means computed before.  Rows are
+// at least 8 elements long (shorter ones take the generic kernel).
 template <int PDT, int GDT, int MDT, int VDT, int NOISE, bool CEN = false>
 __global__ __launch_bounds__(kThreads) void sr_adamw_fast_kernel(const LaunchArgs a) {
     if (a.skip != nullptr && load_const(a.skip) != 0u) return;
-    // Piece workgroups are spread evenly among the unit workgroups: of the first b workgroups,
-    // min(n_piece_wgs, floor(b * piece_rate / 2^32)) serve pieces (piece_rate = ceil(n_piece_wgs * 2^32 /
-    // gridDim.x), or 0 when the launch has only pieces).  Pieces are bound by instruction issue and by
-    // the latency of their short dependent chains, units by memory: resident side by side they overlap.
-    const uint32_t b = blockIdx.x;
-    uint32_t pieces_before = b, pieces_after = b + 1u;
-    if (a.piece_rate != 0u) {
-        pieces_before = min(a.n_piece_wgs, __umulhi(b, a.piece_rate));
-        pieces_after = min(a.n_piece_wgs, __umulhi(b + 1u, a.piece_rate));
-    } else if (a.n_piece_wgs == 0u) {
-        pieces_before = pieces_after = 0u;
-    }
-    if (pieces_after != pieces_before) {
+    uint32_t unit;
+    if (!unit_or_pieces(a, unit)) {
         if constexpr (NOISE == RT_NOISE_PHILOX) {
-            const uint32_t q = (uint32_t)__builtin_amdgcn_readfirstlane((int)(pieces_before * 4u + (threadIdx.x >> 6)));
-            if (q < a.n_pieces) piece_body<PDT, GDT, MDT, VDT>(a, q);
+            if (unit < a.n_pieces) piece_body<PDT, GDT, MDT, VDT, CEN>(a, unit);
         }
         return;
     }
-    const uint32_t unit = b - pieces_before;
     const uint32_t ri = find_range(a.first, a.n_ranges, unit);
-    const DevTensor t = load_const(&a.fast_tensors[ri]);
+    const TensorRec t = load_const(&a.tensors[ri]);
     const uint32_t unit_in_tensor = unit - load_const(&a.first[ri]);
     UpdateCtx c;
     make_ctx(a, t.set_idx, c);
-    const uint64_t tp = t.p, tg = t.g, tm = t.m, tv = t.v, tnp = t.np, tnm = t.nm, tnv = t.nv;
+    const uint64_t tp = t.p, tg = t.g, tm = t.m, tv = t.v;
+    TensorExtra x;
+    if constexpr (NOISE == RT_NOISE_EXPLICIT || CEN) x = load_const(&a.extras[ri]);
 
     struct In {
         Raw8<PDT> p;
@@ -499,7 +537,7 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_fast_kernel(const LaunchArg
         float mean0, mean1;  // CEN: means of the row of the first element and of the row after it
         uint32_t rem;        // CEN: position of the first element inside its row
     };
-    const uint32_t row_len = (uint32_t)t.row_len;  // CEN launches: 8 <= row_len < 2^31
+    const uint32_t row_len = CEN ? (uint32_t)x.row_len : 0u;  // CEN launches: 8 <= row_len < 2^31
     auto fetch = [&](uint64_t i, uint64_t row, uint32_t rem) {
         In r;
         r.p = load_raw<PDT>(tp, i);
@@ -507,14 +545,14 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_fast_kernel(const LaunchArg
         r.m = load_raw<MDT>(tm, i);
         r.v = load_raw<VDT>(tv, i);
         if constexpr (NOISE == RT_NOISE_EXPLICIT) {
-            if constexpr (PDT == RT_DT_BF16) r.zp = ldg128(tnp + i * 2);
-            if constexpr (MDT == RT_DT_BF16) r.zm = ldg128(tnm + i * 2);
-            if constexpr (VDT == RT_DT_BF16) r.zv = ldg128(tnv + i * 2);
+            if constexpr (PDT == RT_DT_BF16) r.zp = ldg128(x.np + i * 2);
+            if constexpr (MDT == RT_DT_BF16) r.zm = ldg128(x.nm + i * 2);
+            if constexpr (VDT == RT_DT_BF16) r.zv = ldg128(x.nv + i * 2);
         }
         if constexpr (CEN) {
             r.rem = rem;
-            r.mean0 = ldg32f(t.row_mean + row * 4);
-            r.mean1 = rem + (kVec - 1) >= row_len ? ldg32f(t.row_mean + row * 4 + 4) : 0.0f;
+            r.mean0 = ldg32f(x.row_mean + row * 4);
+            r.mean1 = rem + (kVec - 1) >= row_len ? ldg32f(x.row_mean + row * 4 + 4) : 0.0f;
         }
         return r;
     };
@@ -567,12 +605,7 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_fast_kernel(const LaunchArg
         u32x4 zp = cur.zp, zm = cur.zm, zv = cur.zv;
         if constexpr (NOISE == RT_NOISE_PHILOX) philox_noise3<PDT, MDT, VDT>(t, c, i, zp, zm, zv);
         scale_grads(g, c);
-        if constexpr (CEN) {
-            // grad.sub_(mean.mul_(c)): the product is rounded, then subtracted
-            const float mc0 = cen_term(cur.mean0, c.s, c.do_clip, c.coef), mc1 = cen_term(cur.mean1, c.s, c.do_clip, c.coef);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) g[j] = g[j] - (cur.rem + (uint32_t)j < row_len ? mc0 : mc1);
-        }
+        if constexpr (CEN) subtract_means(g, cur.mean0, cur.mean1, cur.rem, row_len, c);
         update_n<8>(p, g, m, v, c.s);
         store_out<PDT>(tp, i, p, zp);
         store_out<MDT>(tm, i, m, zm);
@@ -659,13 +692,21 @@ __device__ __forceinline__ void store_out4(uint64_t base, uint64_t e, const floa
 template <int PDT, int GDT, int MDT, int VDT, int NOISE>
 __global__ __launch_bounds__(kThreads) void sr_adamw_fast_wide_kernel(const LaunchArgs a) {
     if (a.skip != nullptr && load_const(a.skip) != 0u) return;
-    const uint32_t unit = blockIdx.x;
+    uint32_t unit;
+    if (!unit_or_pieces(a, unit)) {
+        if constexpr (NOISE == RT_NOISE_PHILOX) {
+            if (unit < a.n_pieces) piece_body<PDT, GDT, MDT, VDT, false>(a, unit);
+        }
+        return;
+    }
     const uint32_t ri = find_range(a.first, a.n_ranges, unit);
-    const DevTensor t = load_const(&a.fast_tensors[ri]);
+    const TensorRec t = load_const(&a.tensors[ri]);
     const uint32_t unit_in_tensor = unit - load_const(&a.first[ri]);
     UpdateCtx c;
     make_ctx(a, t.set_idx, c);
-    const uint64_t tp = t.p, tg = t.g, tm = t.m, tv = t.v, tnp = t.np, tnm = t.nm, tnv = t.nv;
+    const uint64_t tp = t.p, tg = t.g, tm = t.m, tv = t.v;
+    TensorExtra x;
+    if constexpr (NOISE == RT_NOISE_EXPLICIT) x = load_const(&a.extras[ri]);
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const bool odd = (lane & 1u) != 0u;
     constexpr uint32_t kWaveElems = 64 * kVec;       // 512 elements per wave per iteration
@@ -685,9 +726,9 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_fast_wide_kernel(const Laun
             r.m[h] = load_raw4<MDT>(tm, e);
             r.v[h] = load_raw4<VDT>(tv, e);
             if constexpr (NOISE == RT_NOISE_EXPLICIT) {
-                if constexpr (PDT == RT_DT_BF16) r.zp[h] = ldg64(tnp + e * 2);
-                if constexpr (MDT == RT_DT_BF16) r.zm[h] = ldg64(tnm + e * 2);
-                if constexpr (VDT == RT_DT_BF16) r.zv[h] = ldg64(tnv + e * 2);
+                if constexpr (PDT == RT_DT_BF16) r.zp[h] = ldg64(x.np + e * 2);
+                if constexpr (MDT == RT_DT_BF16) r.zm[h] = ldg64(x.nm + e * 2);
+                if constexpr (VDT == RT_DT_BF16) r.zv[h] = ldg64(x.nv + e * 2);
             }
         }
         return r;
@@ -756,7 +797,8 @@ template <int PDT, int GDT, int MDT, int VDT, int NOISE>
 __global__ __launch_bounds__(kThreads) void sr_adamw_generic_kernel(const LaunchArgs a) {
     if (a.skip != nullptr && load_const(a.skip) != 0u) return;
     const ChunkRef cr = load_const(&a.chunks[blockIdx.x]);
-    const DevTensor t = load_const(&a.tensors[cr.tensor]);
+    const TensorRec t = load_const(&a.tensors[cr.tensor]);
+    const TensorExtra x = load_const(&a.extras[cr.tensor]);
     UpdateCtx c;
     make_ctx(a, t.set_idx, c);
 
@@ -778,30 +820,30 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_generic_kernel(const Launch
         }
         if constexpr (NOISE == RT_NOISE_EXPLICIT) {
             if constexpr (PDT == RT_DT_BF16)
-                zp = full ? ldg128(t.np + i * 2) : load_raw_guarded<RT_DT_BF16>(t.np, i, n).a;
+                zp = full ? ldg128(x.np + i * 2) : load_raw_guarded<RT_DT_BF16>(x.np, i, n).a;
             if constexpr (MDT == RT_DT_BF16)
-                zm = full ? ldg128(t.nm + i * 2) : load_raw_guarded<RT_DT_BF16>(t.nm, i, n).a;
+                zm = full ? ldg128(x.nm + i * 2) : load_raw_guarded<RT_DT_BF16>(x.nm, i, n).a;
             if constexpr (VDT == RT_DT_BF16)
-                zv = full ? ldg128(t.nv + i * 2) : load_raw_guarded<RT_DT_BF16>(t.nv, i, n).a;
+                zv = full ? ldg128(x.nv + i * 2) : load_raw_guarded<RT_DT_BF16>(x.nv, i, n).a;
         } else {
             philox_noise3<PDT, MDT, VDT>(t, c, i, zp, zm, zv);
         }
         float p[8], g[8], m[8], v[8];
         decode<PDT>(rp, p); decode<GDT>(rg, g); decode<MDT>(rm, m); decode<VDT>(rv, v);
         scale_grads(g, c);
-        if (t.row_mean != 0) {
+        if (x.row_mean != 0) {
             // grad.sub_(mean.mul_(c)): the product is rounded, then subtracted.
             // One division finds the row of the first element; the rest follow by counting.
             const uint64_t e0 = (t.block_base << 3) + i;
-            uint64_t row = e0 / t.row_len;
-            uint64_t rem = e0 - row * t.row_len;
+            uint64_t row = e0 / x.row_len;
+            uint64_t rem = e0 - row * x.row_len;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 if (i + j < n) {
-                    const float mc = cen_term(ldg32f(t.row_mean + row * 4), c.s, c.do_clip, c.coef);
+                    const float mc = cen_term(ldg32f(x.row_mean + row * 4), c.s, c.do_clip, c.coef);
                     g[j] = g[j] - mc;
                 }
-                if (++rem == t.row_len) {
+                if (++rem == x.row_len) {
                     rem = 0;
                     ++row;
                 }
@@ -810,9 +852,9 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_generic_kernel(const Launch
 #pragma unroll
         for (int j = 0; j < 8; ++j) update1(p[j], g[j], m[j], v[j], c.s);
 
-        if (t.dp != 0) store_out_guarded<RT_DT_F32>(t.dp, i, n, p, zp);
-        if (t.dm != 0) store_out_guarded<RT_DT_F32>(t.dm, i, n, m, zm);
-        if (t.dv != 0) store_out_guarded<RT_DT_F32>(t.dv, i, n, v, zv);
+        if (x.dp != 0) store_out_guarded<RT_DT_F32>(x.dp, i, n, p, zp);
+        if (x.dm != 0) store_out_guarded<RT_DT_F32>(x.dm, i, n, m, zm);
+        if (x.dv != 0) store_out_guarded<RT_DT_F32>(x.dv, i, n, v, zv);
         if (full) {
             store_out<PDT>(t.p, i, p, zp);
             store_out<MDT>(t.m, i, m, zm);
@@ -972,7 +1014,8 @@ template <int NOISE>
 __global__ __launch_bounds__(kThreads) void sr_adamw_any_kernel(const LaunchArgs a) {
     if (a.skip != nullptr && load_const(a.skip) != 0u) return;
     const ChunkRef cr = load_const(&a.chunks[blockIdx.x]);
-    const DevTensor t = load_const(&a.tensors[cr.tensor]);
+    const TensorRec t = load_const(&a.tensors[cr.tensor]);
+    const TensorExtra x = load_const(&a.extras[cr.tensor]);
     UpdateCtx c;
     make_ctx(a, t.set_idx, c);
     const rt_scalars s = c.s;
@@ -984,7 +1027,7 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_any_kernel(const LaunchArgs
                    vdt = (t.dtypes >> 6) & 3u;
     const uint64_t n = t.numel;
     const uint64_t chunk_base = (uint64_t)cr.chunk * kChunkElems;
-    const bool plain = (t.dp | t.dm | t.dv | t.row_mean) == 0;
+    const bool plain = (x.dp | x.dm | x.dv | x.row_mean) == 0;
     __shared__ __attribute__((aligned(16))) float stage_all[kThreads / 64][64 * kVec];
 #pragma unroll 1
     for (int it = 0; it < kItersPerChunk; ++it) {
@@ -1004,18 +1047,18 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_any_kernel(const LaunchArgs
             const uint32_t lane = threadIdx.x & 63u;
             float* stage = stage_all[threadIdx.x >> 6];
             if constexpr (NOISE == RT_NOISE_EXPLICIT) {
-                if (pdt == RT_DT_BF16) zp = ldg128(t.np + i * 2);
-                if (mdt == RT_DT_BF16) zm = ldg128(t.nm + i * 2);
-                if (vdt == RT_DT_BF16) zv = ldg128(t.nv + i * 2);
+                if (pdt == RT_DT_BF16) zp = ldg128(x.np + i * 2);
+                if (mdt == RT_DT_BF16) zm = ldg128(x.nm + i * 2);
+                if (vdt == RT_DT_BF16) zv = ldg128(x.nv + i * 2);
             }
             float p[8], g[8], m[8], v[8];
-            auto load8 = [&](uint64_t base, uint32_t dt, float (&x)[8]) {
-                if (dt == RT_DT_F64 || dt == RT_DT_F32) load8_wave_wide(base, dt, w0, lane, stage, x);
-                else load8_any(base, dt, i, x);
+            auto load8 = [&](uint64_t base, uint32_t dt, float (&y)[8]) {
+                if (dt == RT_DT_F64 || dt == RT_DT_F32) load8_wave_wide(base, dt, w0, lane, stage, y);
+                else load8_any(base, dt, i, y);
             };
-            auto store8 = [&](uint64_t base, uint32_t dt, const float (&x)[8], u32x4 noise) {
-                if (dt == RT_DT_F64 || dt == RT_DT_F32) store8_wave_wide(base, dt, w0, lane, stage, x);
-                else store8_any(base, dt, i, x, noise);
+            auto store8 = [&](uint64_t base, uint32_t dt, const float (&y)[8], u32x4 noise) {
+                if (dt == RT_DT_F64 || dt == RT_DT_F32) store8_wave_wide(base, dt, w0, lane, stage, y);
+                else store8_any(base, dt, i, y, noise);
             };
             load8(t.p, pdt, p);
             load8(t.g, gdt, g);
@@ -1036,9 +1079,9 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_any_kernel(const LaunchArgs
         // outputs and centralization go element by element below.
         if (plain && i + kVec <= n) {
             if constexpr (NOISE == RT_NOISE_EXPLICIT) {
-                if (pdt == RT_DT_BF16) zp = ldg128(t.np + i * 2);
-                if (mdt == RT_DT_BF16) zm = ldg128(t.nm + i * 2);
-                if (vdt == RT_DT_BF16) zv = ldg128(t.nv + i * 2);
+                if (pdt == RT_DT_BF16) zp = ldg128(x.np + i * 2);
+                if (mdt == RT_DT_BF16) zm = ldg128(x.nm + i * 2);
+                if (vdt == RT_DT_BF16) zv = ldg128(x.nv + i * 2);
             }
             float p[8], g[8], m[8], v[8];
             load8_any(t.p, pdt, i, p);
@@ -1057,10 +1100,10 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_any_kernel(const LaunchArgs
             continue;
         }
         uint64_t row = 0, rem = 0;
-        if (t.row_mean != 0) {
+        if (x.row_mean != 0) {
             const uint64_t e0 = (t.block_base << 3) + i;
-            row = e0 / t.row_len;
-            rem = e0 - row * t.row_len;
+            row = e0 / x.row_len;
+            rem = e0 - row * x.row_len;
         }
 #pragma unroll 1
         for (int j = 0; j < kVec; ++j) {
@@ -1072,23 +1115,23 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_any_kernel(const LaunchArgs
             float v = load_any(t.v, vdt, e);
             if (do_unscale) g = g * s.inv_loss_scale;
             if (do_clip) g = g * coef;
-            if (t.row_mean != 0) {
-                const float mc = cen_term(ldg32f(t.row_mean + row * 4), s, do_clip, coef);
+            if (x.row_mean != 0) {
+                const float mc = cen_term(ldg32f(x.row_mean + row * 4), s, do_clip, coef);
                 g = g - mc;
-                if (++rem == t.row_len) {
+                if (++rem == x.row_len) {
                     rem = 0;
                     ++row;
                 }
             }
             update1(p, g, m, v, s);
-            if (t.dp != 0) stg32f(t.dp + e * 4, p);
-            if (t.dm != 0) stg32f(t.dm + e * 4, m);
-            if (t.dv != 0) stg32f(t.dv + e * 4, v);
+            if (x.dp != 0) stg32f(x.dp + e * 4, p);
+            if (x.dm != 0) stg32f(x.dm + e * 4, m);
+            if (x.dv != 0) stg32f(x.dv + e * 4, v);
             uint32_t np16, nm16, nv16;
             if constexpr (NOISE == RT_NOISE_EXPLICIT) {
-                np16 = pdt == RT_DT_BF16 ? ldg16(t.np + e * 2) : 0u;
-                nm16 = mdt == RT_DT_BF16 ? ldg16(t.nm + e * 2) : 0u;
-                nv16 = vdt == RT_DT_BF16 ? ldg16(t.nv + e * 2) : 0u;
+                np16 = pdt == RT_DT_BF16 ? ldg16(x.np + e * 2) : 0u;
+                nm16 = mdt == RT_DT_BF16 ? ldg16(x.nm + e * 2) : 0u;
+                nv16 = vdt == RT_DT_BF16 ? ldg16(x.nv + e * 2) : 0u;
             } else {
                 np16 = noise_field(zp, j);
                 nm16 = noise_field(zm, j);
@@ -1569,7 +1612,7 @@ __global__ __launch_bounds__(kThreads) void row_mean_table_long_kernel(const uin
 // For whole tensors of 16-bit arrays with Philox noise whose rows are a multiple of 8
 // and between 512 and kWaveRowMax elements long -- every matrix of a transformer; the host sends
 // everything else through precomputed means.  `first` lists every tensor's first row number in the
-// launch (ascending), `fast_tensors` its record at the same index; workgroup b takes rows 4b .. 4b+3.
+// launch (ascending), `tensors` its record at the same index; workgroup b takes rows 4b .. 4b+3.
 // Two instances, launched apart: rows of at most kRowwiseShortMax elements keep their gradient in
 // registers (158 registers, three waves per SIMD: 2 % faster on such rows than reading it again, 1.4 %
 // slower on long rows if they shared the instance), longer rows read it again (128 registers, four waves).
@@ -1585,11 +1628,11 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_rowwise_kernel(const Launch
     const uint32_t row = blockIdx.x * (kThreads / 64) + wave;
     if (row >= a.n_rows) return;
     const uint32_t ri = find_range(a.first, a.n_ranges, row);   // each wave searches on its own
-    const DevTensor t = load_const(&a.fast_tensors[ri]);
+    const TensorRec t = load_const(&a.tensors[ri]);
     const uint32_t r = row - load_const(&a.first[ri]);
     UpdateCtx c;
     make_ctx(a, t.set_idx, c);
-    const uint32_t row_len = (uint32_t)t.row_len;
+    const uint32_t row_len = (uint32_t)load_const(&a.extras[ri].row_len);
     const uint64_t e0 = (uint64_t)r * row_len;
     const uint64_t tp = t.p, tg = t.g, tm = t.m, tv = t.v;
 

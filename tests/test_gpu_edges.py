@@ -82,3 +82,25 @@ def test_arrays_may_begin_at_any_element(handle, mix, shifts):
             np.testing.assert_array_equal(bits(got[0]), w, err_msg=f"{mix} n={n} {name}")
         for (view, whole), s in zip(views, shifts):
             check_guards(whole, s, n)
+
+
+@pytest.mark.parametrize("rows,row_len", [(1, 8), (3, 9), (1, 511), (64, 27), (2, 4097), (3, 2731), (9, 1820), (17, 482), (1, 33000)])
+def test_centralized_leftovers_take_their_means_in_pieces(handle, rows, row_len):
+    """Centralization with row means given, in tensors whose rows end anywhere inside a vector, a piece or a unit
+    (bf16, Philox noise: whole units and pieces of 512 both take the centralizing instance)."""
+    n = rows * row_len
+    p, g, m, v = oracle.synth_inputs(n, 300 + row_len)
+    (P, wp), (G, _), (M, wm), (V, wv) = (guarded(a, 0, s) for a, s in zip((p, g, m, v), (0, 1, 0, 0)))
+    means = F.row_means(handle, G, rows, row_len)
+    e = F.Entry(p=P, g=G, m=M, v=V, step=4, scalars_idx=0, tensor_id=5, row_mean=means, row_len=row_len)
+    F.step_resident(handle, [e], [F.make_scalars(step=4, centralization=0.75, **HP0)], seed=3, explicit_noise=False)
+    torch.cuda.synchronize()
+    np.testing.assert_allclose(means.cpu().numpy(), oracle.row_means(g, rows, row_len), rtol=3e-6, atol=1e-9)
+    term = means.cpu().numpy() * np.float32(0.75)
+    g32 = (oracle.bf16_to_f32(g).reshape(rows, row_len) - term[:, None]).astype(np.float32).ravel()
+    po, mo, vo = p.copy(), m.copy(), v.copy()
+    oracle.step_tensor(po, g32, mo, vo, oracle.scalars_from_hparams(step=4, **HP0), g_dtype=oracle.DT_F32, seed=3, step=4, tensor_id=5)
+    for got, want in ((P, po), (M, mo), (V, vo)):
+        np.testing.assert_array_equal(bits(got), want.view(np.int16))
+    for whole in (wp, wm, wv):
+        check_guards(whole, 0, n)
