@@ -140,17 +140,23 @@ int rt_step_multi(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, const r
 /*
  * Same update for tensors whose p/m/v (and optionally g) live in pinned host
  * memory: the CPU-resident flow of adamw.py:152-170 (H2D of ema, ema_squared,
- * grad, p) and :204-222 (D2H write-back), restructured as chunks of
- * `chunk_elems` elements moved H2D / updated / moved D2H on three streams with
- * two staging buffers per array.  Waits for work already queued on `stream`
- * (grads ready) and returns after the last D2H has completed, so host memory
+ * grad, p) and :204-222 (D2H write-back).  When every host array of the call is
+ * pinned (and mapped, and not hipHostMallocNonCoherent) the update kernels read
+ * and write it in place over the host link, on a stream of the handle and with
+ * 32 workgroups, and nothing is staged.  Otherwise -- an array in ordinary CPU
+ * memory, explicit noise, more than 512 chunks of 8192 elements with debug
+ * outputs, in a runtime-typed layout or with centralized rows shorter than 8 --
+ * chunks of `chunk_elems` elements are moved H2D / updated / moved D2H on three
+ * streams with two staging buffers per array.  Waits for work already queued on
+ * `stream` (grads ready) and returns when everything is done, so host memory
  * is final on return (the post-condition of the sync at adamw.py:232).
  * Results are bit-identical to rt_step_multi on the same data.
  * d_clip_coef / d_skip: as for rt_step_multi (device pointers, may be NULL);
  * they must be final for work queued on `stream` before the call.
  * Ordering against `stream`: the update kernels always wait for the work queued
- * on it.  This call, which returns only when everything is done, also waits
- * for `stream` on the host before it uploads anything (unless an asynchronous
+ * on it, and in place that is everything there is.  For staged calls: this one,
+ * which returns only when everything is done, also waits for `stream` on the
+ * host before it uploads anything (unless an asynchronous
  * call on the handle is still running), so whatever that work writes into host
  * arrays -- a gradient copied down with grad.to("cpu", non_blocking=True), a
  * parameter refreshed with p.copy_(gpu_tensor, non_blocking=True) -- is final.
@@ -433,7 +439,8 @@ int rt_streamed_bounce_stats(rt_handle* h, uint64_t out[2]);
 /*
  * Per-chunk timeline of the most recent rt_step_streamed made while timing was
  * enabled (rt_set_timing): four floats per chunk, milliseconds since the first
- * H2D began: H2D begin, H2D end, D2H begin, D2H end.  *n_out receives the
+ * H2D began: H2D begin, H2D end, D2H begin, D2H end.  A call that updated host
+ * memory in place has one row, its kernels' time both ways.  *n_out receives the
  * number of floats available; at most `cap` are written to `out` (may be NULL).
  */
 int rt_streamed_timeline(rt_handle* h, float* out, uint32_t cap, uint32_t* n_out);

@@ -59,6 +59,13 @@ constexpr size_t kTimingRing = 256;   // timed launches whose durations can be r
 constexpr uint64_t kMaxGrid = 0x7FFFFFFFull;  // workgroups of one launch (one per chunk of 8192 elements)
 constexpr int kStageBufs = 2;        // device staging buffers per array (chunks in different stages of the pipeline)
 constexpr int kBounce = 4;           // pinned bounce buffers per array for host arrays that are not pinned
+// Updates of host memory in place.  One layer of a Llama-8B-shaped set (218 M bf16 elements, 1.3 GB each way) took
+// 29.6, 27.9, 27.6, 27.8, 28.8, 30.0 ms with 16, 24, 32, 48, 64, 128 workgroups; 40.1 ms through the staged copies.
+constexpr uint32_t kLinkWorkgroups = 32;
+// The generic and the runtime-typed kernel are launched a workgroup per chunk.  Up to this many of them (4 M
+// elements) fill the link no worse than 42 GB/s each way, and such a call would never reach the copies'
+// steady state; with more the call stages (48 GB/s in the long run).
+constexpr uint32_t kLinkChunksMax = 512;
 constexpr uint64_t kPacedInFlight = 2;  // chunks on the streams while the host feeds the pipeline chunk by chunk
 
 struct DevBuf {
@@ -81,6 +88,7 @@ struct TableSlot {
 struct Streamed {
     hipStream_t h2d = nullptr, comp = nullptr, d2h = nullptr;
     hipEvent_t start = nullptr;
+    hipEvent_t in_place_done = nullptr;
     hipEvent_t h2d_done[kStageBufs] = {};
     hipEvent_t comp_done[kStageBufs] = {};
     hipEvent_t d2h_done[kStageBufs] = {};
@@ -257,6 +265,7 @@ struct KernelPair {
     MultiKernel fast;     // whole fast units, plus (Philox) pieces
     MultiKernel generic;  // debug outputs, leftovers of explicit-noise tensors, rows shorter than 8
     MultiKernel fast_cen; // the same with centralization (16-bit layouts, Philox), or NULL
+    MultiKernel link, link_cen;  // fast and fast_cen for arrays in host memory (Philox), or NULL
     MultiKernel rowwise;  // whole tensors with centralization whose row means the kernel takes itself (same layouts), or NULL
     MultiKernel rowwise_short;  // the same for rows of at most kRowwiseShortMax elements
 };
@@ -265,20 +274,25 @@ template <int P, int G, int M, int V>
 static KernelPair pick_noise(int noise) {
     // combinations with an fp32 array use the lane mapping that keeps every access contiguous across the wave
     constexpr bool wide = P == RT_DT_F32 || G == RT_DT_F32 || M == RT_DT_F32 || V == RT_DT_F32;
-    if constexpr (wide) {
-        if (noise == RT_NOISE_EXPLICIT)
-            return {sr_adamw_fast_wide_kernel<P, G, M, V, RT_NOISE_EXPLICIT>,
-                    sr_adamw_generic_kernel<P, G, M, V, RT_NOISE_EXPLICIT>, nullptr, nullptr, nullptr};
-        return {sr_adamw_fast_wide_kernel<P, G, M, V, RT_NOISE_PHILOX>,
-                sr_adamw_generic_kernel<P, G, M, V, RT_NOISE_PHILOX>, nullptr, nullptr, nullptr};
-    } else {
-        if (noise == RT_NOISE_EXPLICIT)
-            return {sr_adamw_fast_kernel<P, G, M, V, RT_NOISE_EXPLICIT>,
-                    sr_adamw_generic_kernel<P, G, M, V, RT_NOISE_EXPLICIT>, nullptr, nullptr, nullptr};
-        return {sr_adamw_fast_kernel<P, G, M, V, RT_NOISE_PHILOX>, sr_adamw_generic_kernel<P, G, M, V, RT_NOISE_PHILOX>,
-                sr_adamw_fast_kernel<P, G, M, V, RT_NOISE_PHILOX, true>, sr_adamw_rowwise_kernel<P, G, M, V, false>,
-                sr_adamw_rowwise_kernel<P, G, M, V, true>};
+    KernelPair k{};
+    if (noise == RT_NOISE_EXPLICIT) {
+        k.generic = sr_adamw_generic_kernel<P, G, M, V, RT_NOISE_EXPLICIT>;
+        if constexpr (wide) k.fast = sr_adamw_fast_wide_kernel<P, G, M, V, RT_NOISE_EXPLICIT>;
+        else k.fast = sr_adamw_fast_kernel<P, G, M, V, RT_NOISE_EXPLICIT>;
+        return k;
     }
+    k.generic = sr_adamw_generic_kernel<P, G, M, V, RT_NOISE_PHILOX>;
+    k.link = sr_adamw_link_kernel<P, G, M, V, false>;
+    if constexpr (wide) {
+        k.fast = sr_adamw_fast_wide_kernel<P, G, M, V, RT_NOISE_PHILOX>;
+    } else {
+        k.fast = sr_adamw_fast_kernel<P, G, M, V, RT_NOISE_PHILOX>;
+        k.fast_cen = sr_adamw_fast_kernel<P, G, M, V, RT_NOISE_PHILOX, true>;
+        k.link_cen = sr_adamw_link_kernel<P, G, M, V, true>;
+        k.rowwise = sr_adamw_rowwise_kernel<P, G, M, V, false>;
+        k.rowwise_short = sr_adamw_rowwise_kernel<P, G, M, V, true>;
+    }
+    return k;
 }
 // State dtype pairs the templated kernels are instantiated for: every bf16 / fp32 mix, and both fp16.
 template <int P, int G>
@@ -625,7 +639,7 @@ static int stage_image(rt_handle* h, const Plan& plan, const uint8_t* img, uint6
 // few microseconds a marker before and after a dispatch adds.
 static int enqueue_kernels(const Plan& plan, const uint8_t* base, uint64_t seed, int noise_mode,
                            const float* d_clip_coef, const uint32_t* d_skip, hipStream_t stream,
-                           hipEvent_t t_begin = nullptr, hipEvent_t t_end = nullptr) {
+                           hipEvent_t t_begin = nullptr, hipEvent_t t_end = nullptr, bool over_link = false) {
     LaunchArgs a;
     memset(&a, 0, sizeof(a));
     a.sets = (const DevScalars*)(base + plan.off_sets);
@@ -661,11 +675,12 @@ static int enqueue_kernels(const Plan& plan, const uint8_t* base, uint64_t seed,
             const uint64_t grid = (uint64_t)piece_wgs + grp.n_units;
             if (!grid) continue;
             if (grid > kMaxGrid) return fail(RT_EUNSUPPORTED, "too many workgroups in one launch");
-            const MultiKernel kern = c ? k.fast_cen : k.fast;
+            const MultiKernel kern = over_link ? (c ? k.link_cen : k.link) : c ? k.fast_cen : k.fast;
             if (!kern) return fail(RT_EHIP, "internal: units without a kernel for them");
-            launches.push_back(Launch{kern, (uint32_t)grid, a});
+            launches.push_back(Launch{kern, over_link ? std::min((uint32_t)grid, kLinkWorkgroups) : (uint32_t)grid, a});
             LaunchArgs& x = launches.back().args;
             records_from(x, grp.first_tensor);
+            x.n_wgs = (uint32_t)grid;
             x.n_ranges = grp.n_ranges;
             x.piece_tensor = (const uint32_t*)(base + plan.off_piece_tensor) + grp.first_piece;
             x.n_pieces = grp.n_pieces;
@@ -866,6 +881,7 @@ int rt_destroy(rt_handle* h) {
     if (st.ticket_word) (void)hipHostFree((void*)st.ticket_word);
     for (hipEvent_t e : st.tl_events) (void)hipEventDestroy(e);
     if (st.start) (void)hipEventDestroy(st.start);
+    if (st.in_place_done) (void)hipEventDestroy(st.in_place_done);
     if (st.h2d) (void)hipStreamDestroy(st.h2d);
     if (st.comp) (void)hipStreamDestroy(st.comp);
     if (st.d2h) (void)hipStreamDestroy(st.d2h);
@@ -1174,7 +1190,8 @@ static int streamed_init(rt_handle* h) {
     // memory, say) can be repeated without leaking what the first attempt created.
     for (hipStream_t* s : {&st.h2d, &st.comp, &st.d2h})
         if (!*s) HIP_TRY(hipStreamCreateWithFlags(s, hipStreamNonBlocking));
-    if (!st.start) HIP_TRY(hipEventCreateWithFlags(&st.start, hipEventDisableTiming));
+    for (hipEvent_t* e : {&st.start, &st.in_place_done})
+        if (!*e) HIP_TRY(hipEventCreateWithFlags(e, hipEventDisableTiming));
     for (int b = 0; b < kStageBufs; ++b)
         for (hipEvent_t* e : {&st.h2d_done[b], &st.comp_done[b], &st.d2h_done[b]})
             if (!*e) HIP_TRY(hipEventCreateWithFlags(e, hipEventDisableTiming));
@@ -1368,9 +1385,12 @@ static bool sleep_until_word(const volatile uint64_t* word, uint64_t want) {
     if (!word) return false;
     auto read_word = [word] { return __atomic_load_n((const uint64_t*)word, __ATOMIC_ACQUIRE); };
     uint64_t seen = read_word();
-    auto last_progress = std::chrono::steady_clock::now();
+    const auto begin = std::chrono::steady_clock::now();
+    auto last_progress = begin;
     while (seen < want) {
-        std::this_thread::sleep_for(std::chrono::microseconds(100));
+        // a fraction of the time waited so far: a short call is not kept waiting longer than it ran
+        const auto waited = std::chrono::duration_cast<std::chrono::microseconds>(std::chrono::steady_clock::now() - begin);
+        std::this_thread::sleep_for(std::clamp(waited / 64, std::chrono::microseconds(5), std::chrono::microseconds(100)));
         const uint64_t now_done = read_word();
         const auto now = std::chrono::steady_clock::now();
         if (now_done != seen) {
@@ -1427,6 +1447,154 @@ struct FillGuard {
 };
 }  // namespace
 
+// A pool entry for one call's table image (`bytes` at `image`), with the image in its pinned memory.
+static int streamed_table(rt_handle* h, const uint8_t* image, size_t bytes, Streamed::TableRing** out) {
+    Streamed& st = h->st;
+    int rc = RT_OK;
+    // A free pool entry (the call that used it has published its ticket), preferably one that is
+    // already large enough.  With every entry in use the host sleeps until the oldest call is
+    // done -- reading the ticket word, not waiting inside the runtime.
+    size_t slot = st.ring.size();
+    for (;;) {
+        const uint64_t done_now = tickets_done(st);
+        uint64_t oldest = UINT64_MAX;
+        for (size_t i = 0; i < st.ring.size(); ++i) {
+            Streamed::TableRing& r = st.ring[i];
+            if (r.in_flight && r.ticket <= done_now) r.in_flight = false;
+            if (r.in_flight) oldest = std::min(oldest, r.ticket);
+            if (!r.in_flight && (slot == st.ring.size() || (st.ring[slot].host_cap < bytes && r.host_cap >= bytes)))
+                slot = i;
+        }
+        if (slot != st.ring.size()) break;
+        if (!sleep_until_ticket(st, oldest)) {
+            rc = streamed_wait(h);  // blocking fallback; frees every entry or reports the device error
+            if (rc != RT_OK) return rc;
+        }
+    }
+    Streamed::TableRing& tab = st.ring[slot];
+    if (bytes > tab.host_cap) {
+        if (tab.host) HIP_TRY(hipHostFree(tab.host));
+        tab.host = nullptr;
+        tab.host_cap = 0;
+        const size_t want = bytes + bytes / 4 + 4096;
+        hipError_t e = hipHostMalloc(&tab.host, want, hipHostMallocDefault);
+        if (e != hipSuccess) return fail(RT_ENOMEM, "hipHostMalloc(%zu) failed: %s", want, hipGetErrorString(e));
+        tab.host_cap = want;
+    }
+    rc = dev_reserve(tab.dev, bytes + 16);
+    if (rc != RT_OK) return rc;
+    memcpy(tab.host, image, bytes);
+    *out = &tab;
+    return RT_OK;
+}
+
+// Brings the image of `tab` into its device memory, on the compute stream.
+static int upload_table(rt_handle* h, const Streamed::TableRing& tab, size_t bytes) {
+    if (bytes == 0) return RT_OK;
+    const uint64_t n_vec = (bytes + 15) / 16;  // buffers are padded well past the image
+    const uint32_t grid = (uint32_t)std::min<uint64_t>((n_vec + kThreads - 1) / kThreads, 64);
+    hipLaunchKernelGGL(table_upload_kernel, dim3(grid), dim3(kThreads), 0, h->st.comp, (uint64_t)tab.dev.ptr,
+                       (uint64_t)tab.host, n_vec);
+    HIP_TRY(hipGetLastError());
+    return RT_OK;
+}
+
+// The last thing a streamed call queues: a kernel on the download stream that publishes the call's ticket.
+static int issue_ticket(rt_handle* h, Streamed::TableRing& tab) {
+    Streamed& st = h->st;
+    tab.ticket = st.tickets_issued + 1;
+    tab.in_flight = true;
+    ++st.tickets_issued;
+    hipLaunchKernelGGL(publish_ticket_kernel, dim3(1), dim3(1), 0, st.d2h, (uint64_t)st.ticket_word, st.tickets_issued);
+    HIP_TRY(hipGetLastError());
+    return RT_OK;
+}
+
+// ---------------------------------------------------------------------------
+// Updating host memory in place.  The kernels of a call whose host arrays are all pinned read and write
+// them over the host link themselves: no staging, no copies, one pass.  Loads and stores of different
+// waves share the link in both directions all the time, which chunks of a copy pipeline do only while
+// one chunk goes up as another comes down -- the first goes up and the last comes down alone.
+// ---------------------------------------------------------------------------
+
+// The address under which kernels reach `bytes` bytes of pinned host memory at `host`, or NULL.  Both ends
+// must belong to pinned memory that is mapped contiguously; memory made with hipHostMallocNonCoherent
+// stays with the copies (a kernel's writes may linger in the L2s).
+static void* mapped_host(const void* host, size_t bytes) {
+    hipPointerAttribute_t first, last;
+    memset(&first, 0, sizeof(first));
+    memset(&last, 0, sizeof(last));
+    if (hipPointerGetAttributes(&first, host) != hipSuccess ||
+        hipPointerGetAttributes(&last, (const uint8_t*)host + bytes - 1) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (first.type != hipMemoryTypeHost || last.type != hipMemoryTypeHost || !first.devicePointer ||
+        (uint8_t*)last.devicePointer != (uint8_t*)first.devicePointer + (bytes - 1) ||
+        (first.allocationFlags & hipHostMallocNonCoherent) != 0)
+        return nullptr;
+    return first.devicePointer;
+}
+
+// The descriptors with every host array replaced by its mapped address; false if one has none.
+static bool map_host_arrays(const rt_tensor_desc* descs, uint32_t n, std::vector<rt_tensor_desc>& out, double& bytes_up,
+                            double& bytes_down) {
+    out.assign(descs, descs + n);
+    bytes_up = bytes_down = 0;
+    for (rt_tensor_desc& d : out) {
+        const uint32_t mask = d.host_mask;
+        d.host_mask = 0;
+        if (d.numel == 0) continue;
+        const int es[4] = {dtype_size(d.p_dtype), dtype_size(d.g_dtype), dtype_size(d.m_dtype), dtype_size(d.v_dtype)};
+        void* at[4] = {d.p, (void*)d.g, d.m, d.v};
+        for (int a = 0; a < 4; ++a) {
+            if (!(mask & (1u << a))) continue;
+            const size_t bytes = d.numel * es[a];
+            at[a] = mapped_host(at[a], bytes);
+            if (!at[a]) return false;
+            bytes_up += (double)bytes;
+            if (a != 1) bytes_down += (double)bytes;
+        }
+        d.p = at[0]; d.g = at[1]; d.m = at[2]; d.v = at[3];
+    }
+    return true;
+}
+
+// Enqueues one call whose table image (`plan`, h->image) addresses host memory directly.
+static int streamed_in_place(rt_handle* h, const Plan& plan, uint64_t seed, const float* d_clip_coef,
+                             const uint32_t* d_skip, hipStream_t user, bool trace) {
+    Streamed& st = h->st;
+    Streamed::TableRing* tab = nullptr;
+    int rc = streamed_table(h, h->image.data(), plan.bytes, &tab);
+    if (rc != RT_OK) return rc;
+    // the kernels wait for everything queued on the caller's stream, whichever arrays it writes
+    HIP_TRY(hipEventRecord(st.start, user));
+    HIP_TRY(hipStreamWaitEvent(st.comp, st.start, 0));
+    st.pending = true;
+    rc = upload_table(h, *tab, plan.bytes);
+    if (rc != RT_OK) return rc;
+    if (trace) {   // one row: up and down are one kernel's time
+        while (st.tl_events.size() < 4) {
+            hipEvent_t e;
+            HIP_TRY(hipEventCreate(&e));
+            st.tl_events.push_back(e);
+        }
+        for (int k = 0; k < 4; k += 2) HIP_TRY(hipEventRecord(st.tl_events[k], st.comp));
+    }
+    rc = enqueue_kernels(plan, (const uint8_t*)tab->dev.ptr, seed, RT_NOISE_PHILOX, d_clip_coef, d_skip, st.comp,
+                         nullptr, nullptr, /*over_link=*/true);
+    if (rc != RT_OK) return rc;
+    if (trace)
+        for (int k = 1; k < 4; k += 2) HIP_TRY(hipEventRecord(st.tl_events[k], st.comp));
+    // tickets are published in order, behind the copies of earlier calls
+    HIP_TRY(hipEventRecord(st.in_place_done, st.comp));
+    HIP_TRY(hipStreamWaitEvent(st.d2h, st.in_place_done, 0));
+    rc = issue_ticket(h, *tab);
+    if (rc != RT_OK) return rc;
+    if (trace) st.timeline.assign(4, 0.0f);
+    return RT_OK;
+}
+
 // Validates and enqueues the whole pipeline of one call; does not wait for it.
 static int streamed_enqueue_impl(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, const rt_scalars* scalars,
                             uint32_t n_scalars, uint64_t seed, int noise_mode, uint64_t chunk_elems,
@@ -1450,6 +1618,29 @@ static int streamed_enqueue_impl(rt_handle* h, const rt_tensor_desc* descs, uint
     Streamed& st = h->st;
     if (ticket_out) *ticket_out = st.tickets_issued;  // nothing to wait for beyond what is already issued
     if (n == 0) return RT_OK;
+
+    // ---- everything on the host pinned, and (nearly) every tensor one of the fast kernels': no copies at
+    //      all.  Explicit noise stages; so do many chunks with debug outputs, of runtime-typed layouts or of
+    //      centralized rows shorter than 8 elements.
+    if (noise_mode == RT_NOISE_PHILOX) {
+        std::vector<rt_tensor_desc> mapped;
+        double up = 0, down = 0;
+        if (map_host_arrays(descs, n, mapped, up, down)) {
+            Plan plan;
+            build_image(h, mapped.data(), n, scalars, /*want_explicit=*/false, plan, h->image);
+            uint64_t n_generic = 0;
+            for (const Batch& b : plan.batches) n_generic += b.n_generic;
+            if (n_generic <= kLinkChunksMax) {
+                rc = streamed_in_place(h, plan, seed, d_clip_coef, d_skip, user, trace);
+                if (rc != RT_OK) return rc;
+                st.bytes_h2d = up;
+                st.bytes_d2h = down;
+                if (!trace) st.timeline.clear();
+                if (ticket_out) *ticket_out = st.tickets_issued;
+                return RT_OK;
+            }
+        }
+    }
 
     // ---- cut the tensor list into chunks of at most chunk_elems staged elements
     std::vector<std::vector<Segment>> chunks;
@@ -1586,39 +1777,10 @@ static int streamed_enqueue_impl(rt_handle* h, const rt_tensor_desc* descs, uint
         blob.resize(plan_off[c] + plans[c].bytes);
         if (plans[c].bytes) memcpy(blob.data() + plan_off[c], h->image.data(), plans[c].bytes);
     }
-    // A free pool entry (the call that used it has published its ticket), preferably one that is
-    // already large enough.  With every entry in use the host sleeps until the oldest call is
-    // done -- reading the ticket word, not waiting inside the runtime.
-    size_t slot = st.ring.size();
-    for (;;) {
-        const uint64_t done_now = tickets_done(st);
-        uint64_t oldest = UINT64_MAX;
-        for (size_t i = 0; i < st.ring.size(); ++i) {
-            Streamed::TableRing& r = st.ring[i];
-            if (r.in_flight && r.ticket <= done_now) r.in_flight = false;
-            if (r.in_flight) oldest = std::min(oldest, r.ticket);
-            if (!r.in_flight && (slot == st.ring.size() || (st.ring[slot].host_cap < blob.size() && r.host_cap >= blob.size())))
-                slot = i;
-        }
-        if (slot != st.ring.size()) break;
-        if (!sleep_until_ticket(st, oldest)) {
-            rc = streamed_wait(h);  // blocking fallback; frees every entry or reports the device error
-            if (rc != RT_OK) return rc;
-        }
-    }
-    Streamed::TableRing& tab = st.ring[slot];
-    if (blob.size() > tab.host_cap) {
-        if (tab.host) HIP_TRY(hipHostFree(tab.host));
-        tab.host = nullptr;
-        tab.host_cap = 0;
-        const size_t want = blob.size() + blob.size() / 4 + 4096;
-        hipError_t e = hipHostMalloc(&tab.host, want, hipHostMallocDefault);
-        if (e != hipSuccess) return fail(RT_ENOMEM, "hipHostMalloc(%zu) failed: %s", want, hipGetErrorString(e));
-        tab.host_cap = want;
-    }
-    rc = dev_reserve(tab.dev, blob.size() + 16);
+    Streamed::TableRing* tab_slot = nullptr;
+    rc = streamed_table(h, blob.data(), blob.size(), &tab_slot);
     if (rc != RT_OK) return rc;
-    memcpy(tab.host, blob.data(), blob.size());
+    Streamed::TableRing& tab = *tab_slot;
 
     // grads (and anything else already queued by the caller) must be ready
     // The kernels read device arrays (gradients above all) that work on the caller's stream may still
@@ -1644,13 +1806,8 @@ static int streamed_enqueue_impl(rt_handle* h, const rt_tensor_desc* descs, uint
     if (blocking && !st.pending) HIP_TRY(hipStreamSynchronize(user));
     else if (upload_waits) HIP_TRY(hipStreamWaitEvent(st.h2d, st.start, 0));
     HIP_TRY(hipStreamWaitEvent(st.comp, st.start, 0));
-    if (!blob.empty()) {
-        const uint64_t n_vec = (blob.size() + 15) / 16;  // buffers are padded well past the blob
-        const uint32_t grid = (uint32_t)std::min<uint64_t>((n_vec + kThreads - 1) / kThreads, 64);
-        hipLaunchKernelGGL(table_upload_kernel, dim3(grid), dim3(kThreads), 0, st.comp, (uint64_t)tab.dev.ptr,
-                           (uint64_t)tab.host, n_vec);
-        HIP_TRY(hipGetLastError());
-    }
+    rc = upload_table(h, tab, blob.size());
+    if (rc != RT_OK) return rc;
 
     st.bytes_h2d = st.bytes_d2h = 0;
     st.timeline.clear();
@@ -1766,14 +1923,10 @@ static int streamed_enqueue_impl(rt_handle* h, const rt_tensor_desc* descs, uint
                 break;
             case RT_OP_TICKET:
                 st.seq += chunks.size();
-                tab.ticket = st.tickets_issued + 1;
-                tab.in_flight = true;
-                // ticket: published when the last D2H of this call has landed (D2H follows compute, so
+                // published when the last D2H of this call has landed (D2H follows compute, so
                 // device-resident arrays are final by then as well)
-                ++st.tickets_issued;
-                hipLaunchKernelGGL(publish_ticket_kernel, dim3(1), dim3(1), 0, st.d2h, (uint64_t)st.ticket_word,
-                                   st.tickets_issued);
-                HIP_TRY(hipGetLastError());
+                rc = issue_ticket(h, tab);
+                if (rc != RT_OK) return rc;
                 break;
             default: return fail(RT_EHIP, "internal: unknown operation %u in the schedule", op.kind);
         }

@@ -77,7 +77,8 @@ struct LaunchArgs {
     const float* clip_coef;         // optional device float: grads are multiplied by it
     const uint32_t* skip;           // optional device flag: non-zero leaves everything untouched
     uint32_t n_ranges, n_pieces, n_piece_wgs;
-    uint32_t piece_rate;            // how piece workgroups are spread over the grid, see unit_or_pieces
+    uint32_t piece_rate;            // how piece workgroups are spread over the launch, see unit_or_pieces
+    uint32_t n_wgs;                 // workgroups' worth of work (units, and groups of four pieces) in the launch; see sr_adamw_link_kernel
     uint32_t seed_lo, seed_hi;
     uint32_t use_ks;                // every tensor of the launch uses one DevScalars: `ks`, no table read
     uint32_t n_rows;                // row-wise kernel: rows in the launch

@@ -402,13 +402,12 @@ __device__ __forceinline__ uint32_t find_range(const uint32_t* __restrict__ firs
 // ---------------------------------------------------------------------------
 // Which part of a launch a workgroup serves.  Piece workgroups (four pieces each, one per wavefront)
 // are spread evenly among the unit workgroups: of the first b workgroups, min(n_piece_wgs,
-// floor(b * piece_rate / 2^32)) serve pieces (piece_rate = ceil(n_piece_wgs * 2^32 / gridDim.x), or 0 when the
+// floor(b * piece_rate / 2^32)) serve pieces (piece_rate = ceil(n_piece_wgs * 2^32 / n_wgs), or 0 when the
 // launch has only pieces).  Pieces are bound by instruction issue and by the latency of their short
 // dependent chains, units by memory: resident side by side they overlap.
 // Returns true for units and then the unit's number, false for pieces and then the wavefront's piece.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ bool unit_or_pieces(const LaunchArgs& a, uint32_t& which) {
-    const uint32_t b = blockIdx.x;
+__device__ __forceinline__ bool unit_or_pieces(const LaunchArgs& a, uint32_t b, uint32_t& which) {
     uint32_t pieces_before = b, pieces_after = b + 1u;
     if (a.piece_rate != 0u) {
         pieces_before = min(a.n_piece_wgs, __umulhi(b, a.piece_rate));
@@ -509,16 +508,8 @@ __device__ __forceinline__ void piece_body(const LaunchArgs& a, uint32_t q) {
 // ---------------------------------------------------------------------------
 // CEN: the tensors of the launch have their gradients centralized by row means computed before.  Rows are
 // at least 8 elements long (shorter ones take the generic kernel).
-template <int PDT, int GDT, int MDT, int VDT, int NOISE, bool CEN = false>
-__global__ __launch_bounds__(kThreads) void sr_adamw_fast_kernel(const LaunchArgs a) {
-    if (a.skip != nullptr && load_const(a.skip) != 0u) return;
-    uint32_t unit;
-    if (!unit_or_pieces(a, unit)) {
-        if constexpr (NOISE == RT_NOISE_PHILOX) {
-            if (unit < a.n_pieces) piece_body<PDT, GDT, MDT, VDT, CEN>(a, unit);
-        }
-        return;
-    }
+template <int PDT, int GDT, int MDT, int VDT, int NOISE, bool CEN>
+__device__ __forceinline__ void unit_body(const LaunchArgs& a, uint32_t unit) {
     const uint32_t ri = find_range(a.first, a.n_ranges, unit);
     const TensorRec t = load_const(&a.tensors[ri]);
     const uint32_t unit_in_tensor = unit - load_const(&a.first[ri]);
@@ -613,6 +604,17 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_fast_kernel(const LaunchArg
     }
 }
 
+template <int PDT, int GDT, int MDT, int VDT, int NOISE, bool CEN = false>
+__global__ __launch_bounds__(kThreads) void sr_adamw_fast_kernel(const LaunchArgs a) {
+    if (a.skip != nullptr && load_const(a.skip) != 0u) return;
+    uint32_t which;
+    if (unit_or_pieces(a, blockIdx.x, which)) {
+        unit_body<PDT, GDT, MDT, VDT, NOISE, CEN>(a, which);
+    } else if constexpr (NOISE == RT_NOISE_PHILOX) {
+        if (which < a.n_pieces) piece_body<PDT, GDT, MDT, VDT, CEN>(a, which);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Fast kernel for dtype combinations with an fp32 array.  With 8 consecutive
 // elements per lane an fp32 array would be read as two 16-byte accesses 16
@@ -690,15 +692,7 @@ __device__ __forceinline__ void store_out4(uint64_t base, uint64_t e, const floa
 }
 
 template <int PDT, int GDT, int MDT, int VDT, int NOISE>
-__global__ __launch_bounds__(kThreads) void sr_adamw_fast_wide_kernel(const LaunchArgs a) {
-    if (a.skip != nullptr && load_const(a.skip) != 0u) return;
-    uint32_t unit;
-    if (!unit_or_pieces(a, unit)) {
-        if constexpr (NOISE == RT_NOISE_PHILOX) {
-            if (unit < a.n_pieces) piece_body<PDT, GDT, MDT, VDT, false>(a, unit);
-        }
-        return;
-    }
+__device__ __forceinline__ void unit_body_wide(const LaunchArgs& a, uint32_t unit) {
     const uint32_t ri = find_range(a.first, a.n_ranges, unit);
     const TensorRec t = load_const(&a.tensors[ri]);
     const uint32_t unit_in_tensor = unit - load_const(&a.first[ri]);
@@ -784,6 +778,41 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_fast_wide_kernel(const Laun
             store_out4<PDT>(tp, e, p, zp[h]);
             store_out4<MDT>(tm, e, m, zm[h]);
             store_out4<VDT>(tv, e, v, zv[h]);
+        }
+    }
+}
+
+template <int PDT, int GDT, int MDT, int VDT, int NOISE>
+__global__ __launch_bounds__(kThreads) void sr_adamw_fast_wide_kernel(const LaunchArgs a) {
+    if (a.skip != nullptr && load_const(a.skip) != 0u) return;
+    uint32_t which;
+    if (unit_or_pieces(a, blockIdx.x, which)) {
+        unit_body_wide<PDT, GDT, MDT, VDT, NOISE>(a, which);
+    } else if constexpr (NOISE == RT_NOISE_PHILOX) {
+        if (which < a.n_pieces) piece_body<PDT, GDT, MDT, VDT, false>(a, which);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The two fast kernels for host memory: p, g, m, v (or some of them) are pinned host arrays that the kernel
+// reads and writes over the host link.  The link bounds it (57 GB/s one way, 48.4 GB/s each way when both
+// are busy, where HBM does 6400), and a few workgroups' loads fill it: with 8, 16, 32, 64, 256, 1024 of them a
+// math-free probe of this traffic moved 46, 47, 48, 46, 43, 41 GB/s each way.  So kLinkWorkgroups workgroups
+// walk the launch's work a grid apart, and the other CUs stay free for whatever else runs -- the
+// backward pass whose hooks call this.  An instance of its own: the loop around the same bodies takes 136
+// vector registers instead of 99, which would cost the kernel above its fourth wave per SIMD.
+// ---------------------------------------------------------------------------
+template <int PDT, int GDT, int MDT, int VDT, bool CEN>
+__global__ __launch_bounds__(kThreads) void sr_adamw_link_kernel(const LaunchArgs a) {
+    constexpr bool kWide = PDT == RT_DT_F32 || GDT == RT_DT_F32 || MDT == RT_DT_F32 || VDT == RT_DT_F32;
+    if (a.skip != nullptr && load_const(a.skip) != 0u) return;
+    for (uint32_t b = blockIdx.x; b < a.n_wgs; b += gridDim.x) {
+        uint32_t which;
+        if (unit_or_pieces(a, b, which)) {
+            if constexpr (kWide) unit_body_wide<PDT, GDT, MDT, VDT, RT_NOISE_PHILOX>(a, which);
+            else unit_body<PDT, GDT, MDT, VDT, RT_NOISE_PHILOX, CEN>(a, which);
+        } else if (which < a.n_pieces) {
+            piece_body<PDT, GDT, MDT, VDT, CEN>(a, which);
         }
     }
 }

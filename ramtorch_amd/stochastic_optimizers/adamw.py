@@ -106,7 +106,8 @@ class AdamW(Optimizer):
 
     Keyword-only additions (not in the reference):
         seed: Philox key of the rounding noise.
-        stream_chunk_bytes: bytes of bf16 per staged chunk of the host-resident path.
+        stream_chunk_bytes: bytes of bf16 per staged chunk of the host-resident path (pinned arrays are updated
+            in place over the host link and not staged).
         loss_scale: gradients are divided by this inside the kernel.
         max_grad_norm: global L2 clip computed on the GPU before the update.  A non-finite norm
             cancels the step on the GPU (nothing is written) and the step counts it had advanced are

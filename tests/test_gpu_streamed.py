@@ -452,3 +452,100 @@ def test_max_grad_norm_with_host_resident_params_and_states(grads_on):
 def test_host_link_probe_reports_plausible_rates(handle):
     r = handle.host_link_probe(64 << 20, reps=4)
     assert all(5.0 < r[k] < 200.0 for k in ("h2d_GBps", "d2h_GBps", "duplex_GBps_each_way")), r
+
+
+# bf16 p/g/m/v; fp32 gradient and second moment; fp32 parameters; fp16; a runtime-typed pair of states
+LAYOUTS = [("bf16",) * 4, ("bf16", "f32", "bf16", "f32"), ("f32", "f32", "bf16", "bf16"), ("f16",) * 4, ("bf16", "bf16", "f16", "bf16")]
+DTYPES = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}
+
+
+@pytest.mark.parametrize("layout", LAYOUTS, ids="-".join)
+@pytest.mark.parametrize("central", [False, True])
+@pytest.mark.parametrize("host", ["pgmv", "mv", "p"])
+def test_pinned_arrays_are_updated_in_place(handle, layout, central, host):
+    """The kernels that work on pinned host memory themselves against the resident ones, bit for bit: lengths
+    around a piece (512), a unit (8192) and one round of the 32 workgroups, arrays that begin at odd elements
+    of their pinned buffers, arrays partly on the GPU, rows of 7 (generic kernel) and of 8 and more."""
+    rows = [1, 3, 64, 512, 1171, 3]   # with the row lengths below: 7, 24, 512, 4096, 8197, 32 units and 5 elements
+    lens = [7, 24, 512, 4096, 8197, 33 * 8192 + 9]
+    gen = torch.Generator().manual_seed(5)
+    pair = []
+    for i, n in enumerate(lens):
+        row = n // rows[i]
+        n = row * rows[i]
+        vals = [torch.randn(n, generator=gen) * s for s in (0.02, 1e-3, 1e-4, 1e-3)]
+        vals[3] = vals[3] ** 2
+        both = []
+        for where in ("cuda", "host"):
+            arrays = []
+            for k, x in zip("pgmv", vals):
+                x = x.to(DTYPES[layout["pgmv".index(k)]])
+                if where == "host" and k in host:
+                    buf = torch.empty(n + 3, dtype=x.dtype).pin_memory()
+                    buf[i % 3:i % 3 + n] = x
+                    x = buf[i % 3:i % 3 + n]
+                else:
+                    x = x.cuda()
+                arrays.append(x)
+            e = F.Entry(p=arrays[0], g=arrays[1], m=arrays[2], v=arrays[3], step=9, scalars_idx=0, tensor_id=i)
+            if central:
+                e.row_mean, e.row_len = vals[1].view(rows[i], row).mean(1).cuda(), row
+            both.append(e)
+        pair.append(both)
+    sc = [F.make_scalars(step=9, centralization=1.0 if central else 0.0, **HP0)]
+    clip = torch.tensor([0.5, 0.5], device="cuda")
+    F.step_resident(handle, [r for r, _ in pair], sc, seed=3, explicit_noise=False, clip_coef=clip[:1])
+    handle.set_timing(True)
+    F.step_streamed(handle, [s for _, s in pair], sc, seed=3, explicit_noise=False, chunk_elems=4096, clip_coef=clip[:1])
+    rows_of_timeline = len(handle.streamed_timeline())
+    handle.set_timing(False)
+    assert rows_of_timeline == 1     # staged, these lengths would be dozens of chunks
+    torch.cuda.synchronize()
+    for i, (r, s) in enumerate(pair):
+        for name in "pmv":
+            assert nmis(getattr(r, name), getattr(s, name)) == 0, (lens[i], name)
+    # a set skip flag leaves host memory alone
+    before = [getattr(s, k).clone() for _, s in pair for k in "pmv"]
+    skip = torch.ones(1, dtype=torch.int32, device="cuda")
+    F.step_streamed(handle, [s for _, s in pair], sc, seed=3, explicit_noise=False, chunk_elems=4096, clip_coef=clip[:1], skip=skip)
+    torch.cuda.synchronize()
+    assert all(nmis(a, b) == 0 for a, b in zip(before, (getattr(s, k) for _, s in pair for k in "pmv")))
+
+
+def test_in_place_and_staged_calls_take_turns(handle):
+    """Asynchronous calls that alternate between both ways finish in order, and a finished ticket means final
+    host memory either way."""
+    n, state = 700_001, []
+    for i in range(6):
+        p, g, m, v = oracle.synth_inputs(n, 800 + i)
+        state.append((p, g, m, v, F.Entry(p=host16(p, pin=i % 2 == 0), g=dev16(g), m=host16(m), v=host16(v), step=2,
+                                          scalars_idx=0, tensor_id=i)))
+    sc = [F.make_scalars(step=2, **HP0)]
+    torch.cuda.synchronize()
+    tickets = [F.step_streamed(handle, [s[-1]], sc, seed=6, explicit_noise=False, chunk_elems=65_536, wait=False) for s in state]
+    assert tickets == sorted(set(tickets))
+    handle.streamed_wait()
+    assert handle.streamed_completed() == tickets[-1]
+    for i, (p, g, m, v, e) in enumerate(state):
+        oracle.step_tensor(p, g, m, v, oracle.scalars_from_hparams(step=2, **HP0), seed=6, step=2, tensor_id=i)
+        for name, t, a in zip("pmv", (e.p, e.m, e.v), (p, m, v)):
+            np.testing.assert_array_equal(bits16(t), a, err_msg=f"{i} {name}")
+
+
+@pytest.mark.parametrize("chunk_elems", [8, 4096, 65_536])
+def test_pinned_arrays_with_explicit_noise_are_staged(handle, chunk_elems):
+    """The copy pipeline queued up front (nothing unpinned), cut into many chunks."""
+    lens = [n for n in LENS if n < 10_000] if chunk_elems < 64 else LENS
+    sc, sco = F.make_scalars(step=10, **HP0), oracle.scalars_from_hparams(step=10, **HP0)
+    entries, inputs = [], []
+    for i, n in enumerate(lens):
+        arrays, noise = oracle.synth_inputs(n, 70 + i), oracle.synth_noise(n, 70 + i)
+        nz = tuple(torch.from_numpy(z.view(np.int16).copy()).cuda() for z in noise)
+        p, g, m, v = arrays
+        entries.append(F.Entry(p=host16(p), g=dev16(g), m=host16(m), v=host16(v), step=10, scalars_idx=0, tensor_id=i, noise=nz))
+        inputs.append((arrays, noise))
+    F.step_streamed(handle, entries, [sc], seed=0, explicit_noise=True, chunk_elems=chunk_elems)
+    for e, ((p, g, m, v), noise) in zip(entries, inputs):
+        oracle.step_tensor(p, g, m, v, sco, noise=noise)
+        for name, t, a in zip("pmv", (e.p, e.m, e.v), (p, m, v)):
+            np.testing.assert_array_equal(bits16(t), a, err_msg=f"chunk {chunk_elems} n={len(p)} {name}")
