@@ -79,7 +79,7 @@ struct TableSlot {
     DevBuf dev;
     void* host = nullptr;  // pinned; keeps the image last uploaded to `dev`
     size_t host_cap = 0;
-    size_t valid_bytes = 0;  // bytes of `host` that `dev` currently mirrors
+    size_t valid_from = 0, valid_bytes = 0;  // `dev` currently mirrors bytes valid_from .. valid_bytes of `host`
     uint64_t static_gen = 0; // layout generation of the lists behind the scalars, 0 = unknown
     hipEvent_t done = nullptr;
     bool in_flight = false;
@@ -163,7 +163,7 @@ struct Plan {
     size_t off_sets = 0, off_tensors = 0, off_extras = 0, off_first = 0, off_piece_tensor = 0, off_chunks = 0, bytes = 0;
     uint32_t n_sets = 0, n_tensors = 0;
     bool has_extras = false;
-    DevScalars first_set;   // passed by value when n_sets == 1
+    DevScalars arg_sets[kArgSets] = {};   // passed by value when n_sets <= kArgSets
     std::vector<Batch> batches;
     std::vector<std::pair<uint32_t, uint32_t>> set_keys;  // set index -> (scalars_idx, step)
 };
@@ -530,7 +530,7 @@ static void build_image(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, c
     for (const auto& kv : set_index) plan.set_keys[kv.second] = kv.first;
     plan.n_sets = (uint32_t)sets.size();
     plan.n_tensors = (uint32_t)count;
-    if (!sets.empty()) plan.first_set = sets[0];
+    if (!sets.empty()) memcpy(plan.arg_sets, sets.data(), std::min<size_t>(sets.size(), kArgSets) * sizeof(DevScalars));
     plan.off_sets = 0;
     plan.off_tensors = align_up(sets.size() * sizeof(DevScalars), 256);
     plan.off_extras = plan.off_tensors + align_up(count * sizeof(TensorRec), 128);
@@ -613,20 +613,20 @@ static int stage_image(rt_handle* h, const Plan& plan, const uint8_t* img, uint6
         if (rc != RT_OK) return rc;
     }
     // Two regions: the DevScalars sets change with every step, the lists behind them only when the
-    // tensors do; each region is copied only if the device copy differs.
-    const size_t split = std::min(plan.off_tensors, plan.bytes);
-    const bool known = s.valid_bytes == plan.bytes;
-    if (split > 0 && !(known && memcmp(s.host, img, split) == 0)) {
-        memcpy(s.host, img, split);
-        HIP_TRY(hipMemcpyAsync(s.dev.ptr, s.host, split, hipMemcpyHostToDevice, stream));
+    // tensors do; what differs from the device copy goes up in one copy.  Sets that travel as kernel
+    // arguments are not uploaded at all, so steps over the same tensors copy nothing.
+    const size_t lists = std::min(plan.off_tensors, plan.bytes);
+    const size_t begin = plan.n_sets <= kArgSets ? lists : 0;
+    const bool known = s.valid_bytes == plan.bytes && s.valid_from <= begin;
+    const bool same_sets = begin == lists || (known && memcmp(s.host, img, lists) == 0);
+    const bool same_lists = known && ((static_gen != 0 && s.static_gen == static_gen) ||
+                                      memcmp((uint8_t*)s.host + lists, img + lists, plan.bytes - lists) == 0);
+    const size_t lo = same_sets ? lists : 0, hi = same_lists ? lists : plan.bytes;
+    if (lo < hi) {
+        memcpy((uint8_t*)s.host + lo, img + lo, hi - lo);
+        HIP_TRY(hipMemcpyAsync((uint8_t*)s.dev.ptr + lo, (uint8_t*)s.host + lo, hi - lo, hipMemcpyHostToDevice, stream));
     }
-    const bool same_gen = known && static_gen != 0 && s.static_gen == static_gen;
-    if (plan.bytes > split && !same_gen &&
-        !(known && memcmp((uint8_t*)s.host + split, img + split, plan.bytes - split) == 0)) {
-        memcpy((uint8_t*)s.host + split, img + split, plan.bytes - split);
-        HIP_TRY(hipMemcpyAsync((uint8_t*)s.dev.ptr + split, (uint8_t*)s.host + split, plan.bytes - split,
-                               hipMemcpyHostToDevice, stream));
-    }
+    s.valid_from = begin;
     s.valid_bytes = plan.bytes;
     s.static_gen = static_gen;
     *out = &s;
@@ -647,8 +647,8 @@ static int enqueue_kernels(const Plan& plan, const uint8_t* base, uint64_t seed,
     a.skip = d_skip;
     a.seed_lo = (uint32_t)seed;
     a.seed_hi = (uint32_t)(seed >> 32);
-    a.use_ks = plan.n_sets == 1 ? 1u : 0u;
-    a.ks = plan.first_set;
+    a.n_arg_sets = plan.n_sets <= kArgSets ? plan.n_sets : 0u;
+    memcpy(a.arg_sets, plan.arg_sets, sizeof(a.arg_sets));
     struct Launch {
         MultiKernel kernel;
         uint32_t grid;
@@ -759,7 +759,7 @@ static int launch_update(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, 
             sets[j].s = scalars[key.first];
             sets[j].step = key.second;
         }
-        if (!lc.plan.set_keys.empty()) lc.plan.first_set = sets[0];
+        memcpy(lc.plan.arg_sets, sets, std::min<size_t>(lc.plan.set_keys.size(), kArgSets) * sizeof(DevScalars));
         if (delta != 0)
             for (uint32_t i = 0; i < n; ++i) lc.descs[i].step = descs[i].step;
     } else {

@@ -1,6 +1,7 @@
 // Records the update kernels read from device memory, and the launch geometry
 // shared by host and device code.  gfx950 only.
 #pragma once
+#include <stddef.h>
 #include <stdint.h>
 
 #include "../../include/ramtorch_sr_adamw.h"
@@ -66,6 +67,11 @@ constexpr uint32_t kFastUnitElems = kThreads * kVec * kFastIters;
 // has drained (17.7 M elements in 160 ragged fp32 tensors: 66 + 10.5 us of kernels, 66 us with pieces).
 constexpr uint32_t kPieceElems = 64 * kVec;  // 512: one 128-bit vector per lane
 
+// Sets of scalars that travel as kernel arguments.  They are what changes from step to step while the tensors
+// stay where they are: as part of the table they cost a copy in front of every launch (2.5 us of host time and as much
+// on the GPU).  Four cover two param groups at two step counts; 64 bytes of arguments cost 0.04 us a launch.
+constexpr uint32_t kArgSets = 4;
+
 // Kernel arguments of the update kernels (passed by value).
 struct LaunchArgs {
     const TensorRec* tensors;       // the launch's records; tensors with whole units first
@@ -80,9 +86,9 @@ struct LaunchArgs {
     uint32_t piece_rate;            // how piece workgroups are spread over the launch, see unit_or_pieces
     uint32_t n_wgs;                 // workgroups' worth of work (units, and groups of four pieces) in the launch; see sr_adamw_link_kernel
     uint32_t seed_lo, seed_hi;
-    uint32_t use_ks;                // every tensor of the launch uses one DevScalars: `ks`, no table read
+    uint32_t n_arg_sets;            // 1: every tensor of the launch uses arg_sets[0]; 2 .. kArgSets: the launch's sets; 0: they are in `sets`
     uint32_t n_rows;                // row-wise kernel: rows in the launch
-    DevScalars ks;
+    DevScalars arg_sets[kArgSets];
 };
 
 }  // namespace rt

@@ -363,11 +363,15 @@ __device__ __forceinline__ float cen_term(float mean, const rt_scalars& s, bool 
 // Launch-uniform set-up shared by the update kernels.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void make_ctx(const LaunchArgs& a, uint32_t set_idx, UpdateCtx& c) {
-    if (a.use_ks != 0u) {  // the usual case: one param group at one step count; no table read
-        c.s = a.ks.s;
-        c.step = a.ks.step;
+    if (a.n_arg_sets == 1u) {  // the usual case: one param group at one step count; set_idx need not have arrived
+        c.s = a.arg_sets[0].s;
+        c.step = a.arg_sets[0].step;
     } else {
-        const DevScalars set = load_const(&a.sets[set_idx]);
+        // (LaunchArgs is the update kernels' only argument, so their argument segment begins with it)
+        const DevScalars* sets = a.sets;
+        if (a.n_arg_sets != 0u)
+            sets = (const DevScalars*)((uint64_t)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(LaunchArgs, arg_sets));
+        const DevScalars set = load_const(&sets[set_idx]);
         c.s = set.s;
         c.step = set.step;
     }

@@ -104,3 +104,22 @@ def test_centralized_leftovers_take_their_means_in_pieces(handle, rows, row_len)
         np.testing.assert_array_equal(bits(got), want.view(np.int16))
     for whole in (wp, wm, wv):
         check_guards(whole, 0, n)
+
+
+def test_scalar_sets_reach_the_kernels_as_arguments_or_through_the_table(handle):
+    """One set, as many as travel as kernel arguments, and more, in turn over the same tensors (whole units and
+    pieces): the table images have equal lists, and a change of way must not leave one set behind."""
+    lens = [8192, 513, 3 * 8192 + 7, 64, 9, 16384]
+    cpu = [list(oracle.synth_inputs(n, 600 + k)) for k, n in enumerate(lens)]
+    dev = [[torch.from_numpy(a.view(np.int16).copy()).view(torch.bfloat16).cuda() for a in arrays] for arrays in cpu]
+    for round_, n_sets in enumerate((1, 1, 4, 5, 5, 6, 4, 2, 3, 5, 1)):
+        steps = [100 * (round_ + 1) + k % n_sets for k in range(len(lens))]
+        scalars = [F.make_scalars(step=100 * (round_ + 1) + j, **HP0) for j in range(n_sets)]
+        F.step_resident(handle, [F.Entry(p=d[0], g=d[1], m=d[2], v=d[3], step=steps[k], scalars_idx=k % n_sets, tensor_id=k)
+                                 for k, d in enumerate(dev)], scalars, seed=9, explicit_noise=False)
+        for k, a in enumerate(cpu):
+            oracle.step_tensor(a[0], a[1], a[2], a[3], oracle.scalars_from_hparams(step=steps[k], **HP0), seed=9,
+                               step=steps[k], tensor_id=k)
+        for k, (d, a) in enumerate(zip(dev, cpu)):
+            for name, got, want in zip("pmv", (d[0], d[2], d[3]), (a[0], a[2], a[3])):
+                np.testing.assert_array_equal(bits(got), want.view(np.int16), err_msg=f"round {round_}, {n_sets} sets, tensor {k} {name}")
