@@ -183,6 +183,12 @@ def lib() -> ctypes.CDLL:
     L.rt_streamed_stats.argtypes = [vp, ctypes.POINTER(ctypes.c_double)]
     L.rt_streamed_bounce_stats.restype = i32
     L.rt_streamed_bounce_stats.argtypes = [vp, ctypes.POINTER(ctypes.c_uint64)]
+    # the same entry points with the descriptors' address as a plain number
+    for name in ("rt_step_multi", "rt_grad_norm", "rt_row_means_multi"):
+        fn = L[name]
+        fn.restype = i32
+        fn.argtypes = [vp] + [vp if t in (descs, scal) else t for t in getattr(L, name).argtypes[1:]]
+        setattr(L, name + "_at", fn)
     v = L.rt_version()
     if v != ABI_VERSION:
         raise RuntimeError(f"{LIB_PATH} has ABI version {v}, this package expects {ABI_VERSION}; rebuild it")
@@ -233,6 +239,19 @@ class Handle:
         with self._lock:
             check(lib().rt_step_multi(self.ptr, descs, n, scalars, n_scalars, seed, noise_mode, d_clip_coef,
                                       d_skip, stream))
+
+    def step_multi_at(self, descs_addr, n, scalars, n_scalars, seed, noise_mode, d_clip_coef, d_skip, stream):
+        with self._lock:
+            check(lib().rt_step_multi_at(self.ptr, descs_addr, n, scalars, n_scalars, seed, noise_mode, d_clip_coef,
+                                         d_skip, stream))
+
+    def grad_norm_at(self, descs_addr, n, inv_loss_scale, max_norm, d_out, stream):
+        with self._lock:
+            check(lib().rt_grad_norm_at(self.ptr, descs_addr, n, inv_loss_scale, max_norm, d_out, stream))
+
+    def row_means_multi_at(self, descs_addr, n, inv_loss_scale, stream):
+        with self._lock:
+            check(lib().rt_row_means_multi_at(self.ptr, descs_addr, n, inv_loss_scale, stream))
 
     def step_streamed(self, descs, n, scalars, n_scalars, seed, noise_mode, chunk_elems, d_clip_coef=None,
                       d_skip=None, stream=0):

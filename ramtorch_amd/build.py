@@ -80,7 +80,7 @@ def build_gather(verbose: bool = False) -> str:
 
     os.makedirs(LIB_DIR, exist_ok=True)
     torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-unused-function",
+    cmd = [os.environ.get("CXX", "g++"), "-O3", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-unused-function",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            "-I" + sysconfig.get_paths()["include"]]
     cmd += ["-I" + i for i in cpp_extension.include_paths()]

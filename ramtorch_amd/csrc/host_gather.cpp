@@ -18,6 +18,7 @@
 #include <algorithm>
 #include <cstring>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include "../../include/ramtorch_sr_adamw.h"
@@ -29,6 +30,7 @@ namespace {
 PyObject* k_ema = nullptr;
 PyObject* k_ema_squared = nullptr;
 PyObject* k_step = nullptr;
+Py_hash_t h_ema = 0, h_ema_squared = 0, h_step = 0;
 PyTypeObject* t_tensor = nullptr;     // torch.Tensor
 PyTypeObject* t_parameter = nullptr;  // torch.nn.Parameter
 
@@ -43,9 +45,11 @@ inline bool exact_tensor(PyObject* o) {
     return t == t_tensor || t == t_parameter;
 }
 
+inline const c10::TensorImpl* impl_of(PyObject* o) { return THPVariable_Unpack(o).unsafeGetTensorImpl(); }
+
 // dtype code of a param / state (bf16, f32, f16, f64) or -1
-inline int pmv_code(const at::Tensor& t) {
-    switch (t.scalar_type()) {
+inline int pmv_code(const c10::TensorImpl* t) {
+    switch (c10::typeMetaToScalarType(t->dtype())) {
         case at::kBFloat16: return RT_DT_BF16;
         case at::kFloat: return RT_DT_F32;
         case at::kHalf: return RT_DT_F16;
@@ -55,31 +59,42 @@ inline int pmv_code(const at::Tensor& t) {
 }
 
 // dtype code of a gradient (bf16, f32, f16) or -1
-inline int grad_code(const at::Tensor& t) {
-    switch (t.scalar_type()) {
-        case at::kBFloat16: return RT_DT_BF16;
-        case at::kFloat: return RT_DT_F32;
-        case at::kHalf: return RT_DT_F16;
-        default: return -1;
-    }
+inline int grad_code(const c10::TensorImpl* t) {
+    const int code = pmv_code(t);
+    return code == RT_DT_F64 ? -1 : code;
 }
 
 // dev >= 0: on that GPU; dev < 0: in host memory (exercised by the CPU-only tests of this
 // helper; the optimizer only ever passes a GPU index)
-inline bool dense_on(const at::Tensor& t, int dev) {
-    if (t.layout() != at::kStrided || !t.is_contiguous()) return false;
-    return dev >= 0 ? (t.is_cuda() && t.get_device() == dev) : t.is_cpu();
+inline bool dense_on(const c10::TensorImpl* t, int dev) {
+    if (t->layout() != at::kStrided || !t->is_contiguous()) return false;
+    return dev >= 0 ? (t->is_cuda() && t->get_device() == dev) : t->is_cpu();
+}
+
+inline void* data_of(const c10::TensorImpl* t) { return const_cast<c10::TensorImpl*>(t)->mutable_data(); }
+
+// A state dict's entry (borrowed) or NULL.  With the hash at hand a lookup costs half of PyDict_GetItem, which also
+// saves and restores the interpreter's error state.
+inline PyObject* entry(PyObject* dict, PyObject* key, Py_hash_t hash) {
+#if PY_VERSION_HEX < 0x030D0000
+    PyObject* o = _PyDict_GetItem_KnownHash(dict, key, hash);
+    if (!o && PyErr_Occurred()) PyErr_Clear();   // a foreign key's comparison failed: not there
+    return o;
+#else
+    (void)hash;
+    return PyDict_GetItem(dict, key);
+#endif
 }
 
 // The walk below is a chain of dependent loads per tensor (list item -> Python wrapper ->
 // TensorImpl -> autograd meta -> gradient -> storage, and the same through the state dict), and
 // with tens of thousands of tensors none of it is in cache: the chain's latency is the cost.
 // Warm runs ahead of the main loop as a software pipeline: level k of the chain is prefetched
-// for tensor i + (kLevels - k) * kLead while tensor i is processed, so each level finds the
-// previous one already in cache.  It reads what the main loop reads and decides nothing.
-constexpr int kLevels = 5;
-constexpr Py_ssize_t kLead = 6;
-constexpr Py_ssize_t kRing = 64;  // > kLevels * kLead
+// for tensor i + (5 - k) * kLead while tensor i is processed, so each level finds the
+// previous one already in cache.  It hands what it has read to the main loop and decides nothing.  Nothing runs in between
+// that could change it: of what it holds, the main loop only replaces a state's step.
+constexpr size_t kLead = 6;
+constexpr size_t kRing = 64;  // > 5 * kLead, a power of two
 
 inline void touch(const void* p, int lines = 1) {
     const char* c = static_cast<const char*>(p);
@@ -89,76 +104,99 @@ inline void touch(const void* p, int lines = 1) {
 struct Warm {
     PyObject* params;
     PyObject* states;
-    Py_ssize_t n;
-    const c10::TensorImpl* impl[kRing][4];
-    PyObject* obj[kRing][3];
+    PyObject* grads;   // list or NULL
+    size_t n;
+    // What the walk has found out about tensor i, at i % kRing: the main loop uses it too.
+    const c10::TensorImpl* impl[kRing][4];   // p, gradient, ema, ema_squared; NULL: none, or not an exact Tensor / Parameter
+    PyObject* obj[kRing][3];                 // the state's ema, ema_squared, step (borrowed) or NULL
 
-    void level(int k, Py_ssize_t i) {
-        if (i < 0 || i >= n) return;
-        const Py_ssize_t r = i % kRing;
+    template <int LEVEL>
+    void level(size_t i) {
+        if (i >= n) return;
+        const size_t r = i % kRing;
         PyObject* po = PyList_GET_ITEM(params, i);
         PyObject* so = PyList_GET_ITEM(states, i);
-        switch (k) {
-            case 0:  // wrappers and dict headers
-                touch(po);
-                touch(so);
-                break;
-            case 1:  // TensorImpl of the param; key table of the dict
-                impl[r][0] = exact_tensor(po) ? THPVariable_Unpack(po).unsafeGetTensorImpl() : nullptr;
-                if (impl[r][0]) touch(impl[r][0], 4);
-                if (PyDict_CheckExact(so)) touch(reinterpret_cast<PyDictObject*>(so)->ma_keys, 4);
-                break;
-            case 2:  // autograd meta + storage of the param; state objects
-                if (impl[r][0]) {
-                    touch(impl[r][0]->autograd_meta(), 2);
-                    touch(impl[r][0]->unsafe_storage().unsafeGetStorageImpl());
-                }
-                obj[r][0] = obj[r][1] = obj[r][2] = nullptr;
-                if (PyDict_CheckExact(so)) {
-                    obj[r][0] = PyDict_GetItem(so, k_ema);
-                    obj[r][1] = PyDict_GetItem(so, k_ema_squared);
-                    obj[r][2] = PyDict_GetItem(so, k_step);
-                    for (int j = 0; j < 3; ++j)
-                        if (obj[r][j]) touch(obj[r][j]);
-                }
-                break;
-            case 3:  // TensorImpl of the gradient and of both states
-                impl[r][1] = impl[r][2] = impl[r][3] = nullptr;
-                if (impl[r][0]) {
-                    const at::Tensor& g = THPVariable_Unpack(po).grad();
-                    if (g.defined()) impl[r][1] = g.unsafeGetTensorImpl();
-                }
-                for (int j = 0; j < 2; ++j)
-                    if (obj[r][j] && exact_tensor(obj[r][j]))
-                        impl[r][2 + j] = THPVariable_Unpack(obj[r][j]).unsafeGetTensorImpl();
-                for (int j = 1; j < 4; ++j)
-                    if (impl[r][j]) touch(impl[r][j], 4);
-                break;
-            default:  // their storages
-                for (int j = 1; j < 4; ++j)
-                    if (impl[r][j]) touch(impl[r][j]->unsafe_storage().unsafeGetStorageImpl());
+        if constexpr (LEVEL == 0) {   // wrappers and dict headers
+            touch(po);
+            touch(so);
+            if (grads) touch(PyList_GET_ITEM(grads, i));
+        } else if constexpr (LEVEL == 1) {   // TensorImpl of the param; key table of the dict
+            impl[r][0] = exact_tensor(po) ? impl_of(po) : nullptr;
+            if (impl[r][0]) touch(impl[r][0], 4);
+            if (PyDict_CheckExact(so)) touch(reinterpret_cast<PyDictObject*>(so)->ma_keys, 4);
+        } else if constexpr (LEVEL == 2) {   // autograd meta + storage of the param; state objects
+            if (impl[r][0]) {
+                if (!grads) touch(impl[r][0]->autograd_meta(), 2);
+                touch(impl[r][0]->unsafe_storage().unsafeGetStorageImpl());
+            }
+            obj[r][0] = obj[r][1] = obj[r][2] = nullptr;
+            if (PyDict_CheckExact(so)) {
+                obj[r][0] = entry(so, k_ema, h_ema);
+                obj[r][1] = entry(so, k_ema_squared, h_ema_squared);
+                obj[r][2] = entry(so, k_step, h_step);
+                for (int j = 0; j < 3; ++j)
+                    if (obj[r][j]) touch(obj[r][j]);
+            }
+        } else if constexpr (LEVEL == 3) {   // TensorImpl of the gradient and of both states
+            impl[r][1] = nullptr;
+            if (grads) {
+                PyObject* go = PyList_GET_ITEM(grads, i);
+                if (exact_tensor(go)) impl[r][1] = impl_of(go);
+            } else if (impl[r][0]) {
+                const at::Tensor& g = THPVariable_Unpack(po).grad();
+                if (g.defined()) impl[r][1] = g.unsafeGetTensorImpl();
+            }
+            for (int j = 0; j < 2; ++j)
+                impl[r][2 + j] = obj[r][j] && exact_tensor(obj[r][j]) ? impl_of(obj[r][j]) : nullptr;
+            for (int j = 1; j < 4; ++j)
+                if (impl[r][j]) touch(impl[r][j], 4);
+        } else {   // their storages
+            for (int j = 1; j < 4; ++j)
+                if (impl[r][j]) touch(impl[r][j]->unsafe_storage().unsafeGetStorageImpl());
         }
     }
 
-    // called before tensor i is processed
-    void ahead_of(Py_ssize_t i) {
+    // called before tensor i is processed; afterwards its entries are complete
+    void ahead_of(size_t i) {
         if (i == 0) {  // fill the pipeline
-            for (int k = 0; k < kLevels; ++k)
-                for (Py_ssize_t j = 0; j < (kLevels - k) * kLead; ++j) level(k, j);
+            for (size_t j = 0; j < 5 * kLead; ++j) level<0>(j);
+            for (size_t j = 0; j < 4 * kLead; ++j) level<1>(j);
+            for (size_t j = 0; j < 3 * kLead; ++j) level<2>(j);
+            for (size_t j = 0; j < 2 * kLead; ++j) level<3>(j);
+            for (size_t j = 0; j < 1 * kLead; ++j) level<4>(j);
         }
-        for (int k = 0; k < kLevels; ++k) level(k, i + (kLevels - k) * kLead);
+        level<0>(i + 5 * kLead);
+        level<1>(i + 4 * kLead);
+        level<2>(i + 3 * kLead);
+        level<3>(i + 2 * kLead);
+        level<4>(i + 1 * kLead);
     }
 };
 
-// gather_group(params, states, dev, desc_addr, desc_cap, status_addr, scalars_base, tensor_id_base)
-//   -> (rows_written, [distinct new step values, in order of first use])
+// Whether the update can take the row means of such a tensor itself (the rule of the library's row-wise kernel).
+inline bool sums_rows_itself(const rt_tensor_desc& d) {
+    constexpr uint64_t kMin = 512, kMax = 32768;   // elements of a row
+    const auto narrow = [](uint8_t dt) { return dt == RT_DT_BF16 || dt == RT_DT_F16; };
+    return d.row_len % 8 == 0 && d.row_len >= kMin && d.row_len <= kMax && narrow(d.p_dtype) && narrow(d.g_dtype) &&
+           narrow(d.m_dtype) && narrow(d.v_dtype) && (d.m_dtype == RT_DT_F16) == (d.v_dtype == RT_DT_F16);
+}
+
+// gather_group(params, states, dev, desc_addr, desc_cap, status_addr, scalars_base, tensor_id_base
+//              [, grads, centralize])
+//   -> (rows_written, [distinct new step values, in order of first use]
+//       [, tensors left to the caller, row means needed])
 // params: list of tensors; states: list of the per-param state dicts (same order);
 // desc_addr / desc_cap: address and capacity (rows) of an rt_tensor_desc buffer;
 // status_addr: address of a uint8 buffer with len(params) entries.
 // Row r of a written tensor gets scalars_idx = scalars_base + (index of its step in the returned list).
+// grads: None (every parameter's own .grad), or a list of the gradients to use, None for no gradient.
+// centralize: 0, 1 or 2.  Rows get their row_len (adamw.py:179-184: the mean is over every dim but the first, over all
+// of them for 0-d / 1-d); with 2 the update takes the means itself where it can; every other row gets its
+// place among the means, counted in floats from 1, in row_mean (see place_row_means).
+// A call that fails has changed no step count.
 PyObject* gather_group(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-    if (nargs != 8) {
-        PyErr_SetString(PyExc_TypeError, "gather_group takes 8 arguments");
+    if (nargs != 8 && nargs != 10) {
+        PyErr_SetString(PyExc_TypeError, "gather_group takes 8 or 10 arguments");
         return nullptr;
     }
     PyObject* params = args[0];
@@ -173,66 +211,77 @@ PyObject* gather_group(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     auto* status = reinterpret_cast<uint8_t*>(PyLong_AsUnsignedLongLong(args[5]));
     const unsigned long scalars_base = PyLong_AsUnsignedLong(args[6]);
     const unsigned long id_base = PyLong_AsUnsignedLong(args[7]);
+    PyObject* grads = nargs == 10 && args[8] != Py_None ? args[8] : nullptr;
+    const long centralize = nargs == 10 ? PyLong_AsLong(args[9]) : 0;
     if (PyErr_Occurred()) return nullptr;
     const Py_ssize_t n = PyList_GET_SIZE(params);
-    if (PyList_GET_SIZE(states) != n || !rows || !status) {
-        PyErr_SetString(PyExc_ValueError, "params / states length mismatch or NULL buffer");
+    if (PyList_GET_SIZE(states) != n || !rows || !status || (grads && (!PyList_CheckExact(grads) || PyList_GET_SIZE(grads) != n))) {
+        PyErr_SetString(PyExc_ValueError, "params / states length mismatch, NULL buffer, or grads is not a list of that length");
         return nullptr;
     }
-    std::vector<long long> steps;
-    Py_ssize_t w = 0;
+    // (new step, its number as a Python int): tensors at the same step share the object
+    std::vector<std::pair<long long, PyObject*>> steps;
+    Py_ssize_t w = 0, left = 0;
+    uint64_t means = 0;
+    bool failed = false;
     Warm warm;
     warm.params = params;
     warm.states = states;
-    warm.n = n;
-    for (Py_ssize_t i = 0; i < n; ++i) {
+    warm.grads = grads;
+    warm.n = (size_t)n;
+    Py_ssize_t i = 0;
+    for (; i < n; ++i) {
         warm.ahead_of(i);
         status[i] = kPython;
+        ++left;
         PyObject* po = PyList_GET_ITEM(params, i);
         PyObject* so = PyList_GET_ITEM(states, i);
-        if (!exact_tensor(po) || !PyDict_CheckExact(so)) continue;
-        const at::Tensor& p = THPVariable_Unpack(po);
-        const at::Tensor& g = p.grad();
-        if (!g.defined()) {
+        const c10::TensorImpl* const* im = warm.impl[(size_t)i % kRing];
+        const c10::TensorImpl *p = im[0], *g = im[1], *m = im[2], *v = im[3];
+        if (!p || !PyDict_CheckExact(so)) continue;
+        if (!g) {
+            if (grads && PyList_GET_ITEM(grads, i) != Py_None) continue;
             status[i] = kNoGrad;
+            --left;
             continue;
         }
         if (w >= cap) continue;
-        PyObject* mo = PyDict_GetItem(so, k_ema);           // borrowed
-        PyObject* vo = PyDict_GetItem(so, k_ema_squared);
-        PyObject* st = PyDict_GetItem(so, k_step);
-        if (!mo || !vo || !st || !exact_tensor(mo) || !exact_tensor(vo) || !PyLong_CheckExact(st)) continue;
-        const at::Tensor& m = THPVariable_Unpack(mo);
-        const at::Tensor& v = THPVariable_Unpack(vo);
+        PyObject* st = entry(so, k_step, h_step);   // (not the one found ahead: the same dict may have had its turn since)
+        if (!m || !v || !st || !PyLong_CheckExact(st)) continue;
         const int pc = pmv_code(p), mc = pmv_code(m), vc = pmv_code(v), gc = grad_code(g);
         if (pc < 0 || mc < 0 || vc < 0 || gc < 0) continue;
         if (!dense_on(p, (int)dev) || !dense_on(g, (int)dev) || !dense_on(m, (int)dev) || !dense_on(v, (int)dev))
             continue;
-        const int64_t numel = p.numel();
-        if (g.numel() != numel || m.numel() != numel || v.numel() != numel) continue;
+        const int64_t numel = p->numel();
+        if (g->numel() != numel || m->numel() != numel || v->numel() != numel) continue;
         int overflow = 0;
         const long long step = PyLong_AsLongLongAndOverflow(st, &overflow);
         if (overflow || step < 0) continue;
         const long long new_step = step + 1;  // adamw.py:177
-        PyObject* ns = PyLong_FromLongLong(new_step);
-        if (!ns) return nullptr;
-        const int rc = PyDict_SetItem(so, k_step, ns);
-        Py_DECREF(ns);
-        if (rc != 0) return nullptr;
         size_t si = steps.size();
         for (size_t k = steps.size(); k-- > 0;)
-            if (steps[k] == new_step) {
+            if (steps[k].first == new_step) {
                 si = k;
                 break;
             }
-        if (si == steps.size()) steps.push_back(new_step);
+        if (si == steps.size()) {
+            PyObject* ns = PyLong_FromLongLong(new_step);
+            if (!ns) {
+                failed = true;
+                break;
+            }
+            steps.emplace_back(new_step, ns);
+        }
+        if (PyDict_SetItem(so, k_step, steps[si].second) != 0) {
+            failed = true;
+            break;
+        }
 
-        rt_tensor_desc& d = rows[w++];
-        std::memset(&d, 0, sizeof(d));
-        d.p = p.data_ptr();
-        d.g = g.data_ptr();
-        d.m = m.data_ptr();
-        d.v = v.data_ptr();
+        rt_tensor_desc d{};
+        d.p = data_of(p);
+        d.g = data_of(g);
+        d.m = data_of(m);
+        d.v = data_of(v);
         d.numel = (uint64_t)numel;
         d.tensor_id = (uint32_t)(id_base + (unsigned long)i);
         d.step = (uint32_t)((unsigned long long)new_step & 0xFFFFFFFFull);
@@ -242,19 +291,55 @@ PyObject* gather_group(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         d.m_dtype = (uint8_t)mc;
         d.v_dtype = (uint8_t)vc;
         status[i] = kWritten;
-    }
-    PyObject* lst = PyList_New((Py_ssize_t)steps.size());
-    if (!lst) return nullptr;
-    for (size_t k = 0; k < steps.size(); ++k) {
-        PyObject* v = PyLong_FromLongLong(steps[k]);
-        if (!v) {
-            Py_DECREF(lst);
-            return nullptr;
+        --left;
+        if (centralize && numel > 0) {
+            const uint64_t count = g->dim() >= 2 ? (uint64_t)g->size(0) : 1;
+            d.row_len = (uint64_t)numel / count;
+            if (centralize != 2 || !sums_rows_itself(d)) {
+                d.row_mean = reinterpret_cast<float*>(means + 1);
+                means += count;
+            }
         }
-        PyList_SET_ITEM(lst, (Py_ssize_t)k, v);
+        rows[w++] = d;
     }
-    PyObject* out = Py_BuildValue("(nN)", w, lst);
+    PyObject* out = nullptr;
+    if (!failed) {
+        PyObject* lst = PyList_New((Py_ssize_t)steps.size());
+        for (size_t k = 0; lst && k < steps.size(); ++k) {
+            Py_INCREF(steps[k].second);
+            PyList_SET_ITEM(lst, (Py_ssize_t)k, steps[k].second);
+        }
+        if (lst) out = nargs == 10 ? Py_BuildValue("(nNnK)", w, lst, left, (unsigned long long)means) : Py_BuildValue("(nN)", w, lst);
+    }
+    if (!out) {   // put the step counts back; the error stays set
+        PyObject *type, *value, *trace;
+        PyErr_Fetch(&type, &value, &trace);
+        for (Py_ssize_t k = 0, r = 0; k < i; ++k) {
+            if (status[k] != kWritten) continue;
+            PyObject* old = PyLong_FromLongLong(steps[rows[r++].scalars_idx - scalars_base].first - 1);
+            if (!old || PyDict_SetItem(PyList_GET_ITEM(states, k), k_step, old) != 0) PyErr_Clear();
+            Py_XDECREF(old);
+        }
+        PyErr_Restore(type, value, trace);
+    }
+    for (auto& s : steps) Py_DECREF(s.second);
     return out;
+}
+
+// place_row_means(desc_addr, rows, base_addr): turns the places gather_group left in row_mean into addresses
+// in the buffer of means at base_addr.
+PyObject* place_row_means(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    if (nargs != 3) {
+        PyErr_SetString(PyExc_TypeError, "place_row_means takes 3 arguments");
+        return nullptr;
+    }
+    auto* rows = reinterpret_cast<rt_tensor_desc*>(PyLong_AsUnsignedLongLong(args[0]));
+    const Py_ssize_t n = PyLong_AsSsize_t(args[1]);
+    auto* base = reinterpret_cast<float*>(PyLong_AsUnsignedLongLong(args[2]));
+    if (PyErr_Occurred()) return nullptr;
+    for (Py_ssize_t r = 0; r < n; ++r)
+        if (rows[r].row_mean) rows[r].row_mean = base + (reinterpret_cast<uint64_t>(rows[r].row_mean) - 1);
+    Py_RETURN_NONE;
 }
 
 // verify_layout(params, expect_addr, n) -> bool
@@ -308,7 +393,7 @@ bool verify_range(PyObject* params, const uint64_t* expect, Py_ssize_t lo, Py_ss
             continue;
         }
         if (want == 0 || g.layout() != at::kStrided || !g.is_contiguous() || g.numel() != p.numel() ||
-            reinterpret_cast<uint64_t>(g.data_ptr()) != want || (uint64_t)grad_code(g) != expect[3 * i + 2])
+            reinterpret_cast<uint64_t>(g.data_ptr()) != want || (uint64_t)grad_code(g.unsafeGetTensorImpl()) != expect[3 * i + 2])
             return false;
     }
     return true;
@@ -424,6 +509,8 @@ PyObject* set_types(PyObject*, PyObject* args) {
 PyMethodDef methods[] = {
     {"gather_group", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(gather_group)), METH_FASTCALL,
      "rt_tensor_desc rows of the plain tensors of one param group"},
+    {"place_row_means", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(place_row_means)), METH_FASTCALL,
+     "addresses of the row means of gathered rows"},
     {"verify_layout", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(verify_layout)), METH_FASTCALL,
      "whether every parameter and gradient of a recorded layout is still where it was"},
     {"dict_versions", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(dict_versions)), METH_FASTCALL,
@@ -444,6 +531,9 @@ PyMODINIT_FUNC PyInit__rt_gather(void) {
     k_ema_squared = PyUnicode_InternFromString("ema_squared");
     k_step = PyUnicode_InternFromString("step");
     if (!k_ema || !k_ema_squared || !k_step) return nullptr;
+    h_ema = PyObject_Hash(k_ema);
+    h_ema_squared = PyObject_Hash(k_ema_squared);
+    h_step = PyObject_Hash(k_step);
     PyObject* m = PyModule_Create(&moddef);
     if (!m) return nullptr;
     PyModule_AddIntConstant(m, "DESC_SIZE", (long)sizeof(rt_tensor_desc));

@@ -48,17 +48,13 @@ def make_scalars(lr: float, betas: Tuple[float, float], eps: float, weight_decay
     bias_correction = 1 - beta1 ** step
     bias_correction_sqrt = (1 - beta2 ** step) ** (1 / 2)
     step_size = lr / bias_correction
-    f32 = np.float32
     # `tensor / python_float` on the GPU multiplies by the reciprocal of the scalar, taken in
     # double precision and then rounded to float32
-    inv_bcs = f32(1.0 / bias_correction_sqrt)
+    inv_bcs = 1.0 / bias_correction_sqrt
     apply_decay = weight_decay != 0
-    return N.RtScalars(
-        beta1=f32(beta1), one_m_beta1=f32(1 - beta1), beta2=f32(beta2), one_m_beta2=f32(1 - beta2),
-        inv_bcs=inv_bcs, eps=f32(eps),
-        decay=f32(1 - step_size * weight_decay) if apply_decay else f32(1.0),
-        neg_step_size=f32(-step_size), inv_loss_scale=f32(inv_loss_scale), centralization=f32(centralization),
-        apply_decay=int(apply_decay), reserved=0)
+    # (the float fields of the struct round each double to float32)
+    return N.RtScalars(beta1, 1 - beta1, beta2, 1 - beta2, inv_bcs, eps, 1 - step_size * weight_decay if apply_decay else 1.0,
+                       -step_size, inv_loss_scale, centralization, int(apply_decay), 0)
 
 
 @dataclass
@@ -180,11 +176,16 @@ def launch_resident(handle: N.Handle, descs: np.ndarray, scalars: Sequence[N.RtS
         return
     descs = np.ascontiguousarray(descs)
     if stream is None:
-        stream = torch.cuda.current_stream(handle.device).cuda_stream
-    handle.step_multi(_descs_ptr(descs), len(descs), scalars_array(scalars), len(scalars), seed & (2 ** 64 - 1),
-                      N.RT_NOISE_EXPLICIT if explicit_noise else N.RT_NOISE_PHILOX,
-                      None if clip_coef is None else clip_coef.data_ptr(),
-                      None if skip is None else skip.data_ptr(), stream)
+        stream = raw_stream(handle.device)
+    handle.step_multi_at(descs.ctypes.data, len(descs), scalars_array(scalars), len(scalars), seed & (2 ** 64 - 1),
+                         N.RT_NOISE_EXPLICIT if explicit_noise else N.RT_NOISE_PHILOX,
+                         None if clip_coef is None else clip_coef.data_ptr(),
+                         None if skip is None else skip.data_ptr(), stream)
+
+
+def raw_stream(device: int) -> int:
+    """torch's current stream on a device as a ``hipStream_t`` value."""
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 def step_resident(handle: N.Handle, entries: Sequence[Entry], scalars: Sequence[N.RtScalars], *, seed: int,
@@ -243,6 +244,16 @@ def grad_norm(handle: N.Handle, grads: Sequence[torch.Tensor], *, inv_loss_scale
     return out
 
 
+def grad_norm_rows(handle: N.Handle, descs: np.ndarray, *, inv_loss_scale: float = 1.0,
+                   max_norm: float = 1.0) -> torch.Tensor:
+    """``grad_norm`` over the gradients of an ``rt_tensor_desc`` array (all on the GPU)."""
+    descs = np.ascontiguousarray(descs)
+    out = torch.zeros(4, dtype=torch.float32, device=f"cuda:{handle.device}")
+    handle.grad_norm_at(descs.ctypes.data, len(descs), float(inv_loss_scale), float(max_norm), out.data_ptr(),
+                        raw_stream(handle.device))
+    return out
+
+
 def row_means(handle: N.Handle, g: torch.Tensor, rows: int, row_len: int, inv_loss_scale: float = 1.0,
               stream: Optional[int] = None) -> torch.Tensor:
     out = torch.empty(max(rows, 1), dtype=torch.float32, device=g.device)
@@ -253,10 +264,34 @@ def row_means(handle: N.Handle, g: torch.Tensor, rows: int, row_len: int, inv_lo
     return out
 
 
-def row_means_multi(handle: N.Handle, jobs: Sequence[Tuple[Entry, int, int]], inv_loss_scale: float = 1.0,
-                    stream: Optional[int] = None) -> None:
+class GatheredMeans:
+    """Rows 0 .. ``rows`` of the descriptor buffer ``buf`` (at ``addr``) whose gradients are to be centralized.  In the
+    segments, (first row, rows, means needed), ``row_mean`` holds each tensor's place among the means
+    (``place_row_means`` of the gatherer turns places into addresses); elsewhere it is 0, no means needed."""
+
+    def __init__(self, buf, addr, rows, segments, place):
+        self.buf, self.addr, self.rows, self.segments, self.place, self.means = buf, addr, rows, segments, place, None
+
+    def __len__(self) -> int:
+        return int(np.count_nonzero(self.buf["row_mean"][:self.rows]))
+
+    def allocate(self, device: int) -> None:
+        self.means = torch.empty(sum(m for _, _, m in self.segments), dtype=torch.float32, device=f"cuda:{device}")
+        at = self.means.data_ptr()
+        for first, n, m in self.segments:
+            self.place(self.addr + first * self.buf.itemsize, n, at)
+            at += 4 * m
+
+
+def row_means_multi(handle: N.Handle, jobs, inv_loss_scale: float = 1.0, stream: Optional[int] = None) -> None:
     """Row means of the GPU gradients of many entries in one launch.  ``jobs`` holds
-    (entry, rows, row_len); every entry gets ``row_mean`` (a view into one fp32 buffer) and ``row_len``."""
+    (entry, rows, row_len); every entry gets ``row_mean`` (a view into one fp32 buffer) and ``row_len``.
+    Or ``jobs`` is a ``GatheredMeans``, whose descriptors get the same."""
+    if isinstance(jobs, GatheredMeans):
+        jobs.allocate(handle.device)
+        handle.row_means_multi_at(jobs.addr, jobs.rows, float(inv_loss_scale),
+                                  raw_stream(handle.device) if stream is None else stream)
+        return
     jobs = [j for j in jobs if j[1] > 0 and j[2] > 0]
     if not jobs:
         return

@@ -21,6 +21,7 @@ from .. import _native as N
 from .. import functional as F
 
 _handles: Dict[int, N.Handle] = {}
+_FREEZE_MIN_TENSORS = 256   # shorter parameter lists are walked faster than a recorded layout is set up
 
 
 def _handle(device_index: int) -> N.Handle:
@@ -174,7 +175,7 @@ class AdamW(Optimizer):
         self.max_inflight_bytes = 2 << 30  # gradients kept alive for updates still in flight (step_param)
         self.max_inflight_calls = 2       # staging chunks handed to the copy pipeline and not finished yet
         self._poll_seconds = 0.0002       # completion is read from host memory; no runtime call while waiting
-        self.gather_min_tensors = 256     # from this many parameters on, step() gathers descriptors in C++
+        self.gather_min_tensors = 1       # from this many parameters on, step() gathers descriptors in C++
         self._gather_bufs = {}            # device -> descriptor rows the gatherer fills
         self._gather_stat = None
         self._state_lists = {}
@@ -206,7 +207,7 @@ class AdamW(Optimizer):
                             max_grad_norm=None, noise_source="philox", fuse_in_backward=True, host_arrays_ordered=False,
                             fuse_row_means=True,
                             max_inflight_bytes=2 << 30, max_inflight_calls=2, _poll_seconds=0.0002,
-                            gather_min_tensors=256, state_placement="auto", state_pool_min_bytes=1 << 30,
+                            gather_min_tensors=1, state_placement="auto", state_pool_min_bytes=1 << 30,
                             assume_static_layout=False)
 
     def __getstate__(self):
@@ -307,8 +308,14 @@ class AdamW(Optimizer):
             event.synchronize()
             if int(host.view(torch.int32)[2]) != 0:
                 skipped = True
-                for state, old in reversed(journal):
-                    state["step"] = old
+                for entry in reversed(journal):
+                    if len(entry) == 2:
+                        entry[0]["step"] = entry[1]
+                        continue
+                    states, status, written, which, first, steps = entry   # see _step_impl
+                    done = range(len(states)) if status is None else np.flatnonzero(status == written)
+                    for row, k in enumerate(done):
+                        states[int(k)]["step"] = (steps[0] if which is None else steps[int(which[row]) - first]) - 1
         self.last_step_skipped = skipped
         return skipped
 
@@ -479,7 +486,8 @@ class AdamW(Optimizer):
         if noise is None and getattr(self, "noise_source", "philox") == "reference":
             noise = self._reference_noise(grads, self._stepped_early)
         # Every step count this call advances is noted, so that they can be put back:
-        # (state, old value) from the Python loop, (states, status bytes) from the C++ gatherer.
+        # (state, old value) from the Python loop, (states, status bytes or None for all, code of the
+        # written ones) from the C++ gatherer.
         journal: list = []
         launched = [False]
         try:
@@ -492,7 +500,7 @@ class AdamW(Optimizer):
                         entry[0]["step"] = entry[1]
                     else:
                         states, status, written = entry
-                        for k in np.flatnonzero(status == written):
+                        for k in range(len(states)) if status is None else np.flatnonzero(status == written):
                             states[int(k)]["step"] -= 1
             raise
         self._stepped_early.clear()
@@ -512,13 +520,13 @@ class AdamW(Optimizer):
         extras = noise is not None or debug_out is not None
         dt_code = F._DT_CODE
 
-        # Large groups of plain GPU tensors are walked in C++ when the helper is built; it writes
+        # Groups of plain GPU tensors are walked in C++ when the helper is built; it writes
         # their descriptor rows and advances their step counts, and leaves the rest to the loop below.
         gather = None
-        if (grads is None and not extras and not early and self.max_grad_norm is None
-                and sum(len(g["params"]) for g in self.param_groups) >= self.gather_min_tensors):
+        if not extras and not early and sum(len(g["params"]) for g in self.param_groups) >= self.gather_min_tensors:
             gather = G.module()
-        gathered: Dict[int, list] = {}    # dev -> [descriptor buffer, rows used]
+        gathered: Dict[int, list] = {}    # dev -> [descriptor buffer, its address, rows used]
+        gathered_means: Dict[int, list] = {}   # dev -> [(first row, rows, row means they need)] of centralized groups
         cen_jobs: Dict[int, list] = {}    # dev -> [(entry, rows, row_len)] of gradients to centralize
         counted: Dict[int, list] = {}     # dev -> [(state, step count before)] of the tensors under max_grad_norm
         skip_checks = []
@@ -530,26 +538,34 @@ class AdamW(Optimizer):
             last_step, last_si = None, -1
             plist = group["params"]
             work = enumerate(plist)
-            if gather is not None and cen == 0 and row and row[0].plain and isinstance(plist, list):
+            if gather is not None and row and row[0].plain and isinstance(plist, list):
                 dev = row[0].dev
                 slot = gathered.get(dev)
                 if slot is None:
-                    slot = gathered[dev] = [self._gather_buffer(dev), 0]
-                buf, used = slot
-                status = self._gather_status(len(plist))
-                status[:len(plist)] = gather.PYTHON  # nothing written yet, should the call itself fail
+                    slot = gathered[dev] = [*self._gather_buffer(dev), 0]
+                buf, addr, used = slot
+                n = len(plist)
+                status, status_addr = self._gather_status(n)
                 states = self._state_list(gi)
-                journal.append((states, status[:len(plist)], gather.WRITTEN))
-                n_rows, new_steps = gather.gather_group(
-                    plist, states, dev, buf.ctypes.data + used * buf.itemsize, len(buf) - used,
-                    status.ctypes.data, len(scalars), row[0].tensor_id)
-                journal[-1] = (states, status[:len(plist)].copy(), gather.WRITTEN)
-                slot[1] = used + n_rows
+                how = 0 if cen == 0 else 2 if self.__dict__.get("fuse_row_means", True) else 1
+                n_rows, new_steps, left, means = gather.gather_group(
+                    plist, states, dev, addr + used * buf.itemsize, len(buf) - used, status_addr, len(scalars),
+                    row[0].tensor_id, None if grads is None else [grads.get(p, p.grad) for p in plist], how)
+                done = None if n_rows == n else status[:n].copy()
+                journal.append((states, done, gather.WRITTEN))
+                if self.max_grad_norm is not None:
+                    which = None if len(new_steps) == 1 else buf["scalars_idx"][used:used + n_rows].copy()
+                    counted.setdefault(dev, []).append((states, done, gather.WRITTEN, which, len(scalars), new_steps))
+                if means:
+                    gathered_means.setdefault(dev, []).append((used, n_rows, means))
+                slot[2] = used + n_rows
                 for st in new_steps:
                     scalar_key[(gi, st, lr, beta1, beta2, eps, wd, cen)] = len(scalars)
                     scalars.append(F.make_scalars(lr, (beta1, beta2), eps, wd, st, centralization=cen,
                                                   inv_loss_scale=inv_loss_scale))
-                rest = np.flatnonzero(status[:len(plist)] == gather.PYTHON)
+                if not left:
+                    continue
+                rest = np.flatnonzero(done == gather.PYTHON)
                 work = ((int(k), plist[int(k)]) for k in rest)
             for k, p in work:
                 grad = grads.get(p, p.grad) if grads is not None else p.grad
@@ -644,6 +660,13 @@ class AdamW(Optimizer):
                 on_gpu = e.p.is_cuda and e.g.is_cuda and e.m.is_cuda and e.v.is_cuda
                 (resident if on_gpu else streamed).setdefault(dev, []).append(e)
 
+        mean_bufs = []   # kept until the launches that read them are enqueued
+        for dev, segments in gathered_means.items():
+            buf, addr, rows = gathered[dev]
+            with torch.cuda.device(dev):
+                jobs = F.GatheredMeans(buf, addr, rows, segments, gather.place_row_means)
+                mean_bufs.append(jobs)
+                F.row_means_multi(_handle(dev), jobs, inv_loss_scale)
         for dev, jobs in cen_jobs.items():
             with torch.cuda.device(dev):
                 F.row_means_multi(_handle(dev), jobs, inv_loss_scale)   # writes fresh buffers only
@@ -655,8 +678,8 @@ class AdamW(Optimizer):
             res, stm = resident.get(dev, []), streamed.get(dev, [])
             lane = plain.get(dev)
             descs = self._plain_descs(dev, lane) if lane is not None else None
-            if dev in gathered and gathered[dev][1]:
-                d0 = gathered[dev][0][:gathered[dev][1]]
+            if dev in gathered and gathered[dev][2]:
+                d0 = gathered[dev][0][:gathered[dev][2]]
                 descs = d0 if descs is None else np.concatenate([d0, descs])
             if res:
                 d2 = F.pack_descs(res, streamed=False)
@@ -669,9 +692,13 @@ class AdamW(Optimizer):
             with torch.cuda.device(dev):
                 clip = skip = None
                 if self.max_grad_norm is not None:
-                    # one norm over every gradient of the step, wherever its parameter lives
-                    gl = (lane[1] if lane is not None else []) + [e.g for e in res] + [e.g for e in stm]
-                    out = F.grad_norm(h, gl, inv_loss_scale=inv_loss_scale, max_norm=self.max_grad_norm)
+                    # one norm over every gradient of the step, wherever its parameter lives (all of them are
+                    # on the GPU by now)
+                    rows = descs
+                    if stm:
+                        rows = stm_descs.copy() if descs is None else np.concatenate([descs, stm_descs])
+                        rows["host_mask"] = 0
+                    out = F.grad_norm_rows(h, rows, inv_loss_scale=inv_loss_scale, max_norm=self.max_grad_norm)
                     self.last_grad_norm = out
                     clip, skip = out[1:2], out[2:3]
                     # the record goes to pinned host memory behind the norm pass; the next step reads it there
@@ -693,7 +720,7 @@ class AdamW(Optimizer):
         if skip_checks:
             self._skip_check = skip_checks
         if self._freeze_requested:
-            self._record_layout(gathered, plain, resident, streamed, scalar_key, explicit)
+            self._record_layout(gathered, plain, resident, streamed, scalar_key, explicit or grads is not None)
 
     # -- a recorded layout: steps that only check that nothing moved ----------------------------------
     def freeze_layout(self) -> None:
@@ -704,8 +731,8 @@ class AdamW(Optimizer):
         sets of thousands of small tensors whose gradients keep their storage from step to step
         (``zero_grad(set_to_none=False)`` or gradients accumulated in place).
 
-        Applies to steps that the C++ gatherer covers completely: one GPU, at least
-        ``gather_min_tensors`` parameters, every stepping tensor plain (contiguous, on the GPU), no
+        Applies to steps that the C++ gatherer covers completely: one GPU, at least 256
+        parameters, every stepping tensor plain (contiguous, on the GPU), no
         ``centralization`` / ``max_grad_norm`` / ``noise_source="reference"`` / ``step_param``.
         Otherwise nothing is recorded and steps run as usual.
 
@@ -748,9 +775,11 @@ class AdamW(Optimizer):
     def _record_layout(self, gathered, plain, resident, streamed, scalar_key, explicit) -> None:
         self._frozen = None
         if (explicit or plain or resident or streamed or len(gathered) != 1 or self.max_grad_norm is not None
+                or any(g["centralization"] != 0 for g in self.param_groups)
+                or sum(len(g["params"]) for g in self.param_groups) < _FREEZE_MIN_TENSORS
                 or G.module() is None or not hasattr(G.module(), "verify_layout")):
             return
-        (dev, (buf, rows)), = gathered.items()
+        (dev, (buf, _, rows)), = gathered.items()
         if rows == 0:
             return
         descs = buf[:rows].copy()
@@ -1066,19 +1095,21 @@ class AdamW(Optimizer):
                 _handle(dev).streamed_wait()
         self._inflight = []
 
-    def _gather_buffer(self, dev: int) -> np.ndarray:
-        """Descriptor rows the C++ gatherer fills for one device (one row per parameter at most)."""
+    def _gather_buffer(self, dev: int) -> tuple:
+        """Descriptor rows the C++ gatherer fills for one device (one row per parameter at most), and their address."""
         n = sum(len(g["params"]) for g in self.param_groups)
-        buf = self._gather_bufs.get(dev)
-        if buf is None or len(buf) < n:
-            buf = self._gather_bufs[dev] = np.zeros(n, F.DESC_DTYPE)
-        return buf
+        slot = self._gather_bufs.get(dev)
+        if slot is None or len(slot[0]) < n:
+            buf = np.zeros(n, F.DESC_DTYPE)
+            slot = self._gather_bufs[dev] = (buf, buf.ctypes.data)
+        return slot
 
-    def _gather_status(self, n: int) -> np.ndarray:
-        st = self._gather_stat
-        if st is None or len(st) < n:
-            st = self._gather_stat = np.zeros(n, np.uint8)
-        return st
+    def _gather_status(self, n: int) -> tuple:
+        slot = self._gather_stat
+        if slot is None or len(slot[0]) < n:
+            st = np.zeros(n, np.uint8)
+            slot = self._gather_stat = (st, st.ctypes.data)
+        return slot
 
     def _state_list(self, gi: int) -> list:
         """The state dicts of group ``gi`` in parameter order (cached with the records)."""

@@ -604,6 +604,53 @@ def test_gathered_step_equals_the_python_loop():
     assert max(oa.state[p]["step"] for p in a) == 3 and min(oa.state[p]["step"] for p in a) >= 2
 
 
+@pytest.mark.parametrize("option", ["clip", "central", "central_apart", "given_f32", "clip_central_given"])
+def test_gathered_step_equals_the_python_loop_with_every_option(option):
+    """The C++ gatherer under a clip, with centralization (row means inside the update and before it) and with
+    gradients that are given, against the Python loop: the same bits and step counts, also with a parameter
+    that only the loop can take, parameters without gradients, two step counts in a group, and a step that a
+    non-finite norm cancels."""
+    from ramtorch_amd import _gather as G
+    if G.module() is None:
+        pytest.skip("gather helper not built")
+    shapes = [(33, 24), (9000,), (4, 512), (16, 3, 3, 3), (5,), (2, 4104), (40, 700), (3, 7), (1,), (64, 64)]
+    kw = dict(storage_device="cuda", seed=31, loss_scale=4.0 if "given" in option else 1.0,
+              max_grad_norm=0.02 if "clip" in option else None, centralization=0.5 if "central" in option else 0.0)
+
+    def make():
+        ps, _ = _make_params(shapes, 9000)
+        ps[6] = torch.nn.Parameter(torch.stack([ps[6].detach()] * 2, 2)[..., 0], requires_grad=False)  # not contiguous
+        opt = ramtorch_amd.AdamW([{"params": ps[:4]}, {"params": ps[4:], "lr": 3e-4, "centralization": 0.0}], **kw, **{k: v for k, v in HP0.items() if k != "lr"})
+        opt.fuse_row_means = option != "central_apart"
+        return ps, opt
+
+    (a, oa), (b, ob) = make(), make()
+    ob.gather_min_tensors = 10 ** 9
+    for step in range(1, 6):
+        given = []
+        for ps in (a, b):
+            own = {}
+            for i, p in enumerate(ps):
+                g = dev16(oracle.synth_inputs(p.numel(), 9100 + 17 * step + i)[1]).view(p.shape)
+                if step == 4 and "clip" in option and i == 2:
+                    g = g * float("inf")
+                g = None if (i + step) % 7 == 0 else g
+                if "given" in option and i != 3:
+                    own[p] = None if g is None else g.float()
+                    g = torch.ones_like(p)            # must not be used
+                p.grad = g
+            given.append(own if "given" in option else None)
+        oa.step(grads=given[0])
+        ob.step(grads=given[1])
+        assert oa.step_was_skipped() == ob.step_was_skipped() == (step == 4 and "clip" in option)
+        for i, (p, q) in enumerate(zip(a, b)):
+            assert oa.state[p]["step"] == ob.state[q]["step"], (step, i)
+            for x, y in ((p.detach(), q.detach()), (oa.state[p]["ema"], ob.state[q]["ema"]),
+                         (oa.state[p]["ema_squared"], ob.state[q]["ema_squared"])):
+                assert nmis(x, y) == 0, (step, i)
+    assert len({oa.state[p]["step"] for p in a}) > 1
+
+
 def test_pooled_state_placement_changes_nothing_but_addresses():
     """state_placement="auto": ema and ema_squared are views into two pools (placed in different
     HBM regions when the probe finds such a placement).  Results, state_dict and resume are the

@@ -330,6 +330,45 @@ def test_gatherer_writes_the_rows_the_python_loop_would():
     assert rows3 == 0 and stat[0] == g.PYTHON
 
 
+def test_gatherer_takes_given_gradients_and_places_row_means():
+    from ramtorch_amd import _gather as G
+    g = G.module()
+    if g is None:
+        pytest.skip("gather helper not built")
+    shapes = [(5, 16), (4, 512), (3, 513), (600,), (), (2, 3, 256), (2, 32776), (0, 8), (7, 4)]
+    bf = torch.bfloat16
+    ps = [torch.nn.Parameter(torch.zeros(s, dtype=bf)) for s in shapes]
+    sts = [{"step": 8 + i % 2, "ema": torch.zeros_like(p), "ema_squared": torch.zeros_like(p)} for i, p in enumerate(ps)]
+    grads = [torch.ones(s) for s in shapes]          # fp32, which torch would not store in .grad
+    grads[1] = grads[1].to(bf)
+    grads[5] = grads[5].to(bf)
+    ps[8].grad = torch.zeros(7, 4, dtype=bf)
+    grads[8] = None                                  # given as None: no gradient, whatever .grad holds
+    n = len(ps)
+    buf, stat = np.zeros(n, F.DESC_DTYPE), np.zeros(n, np.uint8)
+    for how in (0, 1, 2):
+        steps_before = [s["step"] for s in sts]
+        rows, steps, left, means = g.gather_group(ps, sts, -1, buf.ctypes.data, n, stat.ctypes.data, 0, 0, grads, how)
+        assert rows == n - 1 and left == 0 and list(stat) == [g.WRITTEN] * (n - 1) + [g.NO_GRAD]
+        assert [s["step"] for s in sts] == [k + 1 for k in steps_before[:-1]] + steps_before[-1:]
+        assert [int(d["g"]) for d in buf[:rows]] == [x.data_ptr() for x in grads[:-1]]
+        assert [int(d["step"]) for d in buf[:rows]] == [s["step"] for s in sts[:-1]]
+        assert [steps[d["scalars_idx"]] for d in buf[:rows]] == [s["step"] for s in sts[:-1]]
+        g.place_row_means(buf.ctypes.data, rows, 1 << 20)
+        at = 1 << 20
+        for d, shape, grad in zip(buf, shapes, grads[:-1]):
+            count = shape[0] if len(shape) >= 2 else 1
+            row = grad.numel() // count if count else 0
+            fused = how == 2 and grad.dtype == bf and row % 8 == 0 and F.ROWWISE_MIN_LEN <= row <= F.ROWWISE_MAX_LEN
+            if how == 0 or not grad.numel():
+                assert d["row_len"] == 0 and d["row_mean"] == 0
+                continue
+            assert d["row_len"] == row and d["row_mean"] == (0 if fused else at), (how, shape)
+            at += 0 if fused else 4 * count
+        assert at == (1 << 20) + 4 * means
+    assert fused is False and sum(int(d["row_mean"] == 0) for d in buf[:n - 1]) == 3   # two fused, one empty
+
+
 def test_state_layout_options_are_validated_and_harmless_on_cpu():
     ps = [torch.nn.Parameter(torch.zeros(16, dtype=torch.bfloat16))]
     with pytest.raises(ValueError, match="state_placement"):
