@@ -62,6 +62,12 @@ typedef u32x4 u32x4_any __attribute__((aligned(2)));
 __device__ __forceinline__ u32x4 ldg128(uint64_t addr) {
     return __builtin_nontemporal_load((const RT_GLOBAL u32x4_any*)addr);
 }
+// What the next kernel reads again -- gradients, in the passes before the update -- is loaded without the hint:
+// it then stays in the 256 MB memory-side cache (with the hint it does not).  Those passes walk the
+// gradients backwards, so that what the update reads first is what they read last.  A clipped step of 122 M fp32
+// elements (489 MB of gradients) takes 451 us with the hint in the norm pass and 417 us without; 218 M with
+// bf16 gradients 616 and 577 us, with fp32 gradients (872 MB) 917 and 886 us.  Walking backwards with the hint: no change.
+__device__ __forceinline__ u32x4 ldg128_keep(uint64_t addr) { return *(const RT_GLOBAL u32x4_any*)addr; }
 __device__ __forceinline__ void stg128(uint64_t addr, u32x4 v) {
     __builtin_nontemporal_store(v, (RT_GLOBAL u32x4_any*)addr);
 }
@@ -1334,7 +1340,7 @@ __device__ __forceinline__ float chunk_sumsq_full(uint64_t g_addr, uint32_t chun
     const uint64_t base = g_addr + (uint64_t)chunk * kChunkElems * esize<GDT>() + (uint64_t)threadIdx.x * 16;
     u32x4 r[kLoads];
 #pragma unroll
-    for (int k = 0; k < kLoads; ++k) r[k] = ldg128(base + (uint64_t)k * (kThreads * 16));
+    for (int k = 0; k < kLoads; ++k) r[k] = ldg128_keep(base + (uint64_t)k * (kThreads * 16));
     float acc = 0.0f;
 #pragma unroll
     for (int k = 0; k < kLoads; ++k) {
@@ -1426,7 +1432,9 @@ __global__ __launch_bounds__(kThreads) void grad_sumsq_table_kernel(const NormEn
                                                                     double* __restrict__ partials) {
     __shared__ float lds[kThreads / 64];
     double total = 0.0;
-    for (uint32_t c = blockIdx.x; c < n_chunks; c += gridDim.x) {
+    // backwards, see ldg128_keep
+    for (uint32_t left = (n_chunks - blockIdx.x + gridDim.x - 1u) / gridDim.x; left-- > 0u;) {
+        const uint32_t c = blockIdx.x + left * gridDim.x;
         const bool whole = c < total_whole;
         const uint32_t key = whole ? c : c - total_whole;
         uint32_t lo = 0, hi = n;  // last entry whose first chunk number in this sequence is <= key
@@ -1504,18 +1512,18 @@ __device__ __forceinline__ float load_elem(uint64_t base, uint64_t idx) {
 // Sum of row [base, base + row_len) of g by the calling wavefront; the result is in every lane.
 // A row moves as whole vectors, 32 registers of them in flight per lane, and at most 7 single
 // elements at its end.
-// KEEP: the row is read again right away (by the update that takes its own row means), so its
-// lines are loaded the ordinary way and stay in the L2; the values and their order are the same.
+// The row is read again, by the update behind this pass or right away by the update that takes its own row
+// means: its lines are loaded the ordinary way and stay in the caches.
 template <int DT>
 __device__ __forceinline__ Raw8<DT> load_raw_cached(uint64_t base, uint64_t i) {
     Raw8<DT> r;
     const uint64_t addr = base + i * esize<DT>();
-    r.a = *(const RT_GLOBAL u32x4_any*)addr;
-    if constexpr (DT == RT_DT_F32) r.b = *(const RT_GLOBAL u32x4_any*)(addr + 16);
+    r.a = ldg128_keep(addr);
+    if constexpr (DT == RT_DT_F32) r.b = ldg128_keep(addr + 16);
     return r;
 }
 
-template <int GDT, bool KEEP = false>
+template <int GDT>
 __device__ __forceinline__ float row_sum_wave(uint64_t g, uint64_t base, uint32_t row_len, float inv_loss_scale) {
     constexpr int kB = GDT == RT_DT_F32 ? kRowVecs / 2 : kRowVecs;   // an fp32 vector of 8 elements is two loads
     const uint32_t lane = threadIdx.x & 63u;
@@ -1526,8 +1534,7 @@ __device__ __forceinline__ float row_sum_wave(uint64_t g, uint64_t base, uint32_
 #pragma unroll
         for (int k = 0; k < kB; ++k) {
             const uint32_t v = v0 + (uint32_t)k * 64u + lane;
-            if (v < n_vec)
-                r[k] = KEEP ? load_raw_cached<GDT>(g, base + (uint64_t)v * kVec) : load_raw<GDT>(g, base + (uint64_t)v * kVec);
+            if (v < n_vec) r[k] = load_raw_cached<GDT>(g, base + (uint64_t)v * kVec);
         }
 #pragma unroll
         for (int k = 0; k < kB; ++k) {
@@ -1552,8 +1559,8 @@ __device__ __forceinline__ float row_sum_block(uint64_t g, uint64_t base, uint64
         for (int k = 0; k < kInFlight; ++k) {
             const uint64_t e = c0 + ((uint64_t)k * kThreads + threadIdx.x) * kVec;
             if (e < row_len)
-                r[k] = (e + kVec <= row_len) ? load_raw<GDT>(g, base + e)
-                                                        : load_raw_guarded<GDT>(g, base + e, base + row_len);
+                r[k] = (e + kVec <= row_len) ? load_raw_cached<GDT>(g, base + e)
+                                             : load_raw_guarded<GDT>(g, base + e, base + row_len);
         }
 #pragma unroll
         for (int k = 0; k < kInFlight; ++k) {
@@ -1607,15 +1614,16 @@ struct alignas(16) RowMeanEntry {
 };
 static_assert(sizeof(RowMeanEntry) == 48, "RowMeanEntry layout");
 
-// Workgroup b takes rows 4b .. 4b+3, one per wave.  (A fixed number of workgroups whose waves walk rows
+// Workgroup b takes the four rows that end 4b rows before the last, one per wave.  (A fixed number of workgroups whose waves walk rows
 // a launch-width apart, looking their gradient up only when it changes, measured 8 % slower: a wave
 // then has nothing in flight while it reduces a row.)
 __global__ __launch_bounds__(kThreads) void row_mean_table_kernel(const uint32_t* __restrict__ first,
                                                                   const RowMeanEntry* __restrict__ table, uint32_t n,
                                                                   uint32_t rows_total, float inv_loss_scale) {
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const uint32_t row = blockIdx.x * (kThreads / 64) + wave;
+    uint32_t row = blockIdx.x * (kThreads / 64) + wave;
     if (row >= rows_total) return;
+    row = rows_total - 1u - row;   // backwards, see ldg128_keep (61 M fp32 gradients: 315 -> 294 us a step, 218 M: 1020 -> 999 us)
     const uint32_t idx = find_range(first, n, row);   // each wave searches on its own
     const RowMeanEntry e = load_const(&table[idx]);
     const uint64_t r = row - e.first_row;
@@ -1627,7 +1635,7 @@ __global__ __launch_bounds__(kThreads) void row_mean_table_long_kernel(const uin
                                                                        const RowMeanEntry* __restrict__ table, uint32_t n,
                                                                        float inv_loss_scale) {
     __shared__ float lds[kThreads / 64];
-    const uint32_t row = blockIdx.x;
+    const uint32_t row = gridDim.x - 1u - blockIdx.x;   // backwards as well
     const uint32_t idx = find_range(first, n, row);
     const RowMeanEntry e = load_const(&table[idx]);
     const uint64_t r = row - e.first_row;
@@ -1736,7 +1744,7 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_rowwise_kernel(const Launch
     }
     // (sixteen vectors per lane on the way at once instead of eight -- a lane adds its vectors in ascending
     // order whatever the batch, so no bit changes -- measured the same time on the 8B set)
-    const float sum = row_sum_wave<GDT, true>(tg, e0, row_len, c.s.inv_loss_scale);
+    const float sum = row_sum_wave<GDT>(tg, e0, row_len, c.s.inv_loss_scale);
     const float mc = cen_term(sum / (float)row_len, c.s, c.do_clip, c.coef);
 
     struct In {
