@@ -264,9 +264,9 @@ using MultiKernel = void (*)(const LaunchArgs);
 struct KernelPair {
     MultiKernel fast;     // whole fast units, plus (Philox) pieces
     MultiKernel generic;  // debug outputs, leftovers of explicit-noise tensors, rows shorter than 8
-    MultiKernel fast_cen; // the same with centralization (16-bit layouts, Philox), or NULL
-    MultiKernel link, link_cen;  // fast and fast_cen for arrays in host memory (Philox), or NULL
-    MultiKernel rowwise;  // whole tensors with centralization whose row means the kernel takes itself (same layouts), or NULL
+    MultiKernel fast_cen; // the same with centralization (Philox), or NULL
+    MultiKernel link, link_cen;  // fast and (16-bit layouts) fast_cen for arrays in host memory (Philox), or NULL
+    MultiKernel rowwise;  // whole tensors with centralization whose row means the kernel takes itself (16-bit layouts, Philox), or NULL
     MultiKernel rowwise_short;  // the same for rows of at most kRowwiseShortMax elements
 };
 
@@ -285,6 +285,7 @@ static KernelPair pick_noise(int noise) {
     k.link = sr_adamw_link_kernel<P, G, M, V, false>;
     if constexpr (wide) {
         k.fast = sr_adamw_fast_wide_kernel<P, G, M, V, RT_NOISE_PHILOX>;
+        k.fast_cen = sr_adamw_fast_wide_kernel<P, G, M, V, RT_NOISE_PHILOX, true>;
     } else {
         k.fast = sr_adamw_fast_kernel<P, G, M, V, RT_NOISE_PHILOX>;
         k.fast_cen = sr_adamw_fast_kernel<P, G, M, V, RT_NOISE_PHILOX, true>;
@@ -410,8 +411,9 @@ static int validate(const rt_tensor_desc* descs, uint32_t n, const rt_scalars* s
 // pieces (Philox noise; with explicit noise chunks of the generic kernel); tensors whose row means the
 // update takes itself go to the row-wise kernel; everything else goes to the generic kernel chunk by chunk.
 // One pass classifies the tensors, one writes the records where they belong.
+// over_link: for the kernels that work on host memory, which have no centralizing instance for fp32 layouts.
 static void build_image(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, const rt_scalars* scalars,
-                        bool want_explicit, Plan& plan, std::vector<uint8_t>& image) {
+                        bool want_explicit, Plan& plan, std::vector<uint8_t>& image, bool over_link = false) {
     enum Kind : uint8_t { kUnits, kPieces, kCenUnits, kCenPieces, kRowLong, kRowShort, kGeneric, kKinds };
     constexpr uint64_t unit = kFastUnitElems;
     static_assert(kFastUnitElems == kChunkElems, "what a tensor's units leave over is its last chunk");
@@ -438,7 +440,7 @@ static void build_image(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, c
     auto it = set_index.end();
     for (size_t k0 = 0; k0 < count;) {
         const uint32_t combo = combo_of(descs[order[k0]]);
-        const bool templated = combo != kComboAny, cen_kernel = narrow_combo(combo) && !want_explicit;
+        const bool templated = combo != kComboAny, cen_kernel = (over_link ? narrow_combo(combo) : templated) && !want_explicit;
         uint32_t in_kind[kKinds] = {};
         size_t k1 = k0;
         for (; k1 < count && combo_of(descs[order[k1]]) == combo; ++k1) {
@@ -1627,7 +1629,7 @@ static int streamed_enqueue_impl(rt_handle* h, const rt_tensor_desc* descs, uint
         double up = 0, down = 0;
         if (map_host_arrays(descs, n, mapped, up, down)) {
             Plan plan;
-            build_image(h, mapped.data(), n, scalars, /*want_explicit=*/false, plan, h->image);
+            build_image(h, mapped.data(), n, scalars, /*want_explicit=*/false, plan, h->image, /*over_link=*/true);
             uint64_t n_generic = 0;
             for (const Batch& b : plan.batches) n_generic += b.n_generic;
             if (n_generic <= kLinkChunksMax) {

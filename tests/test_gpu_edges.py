@@ -123,3 +123,33 @@ def test_scalar_sets_reach_the_kernels_as_arguments_or_through_the_table(handle)
         for k, (d, a) in enumerate(zip(dev, cpu)):
             for name, got, want in zip("pmv", (d[0], d[2], d[3]), (a[0], a[2], a[3])):
                 np.testing.assert_array_equal(bits(got), want.view(np.int16), err_msg=f"round {round_}, {n_sets} sets, tensor {k} {name}")
+
+
+@pytest.mark.parametrize("mix", ["bf16_f32grad_f32v", "f32_bf16states"])
+@pytest.mark.parametrize("rows,row_len", [(2049, 8), (1111, 9), (700, 27), (40, 250), (9, 2731), (3, 8193), (2, 40000)])
+def test_centralized_fp32_layouts_take_their_means_in_units(handle, mix, rows, row_len):
+    """The layouts with an fp32 array: four elements of a lane in two rows, rows shorter and longer than a half block
+    (256), a block (512) and a unit (8192), loss scale and clip on gradient and mean."""
+    codes = _MIX[mix]
+    n = rows * row_len
+    raw = oracle.synth_inputs(n, 700 + row_len)
+    arrays = [a if c == 0 else oracle.bf16_to_f32(a) for a, c in zip(raw, codes)]
+    (P, wp), (G, _), (M, wm), (V, wv) = (guarded(a, c, s) for a, c, s in zip(arrays, codes, (1, 0, 0, 3)))
+    means = F.row_means(handle, G, rows, row_len, 0.5)
+    e = F.Entry(p=P, g=G, m=M, v=V, step=4, scalars_idx=0, tensor_id=5, row_mean=means, row_len=row_len)
+    clip = torch.tensor([0.75], device="cuda")
+    F.step_resident(handle, [e], [F.make_scalars(step=4, centralization=0.75, inv_loss_scale=0.5, **HP0)], seed=3,
+                    explicit_noise=False, clip_coef=clip)
+    torch.cuda.synchronize()
+    # each product and the difference round as in the kernel
+    g32 = arrays[1] if codes[1] else oracle.bf16_to_f32(arrays[1])
+    g32 = (g32 * np.float32(0.5)) * np.float32(0.75)
+    term = (means.cpu().numpy() * np.float32(0.75)) * np.float32(0.75)
+    g32 = (g32.reshape(rows, row_len) - term[:, None]).astype(np.float32).ravel()
+    po, mo, vo = arrays[0].copy(), arrays[2].copy(), arrays[3].copy()
+    oracle.step_tensor(po, g32, mo, vo, oracle.scalars_from_hparams(step=4, **HP0), p_dtype=codes[0], g_dtype=oracle.DT_F32,
+                       m_dtype=codes[2], v_dtype=codes[3], seed=3, step=4, tensor_id=5)
+    for got, want in ((P, po), (M, mo), (V, vo)):
+        np.testing.assert_array_equal(bits(got), want.view({2: np.int16, 4: np.int32}[want.dtype.itemsize]))
+    for whole, s in ((wp, 1), (wm, 0), (wv, 3)):
+        check_guards(whole, s, n)
