@@ -393,19 +393,20 @@ __device__ __forceinline__ void make_ctx(const LaunchArgs& a, uint32_t set_idx, 
 // counts the lanes whose entry is <= unit.  One dependent load for up to 64 tensors, two for up
 // to 4096 -- a scalar binary search would chain one load per halving in front of every
 // workgroup's first vector load.  (Loading up to eight entries per lane at once, one latency for up
-// to 512 tensors, measured no faster on the 8B set's 226 ranges.)
+// to 512 tensors, measured no faster on the 8B set's 226 ranges.)  Entries lie kStep words apart.
+template <uint32_t kStep = 1>
 __device__ __forceinline__ uint32_t find_range(const uint32_t* __restrict__ first, uint32_t n, uint32_t unit) {
     const uint32_t lane = threadIdx.x & 63u;
     uint32_t lo = 0, len = n;
     while (len > 64u) {
         const uint32_t stride = (len + 63u) >> 6;
         const uint32_t k = lane * stride;
-        const bool le = k < len && first[lo + k] <= unit;
+        const bool le = k < len && first[(size_t)(lo + k) * kStep] <= unit;
         const uint32_t c = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(le));  // >= 1: first[lo] <= unit
         lo += (c - 1u) * stride;
         len = min(stride, len - (c - 1u) * stride);
     }
-    const bool le = lane < len && first[lo + lane] <= unit;
+    const bool le = lane < len && first[(size_t)(lo + lane) * kStep] <= unit;
     return lo + (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(le)) - 1u;
 }
 
@@ -1436,9 +1437,12 @@ __device__ __forceinline__ float chunk_sumsq_dt(int dt, uint64_t g_addr, uint64_
 // b, b + gridDim.x, ... and writes one partial sum of squares.  The only table
 // is one NormEntry per gradient (small enough to live in a fixed device array
 // for the entry point that allocates nothing); a chunk finds its gradient by
-// binary search.  Chunks are numbered in two sequences -- first every whole
-// chunk of the gradients, then the partial ones, each in tensor
+// the 64-way search of the update kernels, each wavefront on its own.  Chunks
+// are numbered in two sequences -- first every whole chunk of the gradients, then the partial ones, each in tensor
 // order -- so that most workgroups see nothing but whole chunks.
+// A lane keeps its sum in fp64 from chunk to chunk and the workgroup reduces once, at the end, so that the
+// four waves never wait for each other between chunks.  17.7 M fp32 elements in 160 ragged gradients
+// 16.6 -> 15.2 us, 218 M in nine 144.6 -> 141.7 us, against a binary search and a reduction with two barriers per chunk.
 // ---------------------------------------------------------------------------
 struct alignas(16) NormEntry {
     uint64_t g;
@@ -1466,26 +1470,26 @@ __global__ __launch_bounds__(kThreads) void grad_sumsq_table_kernel(const NormEn
                                                                     uint32_t total_whole, uint32_t n_chunks,
                                                                     float inv_loss_scale,
                                                                     double* __restrict__ partials) {
-    __shared__ float lds[kThreads / 64];
+    constexpr uint32_t kStep = sizeof(NormEntry) / 4;
     double total = 0.0;
     // backwards, see ldg128_keep
     for (uint32_t left = (n_chunks - blockIdx.x + gridDim.x - 1u) / gridDim.x; left-- > 0u;) {
         const uint32_t c = blockIdx.x + left * gridDim.x;
         const bool whole = c < total_whole;
         const uint32_t key = whole ? c : c - total_whole;
-        uint32_t lo = 0, hi = n;  // last entry whose first chunk number in this sequence is <= key
-        while (hi - lo > 1u) {
-            const uint32_t mid = (lo + hi) >> 1;
-            const uint32_t f = whole ? table[mid].first_whole : table[mid].first_rest;
-            if (f <= key) lo = mid; else hi = mid;
-        }
-        const NormEntry e = table[lo];
+        // the last entry whose first chunk number in this sequence is <= key is the one with chunks: entries
+        // without any share their number with the entry behind them
+        const uint32_t at = find_range<kStep>(whole ? &table->first_whole : &table->first_rest, n, key);
+        const NormEntry e = table[__builtin_amdgcn_readfirstlane(at)];
         const uint32_t chunk = whole ? key - e.first_whole : e.n_whole + (key - e.first_rest);
-        const float acc = chunk_sumsq_dt((int)e.dtype, e.g, e.numel, chunk, inv_loss_scale);
-        const float bs = block_sum(acc, lds);
-        total += (double)bs;  // meaningful in thread 0 only
+        total += (double)chunk_sumsq_dt((int)e.dtype, e.g, e.numel, chunk, inv_loss_scale);
     }
-    if (threadIdx.x == 0) partials[blockIdx.x] = total;
+    __shared__ double lds[kThreads / 64];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off, 64);
+    if ((threadIdx.x & 63u) == 0u) lds[threadIdx.x >> 6] = total;
+    __syncthreads();
+    if (threadIdx.x == 0) partials[blockIdx.x] = (lds[0] + lds[1]) + (lds[2] + lds[3]);
 }
 
 // Pass 2: one workgroup folds the partials in index order and derives the

@@ -153,3 +153,25 @@ def test_centralized_fp32_layouts_take_their_means_in_units(handle, mix, rows, r
         np.testing.assert_array_equal(bits(got), want.view({2: np.int16, 4: np.int32}[want.dtype.itemsize]))
     for whole, s in ((wp, 1), (wm, 0), (wv, 3)):
         check_guards(whole, s, n)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 129, 4097])
+def test_norm_pass_finds_every_gradient(handle, n):
+    """Tables of one, two and three search steps, with gradients that have no whole chunk of 8192 elements, no
+    remainder, neither (empty) or both, at either end too.  Each gradient's values lie in a range of its own, so
+    that a chunk looked up in the wrong gradient shows; fp32 sums of at most 32 squares a lane: 32 * 2^-24 at most."""
+    rng = np.random.default_rng(n)
+    sizes = [(8192, 5, 0, 8193, 8192 * 2, 1, 700)[k] for k in rng.integers(0, 7, n)]
+    total = sum(sizes)
+    flat = torch.randn(total, generator=torch.Generator().manual_seed(n))
+    scale = torch.from_numpy(np.repeat(10.0 ** rng.uniform(-3, 0, n), sizes)).float()
+    flat = (flat * scale).cuda()
+    pick = [torch.float32, torch.bfloat16, torch.float16]
+    grads, at = [], 0
+    for k, s in enumerate(sizes):
+        g = flat[at:at + s].to(pick[k % 3])
+        grads.append(g)
+        at += s
+    want = float(torch.cat([g.float() for g in grads]).double().square().sum()) ** 0.5
+    out = F.grad_norm(handle, grads, inv_loss_scale=1.0, max_norm=1.0)
+    assert float(out[0]) == pytest.approx(want, rel=32 * 2 ** -24)
