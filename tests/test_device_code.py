@@ -43,11 +43,19 @@ def test_division_and_sqrt_are_the_correctly_rounded_sequences(device_asm):
     assert any(o.startswith("v_fma_f32") for o in ops)
 
 
-def test_kernels_use_no_scratch_memory_and_no_scalar_stores(device_asm):
+def test_kernels_write_through_vector_memory_and_lds_only(device_asm):
+    """What touches memory is an allow-list: whatever stores or works atomically is a global or an LDS
+    instruction, the scalar unit only ever loads, and nothing lives in scratch memory."""
     ops = _mnemonics(device_asm)
-    bad = sorted(o for o in ops if o.startswith(("scratch_", "s_store", "s_atomic", "s_buffer_store", "s_dcache_wb",
-                                                 "s_dcache_inv")))
+    writes = {o for o in ops if "store" in o or "atomic" in o or o.startswith("ds_write")}
+    assert any(o.startswith("global_store") for o in writes)
+    bad = sorted(o for o in writes if not o.startswith(("global_", "ds_")))
     assert not bad, bad
+    scalar_memory = {o for o in ops if o.startswith("s_") and re.search("load|store|atomic|buffer|cache|scratch|mem", o)}
+    assert scalar_memory
+    bad = sorted(o for o in scalar_memory if not re.fullmatch(r"s_load_dword(x\d+)?", o))
+    assert not bad, bad
+    assert not [o for o in ops if o.startswith("scratch_")]
     sizes = [int(x) for x in re.findall(r"\.private_segment_fixed_size:\s*(\d+)", device_asm)]
     assert sizes and max(sizes) == 0, max(sizes)
 
