@@ -166,6 +166,13 @@ def _descs_ptr(d: np.ndarray):
     return d.ctypes.data_as(ctypes.POINTER(N.RtTensorDesc))
 
 
+def _contiguous_descs(d) -> np.ndarray:
+    """``d`` in one piece; its address goes to the library, which reads ``len(d)`` records there."""
+    if not isinstance(d, np.ndarray) or d.dtype != DESC_DTYPE or d.ndim != 1:
+        raise TypeError(f"expected a one-dimensional array of rt_tensor_desc records, got {type(d).__name__}")
+    return np.ascontiguousarray(d)
+
+
 def launch_resident(handle: N.Handle, descs: np.ndarray, scalars: Sequence[N.RtScalars], *, seed: int,
                     explicit_noise: bool, clip_coef: Optional[torch.Tensor] = None,
                     skip: Optional[torch.Tensor] = None, stream: Optional[int] = None) -> None:
@@ -174,7 +181,7 @@ def launch_resident(handle: N.Handle, descs: np.ndarray, scalars: Sequence[N.RtS
     stream) and returns without synchronising; the caller keeps the tensors alive."""
     if len(descs) == 0:
         return
-    descs = np.ascontiguousarray(descs)
+    descs = _contiguous_descs(descs)
     if stream is None:
         stream = raw_stream(handle.device)
     handle.step_multi_at(descs.ctypes.data, len(descs), scalars_array(scalars), len(scalars), seed & (2 ** 64 - 1),
@@ -247,7 +254,7 @@ def grad_norm(handle: N.Handle, grads: Sequence[torch.Tensor], *, inv_loss_scale
 def grad_norm_rows(handle: N.Handle, descs: np.ndarray, *, inv_loss_scale: float = 1.0,
                    max_norm: float = 1.0) -> torch.Tensor:
     """``grad_norm`` over the gradients of an ``rt_tensor_desc`` array (all on the GPU)."""
-    descs = np.ascontiguousarray(descs)
+    descs = _contiguous_descs(descs)
     out = torch.zeros(4, dtype=torch.float32, device=f"cuda:{handle.device}")
     handle.grad_norm_at(descs.ctypes.data, len(descs), float(inv_loss_scale), float(max_norm), out.data_ptr(),
                         raw_stream(handle.device))

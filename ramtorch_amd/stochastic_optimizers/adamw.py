@@ -674,11 +674,13 @@ class AdamW(Optimizer):
         # ---- everything that can still raise for a bad argument happens before the first launch
         explicit = noise is not None
         work_by_dev = []
-        for dev in sorted(set(plain) | set(resident) | set(streamed) | set(gathered)):
+        # (a device whose tensors all lack gradients has a descriptor buffer without rows: nothing to launch there)
+        with_rows = {dev for dev, slot in gathered.items() if slot[2]}
+        for dev in sorted(set(plain) | set(resident) | set(streamed) | with_rows):
             res, stm = resident.get(dev, []), streamed.get(dev, [])
             lane = plain.get(dev)
             descs = self._plain_descs(dev, lane) if lane is not None else None
-            if dev in gathered and gathered[dev][2]:
+            if dev in with_rows:
                 d0 = gathered[dev][0][:gathered[dev][2]]
                 descs = d0 if descs is None else np.concatenate([d0, descs])
             if res:

@@ -757,3 +757,76 @@ def test_recorded_layout_keeps_its_step_counts_in_step_with_the_states():
     st["ema"] = st["ema"].clone()            # somebody else's does
     assert not G.module().verify_versions(dicts, versions.ctypes.data, 2)
     opt._frozen = None
+
+
+@pytest.fixture
+def launches(monkeypatch):
+    """Steps of CPU parameters as if they lay on one GPU, with the launches recorded instead of made: the
+    gatherer takes device -1 for host memory, and records made by ``_make_rec`` are taken for plain ones."""
+    import contextlib
+    from ramtorch_amd import _gather as G
+    from ramtorch_amd.stochastic_optimizers import adamw as A
+    if G.module() is None:
+        pytest.skip("the gather helper is not built")
+    made = []
+
+    class Handle:
+        device = -1
+
+    class Event:
+        def record(self): pass
+        def synchronize(self): pass
+
+    make_rec = ramtorch_amd.AdamW._make_rec
+    def plain_rec(self, p, tensor_id):
+        r = make_rec(self, p, tensor_id)
+        r.plain, r.dev, r.codes = True, -1, tuple(F.dtype_code(t.dtype, "param") for t in (p, r.m, r.v))
+        return r
+
+    def grad_norm_rows(h, descs, **kw):
+        made.append(("norm", None if descs is None else descs.copy()))
+        return torch.zeros(4)
+
+    empty = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, **kw: empty(*a, **{k: v for k, v in kw.items() if k != "pin_memory"}))
+    monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: -1)
+    monkeypatch.setattr(torch.cuda, "device", lambda dev: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    monkeypatch.setattr(torch.Tensor, "pin_memory", lambda self: self)
+    monkeypatch.setattr(A, "_handle", lambda dev: Handle())
+    monkeypatch.setattr(ramtorch_amd.AdamW, "_make_rec", plain_rec)
+    monkeypatch.setattr(F, "grad_norm_rows", grad_norm_rows)
+    monkeypatch.setattr(F, "launch_resident", lambda h, descs, scalars, **kw: made.append(("step", descs.copy())))
+    return made
+
+
+@pytest.mark.parametrize("groups", [1, 2])
+@pytest.mark.parametrize("given", [None, {}])
+def test_clipped_step_without_any_gradient_launches_nothing(launches, groups, given):
+    """A step under a clip with no gradient anywhere has nothing to take a norm of; with one somewhere the norm
+    runs over the records of exactly those tensors."""
+    ps = [torch.nn.Parameter(torch.zeros(n, dtype=torch.bfloat16)) for n in (8, 5, 300)]
+    opt = ramtorch_amd.AdamW([{"params": ps[:2]}, {"params": ps[2:]}] if groups == 2 else ps, max_grad_norm=1.0)
+    opt.step(grads=given)
+    assert launches == [] and opt.last_grad_norm is None and not opt.step_was_skipped()
+    assert [opt.state[p]["step"] for p in ps] == [0, 0, 0]
+    ps[2].grad = torch.ones_like(ps[2])
+    opt.step(grads=given)
+    assert [(what, len(rows), int(rows["numel"][0])) for what, rows in launches] == [("norm", 1, 300), ("step", 1, 300)]
+    assert [opt.state[p]["step"] for p in ps] == [0, 0, 1]
+
+
+def test_only_descriptor_arrays_reach_the_library():
+    class Handle:
+        device = 0
+
+        def grad_norm_at(self, *a): raise AssertionError("called")
+        step_multi_at = grad_norm_at
+
+    for bad in (None, np.zeros(1, object), np.zeros(200, np.uint8), [1], np.zeros((2, 2), F.DESC_DTYPE)):
+        with pytest.raises(TypeError):
+            F.grad_norm_rows(Handle(), bad)
+        if bad is not None:
+            with pytest.raises(TypeError):
+                F.launch_resident(Handle(), bad, [], seed=0, explicit_noise=False)
