@@ -182,7 +182,7 @@ inline bool sums_rows_itself(const rt_tensor_desc& d) {
 }
 
 // gather_group(params, states, dev, desc_addr, desc_cap, status_addr, scalars_base, tensor_id_base
-//              [, grads, centralize])
+//              [, grads, centralize[, recorded]])
 //   -> (rows_written, [distinct new step values, in order of first use]
 //       [, tensors left to the caller, row means needed])
 // params: list of tensors; states: list of the per-param state dicts (same order);
@@ -193,10 +193,12 @@ inline bool sums_rows_itself(const rt_tensor_desc& d) {
 // centralize: 0, 1 or 2.  Rows get their row_len (adamw.py:179-184: the mean is over every dim but the first, over all
 // of them for 0-d / 1-d); with 2 the update takes the means itself where it can; every other row gets its
 // place among the means, counted in floats from 1, in row_mean (see place_row_means).
+// recorded: the parameters that `states` was made for, in the same order.  A parameter that is another object than the one
+// recorded in its place has other states: it is left to the caller.
 // A call that fails has changed no step count.
 PyObject* gather_group(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-    if (nargs != 8 && nargs != 10) {
-        PyErr_SetString(PyExc_TypeError, "gather_group takes 8 or 10 arguments");
+    if (nargs != 8 && nargs != 10 && nargs != 11) {
+        PyErr_SetString(PyExc_TypeError, "gather_group takes 8, 10 or 11 arguments");
         return nullptr;
     }
     PyObject* params = args[0];
@@ -211,12 +213,14 @@ PyObject* gather_group(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     auto* status = reinterpret_cast<uint8_t*>(PyLong_AsUnsignedLongLong(args[5]));
     const unsigned long scalars_base = PyLong_AsUnsignedLong(args[6]);
     const unsigned long id_base = PyLong_AsUnsignedLong(args[7]);
-    PyObject* grads = nargs == 10 && args[8] != Py_None ? args[8] : nullptr;
-    const long centralize = nargs == 10 ? PyLong_AsLong(args[9]) : 0;
+    PyObject* grads = nargs >= 10 && args[8] != Py_None ? args[8] : nullptr;
+    const long centralize = nargs >= 10 ? PyLong_AsLong(args[9]) : 0;
+    PyObject* recorded = nargs == 11 ? args[10] : nullptr;
     if (PyErr_Occurred()) return nullptr;
     const Py_ssize_t n = PyList_GET_SIZE(params);
-    if (PyList_GET_SIZE(states) != n || !rows || !status || (grads && (!PyList_CheckExact(grads) || PyList_GET_SIZE(grads) != n))) {
-        PyErr_SetString(PyExc_ValueError, "params / states length mismatch, NULL buffer, or grads is not a list of that length");
+    const auto list_of_n = [n](PyObject* o) { return !o || (PyList_CheckExact(o) && PyList_GET_SIZE(o) == n); };
+    if (PyList_GET_SIZE(states) != n || !rows || !status || !list_of_n(grads) || !list_of_n(recorded)) {
+        PyErr_SetString(PyExc_ValueError, "params / states length mismatch, NULL buffer, or grads / recorded is not a list of that length");
         return nullptr;
     }
     // (new step, its number as a Python int): tensors at the same step share the object
@@ -238,7 +242,7 @@ PyObject* gather_group(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         PyObject* so = PyList_GET_ITEM(states, i);
         const c10::TensorImpl* const* im = warm.impl[(size_t)i % kRing];
         const c10::TensorImpl *p = im[0], *g = im[1], *m = im[2], *v = im[3];
-        if (!p || !PyDict_CheckExact(so)) continue;
+        if (!p || !PyDict_CheckExact(so) || (recorded && PyList_GET_ITEM(recorded, i) != po)) continue;
         if (!g) {
             if (grads && PyList_GET_ITEM(grads, i) != Py_None) continue;
             status[i] = kNoGrad;
@@ -309,7 +313,7 @@ PyObject* gather_group(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
             Py_INCREF(steps[k].second);
             PyList_SET_ITEM(lst, (Py_ssize_t)k, steps[k].second);
         }
-        if (lst) out = nargs == 10 ? Py_BuildValue("(nNnK)", w, lst, left, (unsigned long long)means) : Py_BuildValue("(nN)", w, lst);
+        if (lst) out = nargs >= 10 ? Py_BuildValue("(nNnK)", w, lst, left, (unsigned long long)means) : Py_BuildValue("(nN)", w, lst);
     }
     if (!out) {   // put the step counts back; the error stays set
         PyObject *type, *value, *trace;

@@ -546,11 +546,11 @@ class AdamW(Optimizer):
                 buf, addr, used = slot
                 n = len(plist)
                 status, status_addr = self._gather_status(n)
-                states = self._state_list(gi)
+                recorded, states = self._state_list(gi)
                 how = 0 if cen == 0 else 2 if self.__dict__.get("fuse_row_means", True) else 1
                 n_rows, new_steps, left, means = gather.gather_group(
                     plist, states, dev, addr + used * buf.itemsize, len(buf) - used, status_addr, len(scalars),
-                    row[0].tensor_id, None if grads is None else [grads.get(p, p.grad) for p in plist], how)
+                    row[0].tensor_id, None if grads is None else [grads.get(p, p.grad) for p in plist], how, recorded)
                 done = None if n_rows == n else status[:n].copy()
                 journal.append((states, done, gather.WRITTEN))
                 if self.max_grad_norm is not None:
@@ -580,6 +580,7 @@ class AdamW(Optimizer):
                 if (r.p is not p or state.get("ema") is not r.m or state.get("ema_squared") is not r.v
                         or p.data_ptr() != r.p_ptr or r.m.data_ptr() != r.m_ptr or r.v.data_ptr() != r.v_ptr):
                     r = row[k] = self._make_rec(p, r.tensor_id)
+                    self._state_lists.pop(gi, None)
                     state = r.state
                 step = state["step"] + 1  # adamw.py:177
                 journal.append((state, state["step"]))
@@ -953,6 +954,7 @@ class AdamW(Optimizer):
         if (state.get("ema") is not r.m or state.get("ema_squared") is not r.v or p.data_ptr() != r.p_ptr
                 or r.m.data_ptr() != r.m_ptr or r.v.data_ptr() != r.v_ptr):
             r = recs[gi][k] = self._make_rec(p, r.tensor_id)
+            self._state_lists.pop(gi, None)
             state = r.state
         if not (p.is_contiguous() and r.m.is_contiguous() and r.v.is_contiguous()):
             raise NotImplementedError("step_param needs contiguous parameter and state tensors")
@@ -1113,12 +1115,12 @@ class AdamW(Optimizer):
             slot = self._gather_stat = (st, st.ctypes.data)
         return slot
 
-    def _state_list(self, gi: int) -> list:
-        """The state dicts of group ``gi`` in parameter order (cached with the records)."""
-        lst = self._state_lists.get(gi)
-        if lst is None or len(lst) != len(self._recs[gi]):
-            lst = self._state_lists[gi] = [r.state for r in self._recs[gi]]
-        return lst
+    def _state_list(self, gi: int) -> tuple:
+        """The recorded parameters of group ``gi`` and their state dicts, in parameter order (cached with the records)."""
+        pair = self._state_lists.get(gi)
+        if pair is None or len(pair[0]) != len(self._recs[gi]):
+            pair = self._state_lists[gi] = ([r.p for r in self._recs[gi]], [r.state for r in self._recs[gi]])
+        return pair
 
     def _plain_descs(self, dev: int, lane) -> np.ndarray:
         """Descriptor array of the plain lane.  The columns that describe p / m / v are

@@ -798,6 +798,7 @@ def launches(monkeypatch):
     monkeypatch.setattr(ramtorch_amd.AdamW, "_make_rec", plain_rec)
     monkeypatch.setattr(F, "grad_norm_rows", grad_norm_rows)
     monkeypatch.setattr(F, "launch_resident", lambda h, descs, scalars, **kw: made.append(("step", descs.copy())))
+    monkeypatch.setattr(F, "step_streamed", lambda h, entries, scalars, descs, **kw: made.append(("streamed", descs.copy())))
     return made
 
 
@@ -830,3 +831,36 @@ def test_only_descriptor_arrays_reach_the_library():
         if bad is not None:
             with pytest.raises(TypeError):
                 F.launch_resident(Handle(), bad, [], seed=0, explicit_noise=False)
+
+
+def test_replaced_parameter_gets_states_of_its_own(launches):
+    """A wrapper puts another tensor of the same size into ``group["params"]``: it is stepped with states and a step
+    count of its own, by the gatherer as by the Python loop, and the states of the old one are left alone."""
+    routes = []
+
+    def run(gather_min_tensors):
+        del routes[:]
+        ps = [torch.nn.Parameter(torch.zeros(n, dtype=torch.bfloat16)) for n in (8, 5, 300)]
+        opt = ramtorch_amd.AdamW(ps)
+        opt.gather_min_tensors = gather_min_tensors
+        new, seen = torch.nn.Parameter(torch.ones(5, dtype=torch.bfloat16)), []
+        for step in range(4):
+            if step == 2:
+                opt.param_groups[0]["params"][1] = new
+            del launches[:]
+            for p in opt.param_groups[0]["params"]:
+                p.grad = torch.ones_like(p)
+            opt.step()
+            rows = np.concatenate([descs for _, descs in launches])
+            assert (new in opt.state) == (step >= 2)
+            where = {opt.state[p]["ema"].data_ptr(): i for i, p in enumerate((*ps, new)) if p in opt.state}
+            params = {p.data_ptr(): i for i, p in enumerate((*ps, new))}
+            seen.append(sorted((params[int(r["p"])], where[int(r["m"])], int(r["tensor_id"]), int(r["step"])) for r in rows))
+            routes.append([what for what, _ in launches])
+        return seen, [opt.state[p]["step"] for p in (*ps, new)]
+
+    want = [[(0, 0, 0, s), (1, 1, 1, s), (2, 2, 2, s)] for s in (1, 2)] + [[(0, 0, 0, s), (2, 2, 2, s), (3, 3, 1, s - 2)] for s in (3, 4)]
+    for gather_min_tensors in (10 ** 9, 1):
+        assert run(gather_min_tensors) == (want, [4, 2, 4, 2])
+    # the gatherer leaves the replaced one to the loop once (CPU tensors are streamed ones there) and knows it from then on
+    assert routes == [["step"], ["step"], ["step", "streamed"], ["step"]]
