@@ -346,6 +346,24 @@ PyObject* place_row_means(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
 }
 
+// same_objects(flat, lists) -> bool: whether `lists`, one behind the other, hold the very objects of `flat`.
+PyObject* same_objects(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    if (nargs != 2 || !PyList_CheckExact(args[0]) || !PyList_CheckExact(args[1])) {
+        PyErr_SetString(PyExc_TypeError, "same_objects takes a list and a list of lists");
+        return nullptr;
+    }
+    const Py_ssize_t n = PyList_GET_SIZE(args[0]);
+    Py_ssize_t at = 0;
+    for (Py_ssize_t k = 0; k < PyList_GET_SIZE(args[1]); ++k) {
+        PyObject* lst = PyList_GET_ITEM(args[1], k);
+        if (!PyList_Check(lst) || PyList_GET_SIZE(lst) > n - at) Py_RETURN_FALSE;
+        for (Py_ssize_t i = 0; i < PyList_GET_SIZE(lst); ++i)
+            if (PyList_GET_ITEM(lst, i) != PyList_GET_ITEM(args[0], at + i)) Py_RETURN_FALSE;
+        at += PyList_GET_SIZE(lst);
+    }
+    return PyBool_FromLong(at == n);
+}
+
 // verify_layout(params, expect_addr, n) -> bool
 // The cheap per-step check of a frozen layout: params is the flat list of parameters the layout was
 // recorded for, expect_addr the address of n triples of uint64 (data pointer of the parameter, data
@@ -515,6 +533,8 @@ PyMethodDef methods[] = {
      "rt_tensor_desc rows of the plain tensors of one param group"},
     {"place_row_means", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(place_row_means)), METH_FASTCALL,
      "addresses of the row means of gathered rows"},
+    {"same_objects", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(same_objects)), METH_FASTCALL,
+     "whether some lists hold the very objects of another"},
     {"verify_layout", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(verify_layout)), METH_FASTCALL,
      "whether every parameter and gradient of a recorded layout is still where it was"},
     {"dict_versions", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(dict_versions)), METH_FASTCALL,

@@ -822,7 +822,7 @@ class AdamW(Optimizer):
         self._frozen = {"dev": dev, "descs": descs, "params": params, "expect": expect,
                         "states": states, "state_dicts": state_dicts, "versions": versions, "keep": keep,
                         "keys": keys, "pending": 0,
-                        "group_lists": [(g["params"], len(g["params"])) for g in self.param_groups]}
+                        "group_lists": [g["params"] for g in self.param_groups]}
         if not self.assume_static_layout:
             self._freeze_requested = False
 
@@ -831,8 +831,8 @@ class AdamW(Optimizer):
         fz = self._frozen
         groups = self.param_groups
         ok = len(groups) == len(fz["group_lists"]) and all(
-            g["params"] is lst and len(lst) == n and g["centralization"] == 0
-            for g, (lst, n) in zip(groups, fz["group_lists"]))
+            g["params"] is lst and g["centralization"] == 0 for g, lst in zip(groups, fz["group_lists"]))
+        ok = ok and G.module().same_objects(fz["params"], fz["group_lists"])
         ok = ok and self.max_grad_norm is None and getattr(self, "noise_source", "philox") == "philox"
         if ok:
             ok = (fz["state_dicts"][-1] is self.state

@@ -864,3 +864,30 @@ def test_replaced_parameter_gets_states_of_its_own(launches):
         assert run(gather_min_tensors) == (want, [4, 2, 4, 2])
     # the gatherer leaves the replaced one to the loop once (CPU tensors are streamed ones there) and knows it from then on
     assert routes == [["step"], ["step"], ["step", "streamed"], ["step"]]
+
+
+def test_recorded_layout_ends_when_a_parameter_is_replaced(launches):
+    """Another tensor in the same place of the same ``params`` list: the recorded layout does not cover it."""
+    ps = [torch.nn.Parameter(torch.zeros(8, dtype=torch.bfloat16)) for _ in range(300)]
+    opt = ramtorch_amd.AdamW([{"params": ps[:40]}, {"params": ps[40:]}], assume_static_layout=True)
+    for p in ps:
+        p.grad = torch.ones_like(p)
+    for _ in range(3):
+        opt.step()
+    assert opt._frozen is not None and opt._frozen["pending"] == 2 and opt.layout_refreezes == 0
+    new = torch.nn.Parameter(torch.zeros(8, dtype=torch.bfloat16))
+    new.grad = torch.ones_like(new)
+    opt.param_groups[1]["params"][17] = new
+    del launches[:]
+    opt.step()
+    assert opt.layout_refreezes == 1
+    rows = np.concatenate([descs for _, descs in launches])
+    stepped = set(int(x) for x in rows["p"])
+    assert len(rows) == 300 and new.data_ptr() in stepped and ps[57].data_ptr() not in stepped
+    assert opt.state[new]["step"] == 1 and opt.state[ps[57]]["step"] == 3 and opt.state[ps[0]]["step"] == 4
+    # lists of other lengths, in another order, or of another kind are not the recorded ones either
+    from ramtorch_amd import _gather as G
+    same, a, b, c = G.module().same_objects, *ps[:3]
+    assert same([a, b, c], [[a], [], [b, c]]) and same([], []) and same([a], [[a]])
+    for flat, lists in (([a, b], [[a]]), ([a], [[a, b]]), ([a, b], [[b, a]]), ([a, b], [[a], (b,)]), ([a], []), ([], [[a]])):
+        assert not same(flat, lists)
