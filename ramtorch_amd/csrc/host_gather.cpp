@@ -67,6 +67,8 @@ inline int grad_code(const c10::TensorImpl* t) {
 // dev >= 0: on that GPU; dev < 0: in host memory (exercised by the CPU-only tests of this
 // helper; the optimizer only ever passes a GPU index)
 inline bool dense_on(const c10::TensorImpl* t, int dev) {
+    // (function transforms' tensors have no storage; a Python subclass and a nested tensor have sizes of their own kind)
+    if (!t->has_storage() || t->key_set().has(c10::DispatchKey::Python) || t->is_nested()) return false;
     if (t->layout() != at::kStrided || !t->is_contiguous()) return false;
     return dev >= 0 ? (t->is_cuda() && t->get_device() == dev) : t->is_cpu();
 }
@@ -234,77 +236,83 @@ PyObject* gather_group(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     warm.grads = grads;
     warm.n = (size_t)n;
     Py_ssize_t i = 0;
-    for (; i < n; ++i) {
-        warm.ahead_of(i);
-        status[i] = kPython;
-        ++left;
-        PyObject* po = PyList_GET_ITEM(params, i);
-        PyObject* so = PyList_GET_ITEM(states, i);
-        const c10::TensorImpl* const* im = warm.impl[(size_t)i % kRing];
-        const c10::TensorImpl *p = im[0], *g = im[1], *m = im[2], *v = im[3];
-        if (!p || !PyDict_CheckExact(so) || (recorded && PyList_GET_ITEM(recorded, i) != po)) continue;
-        if (!g) {
-            if (grads && PyList_GET_ITEM(grads, i) != Py_None) continue;
-            status[i] = kNoGrad;
-            --left;
-            continue;
-        }
-        if (w >= cap) continue;
-        PyObject* st = entry(so, k_step, h_step);   // (not the one found ahead: the same dict may have had its turn since)
-        if (!m || !v || !st || !PyLong_CheckExact(st)) continue;
-        const int pc = pmv_code(p), mc = pmv_code(m), vc = pmv_code(v), gc = grad_code(g);
-        if (pc < 0 || mc < 0 || vc < 0 || gc < 0) continue;
-        if (!dense_on(p, (int)dev) || !dense_on(g, (int)dev) || !dense_on(m, (int)dev) || !dense_on(v, (int)dev))
-            continue;
-        const int64_t numel = p->numel();
-        if (g->numel() != numel || m->numel() != numel || v->numel() != numel) continue;
-        int overflow = 0;
-        const long long step = PyLong_AsLongLongAndOverflow(st, &overflow);
-        if (overflow || step < 0) continue;
-        const long long new_step = step + 1;  // adamw.py:177
-        size_t si = steps.size();
-        for (size_t k = steps.size(); k-- > 0;)
-            if (steps[k].first == new_step) {
-                si = k;
-                break;
+    try {
+        for (; i < n; ++i) {
+            warm.ahead_of(i);
+            status[i] = kPython;
+            ++left;
+            PyObject* po = PyList_GET_ITEM(params, i);
+            PyObject* so = PyList_GET_ITEM(states, i);
+            const c10::TensorImpl* const* im = warm.impl[(size_t)i % kRing];
+            const c10::TensorImpl *p = im[0], *g = im[1], *m = im[2], *v = im[3];
+            if (!p || !PyDict_CheckExact(so) || (recorded && PyList_GET_ITEM(recorded, i) != po)) continue;
+            if (!g) {
+                if (grads && PyList_GET_ITEM(grads, i) != Py_None) continue;
+                status[i] = kNoGrad;
+                --left;
+                continue;
             }
-        if (si == steps.size()) {
-            PyObject* ns = PyLong_FromLongLong(new_step);
-            if (!ns) {
+            if (w >= cap) continue;
+            PyObject* st = entry(so, k_step, h_step);   // (not the one found ahead: the same dict may have had its turn since)
+            if (!m || !v || !st || !PyLong_CheckExact(st)) continue;
+            const int pc = pmv_code(p), mc = pmv_code(m), vc = pmv_code(v), gc = grad_code(g);
+            if (pc < 0 || mc < 0 || vc < 0 || gc < 0) continue;
+            if (!dense_on(p, (int)dev) || !dense_on(g, (int)dev) || !dense_on(m, (int)dev) || !dense_on(v, (int)dev))
+                continue;
+            const int64_t numel = p->numel();
+            if (g->numel() != numel || m->numel() != numel || v->numel() != numel) continue;
+            int overflow = 0;
+            const long long step = PyLong_AsLongLongAndOverflow(st, &overflow);
+            if (overflow || step < 0) continue;
+            const long long new_step = step + 1;  // adamw.py:177
+            size_t si = steps.size();
+            for (size_t k = steps.size(); k-- > 0;)
+                if (steps[k].first == new_step) {
+                    si = k;
+                    break;
+                }
+            if (si == steps.size()) {
+                PyObject* ns = PyLong_FromLongLong(new_step);
+                if (!ns) {
+                    failed = true;
+                    break;
+                }
+                steps.emplace_back(new_step, ns);
+            }
+
+            rt_tensor_desc d{};
+            d.p = data_of(p);
+            d.g = data_of(g);
+            d.m = data_of(m);
+            d.v = data_of(v);
+            d.numel = (uint64_t)numel;
+            d.tensor_id = (uint32_t)(id_base + (unsigned long)i);
+            d.step = (uint32_t)((unsigned long long)new_step & 0xFFFFFFFFull);
+            d.scalars_idx = (uint32_t)(scalars_base + si);
+            d.p_dtype = (uint8_t)pc;
+            d.g_dtype = (uint8_t)gc;
+            d.m_dtype = (uint8_t)mc;
+            d.v_dtype = (uint8_t)vc;
+            uint64_t count = 0;   // rows that need a mean
+            if (centralize && numel > 0) {
+                count = g->dim() >= 2 ? (uint64_t)g->size(0) : 1;
+                d.row_len = (uint64_t)numel / count;
+                if (centralize == 2 && sums_rows_itself(d)) count = 0;
+                else d.row_mean = reinterpret_cast<float*>(means + 1);
+            }
+            // from here on nothing can fail but the dict
+            if (PyDict_SetItem(so, k_step, steps[si].second) != 0) {
                 failed = true;
                 break;
             }
-            steps.emplace_back(new_step, ns);
+            rows[w++] = d;
+            means += count;
+            status[i] = kWritten;
+            --left;
         }
-        if (PyDict_SetItem(so, k_step, steps[si].second) != 0) {
-            failed = true;
-            break;
-        }
-
-        rt_tensor_desc d{};
-        d.p = data_of(p);
-        d.g = data_of(g);
-        d.m = data_of(m);
-        d.v = data_of(v);
-        d.numel = (uint64_t)numel;
-        d.tensor_id = (uint32_t)(id_base + (unsigned long)i);
-        d.step = (uint32_t)((unsigned long long)new_step & 0xFFFFFFFFull);
-        d.scalars_idx = (uint32_t)(scalars_base + si);
-        d.p_dtype = (uint8_t)pc;
-        d.g_dtype = (uint8_t)gc;
-        d.m_dtype = (uint8_t)mc;
-        d.v_dtype = (uint8_t)vc;
-        status[i] = kWritten;
-        --left;
-        if (centralize && numel > 0) {
-            const uint64_t count = g->dim() >= 2 ? (uint64_t)g->size(0) : 1;
-            d.row_len = (uint64_t)numel / count;
-            if (centralize != 2 || !sums_rows_itself(d)) {
-                d.row_mean = reinterpret_cast<float*>(means + 1);
-                means += count;
-            }
-        }
-        rows[w++] = d;
+    } catch (const std::exception& e) {   // torch does not give away a tensor's sizes or memory
+        if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
+        failed = true;
     }
     PyObject* out = nullptr;
     if (!failed) {
@@ -407,14 +415,14 @@ bool verify_range(PyObject* params, const uint64_t* expect, Py_ssize_t lo, Py_ss
         PyObject* po = PyList_GET_ITEM(params, i);
         if (!exact_tensor(po)) return false;
         const at::Tensor& p = THPVariable_Unpack(po);
-        if (reinterpret_cast<uint64_t>(p.data_ptr()) != expect[3 * i]) return false;
+        if (!p.has_storage() || reinterpret_cast<uint64_t>(p.data_ptr()) != expect[3 * i]) return false;
         const at::Tensor& g = p.grad();
         const uint64_t want = expect[3 * i + 1];
         if (!g.defined()) {
             if (want != 0) return false;
             continue;
         }
-        if (want == 0 || g.layout() != at::kStrided || !g.is_contiguous() || g.numel() != p.numel() ||
+        if (want == 0 || !g.has_storage() || g.key_set().has(c10::DispatchKey::Python) || g.layout() != at::kStrided || !g.is_contiguous() || g.numel() != p.numel() ||
             reinterpret_cast<uint64_t>(g.data_ptr()) != want || (uint64_t)grad_code(g.unsafeGetTensorImpl()) != expect[3 * i + 2])
             return false;
     }

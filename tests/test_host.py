@@ -891,3 +891,52 @@ def test_recorded_layout_ends_when_a_parameter_is_replaced(launches):
     assert same([a, b, c], [[a], [], [b, c]]) and same([], []) and same([a], [[a]])
     for flat, lists in (([a, b], [[a]]), ([a], [[a, b]]), ([a, b], [[b, a]]), ([a, b], [[a], (b,)]), ([a], []), ([], [[a]])):
         assert not same(flat, lists)
+
+
+class _Wrapped(torch.Tensor):
+    """A tensor without memory that leaves every operation to Python."""
+    @staticmethod
+    def __new__(cls, like):
+        return torch.Tensor._make_wrapper_subclass(cls, like.shape, dtype=like.dtype)
+
+    __torch_function__ = torch._C._disabled_torch_function_impl
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        raise NotImplementedError(str(func))
+
+
+def test_gatherer_leaves_unusual_gradients_to_the_caller():
+    """Gradients inside a function transform, of a wrapper class, or nested: left to the caller, who raises as
+    for any of them, and their step count has not moved."""
+    import subprocess
+    import sys
+    from ramtorch_amd import _gather as G
+    if G.module() is None:
+        pytest.skip("the gather helper is not built")
+    # (in a process of its own: an exception that leaves the helper would end it)
+    code = r"""
+import warnings, numpy as np, torch
+warnings.simplefilter("ignore")
+from ramtorch_amd import _gather as G, functional as F
+from tests.test_host import _Wrapped
+def gather(g, own, centralize):
+    ps = [torch.nn.Parameter(torch.zeros(8), requires_grad=False) for _ in range(3)]
+    states = [{"step": 5, "ema": torch.zeros(8), "ema_squared": torch.zeros(8)} for _ in ps]
+    given = [torch.ones(8), g, torch.ones(8)]
+    if own:
+        for p, x in zip(ps, given):
+            p.grad = x
+    rows, status = np.zeros(3, F.DESC_DTYPE), np.zeros(3, np.uint8)
+    n, *_ = G.module().gather_group(ps, states, -1, rows.ctypes.data, 3, status.ctypes.data, 0, 0, None if own else given, centralize)
+    assert n == 2 and [s["step"] for s in states] == [6, 5, 6] and status[1] == G.module().PYTHON
+    return "left"
+for centralize in (0, 1):
+    torch.vmap(lambda x: (print(gather(x, False, centralize)), x)[1])(torch.zeros(3, 8))
+    print(gather(_Wrapped(torch.zeros(8)), True, centralize))
+    print(gather(torch.nested.nested_tensor([torch.zeros(3), torch.zeros(5)]), False, centralize))
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300, cwd=root)
+    assert res.returncode == 0, res.stderr[-2000:]
+    assert res.stdout.split() == ["left"] * 6
