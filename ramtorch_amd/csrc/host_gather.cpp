@@ -67,10 +67,15 @@ inline int grad_code(const c10::TensorImpl* t) {
 // dev >= 0: on that GPU; dev < 0: in host memory (exercised by the CPU-only tests of this
 // helper; the optimizer only ever passes a GPU index)
 inline bool dense_on(const c10::TensorImpl* t, int dev) {
-    // (function transforms' tensors have no storage; a Python subclass and a nested tensor have sizes of their own kind)
-    if (!t->has_storage() || t->key_set().has(c10::DispatchKey::Python) || t->is_nested()) return false;
     if (t->layout() != at::kStrided || !t->is_contiguous()) return false;
     return dev >= 0 ? (t->is_cuda() && t->get_device() == dev) : t->is_cpu();
+}
+
+// Function transforms' tensors have no storage; a Python subclass and a nested tensor have sizes of their own kind.
+inline bool ordinary(const c10::TensorImpl* t) {
+    const uint64_t odd = c10::DispatchKeySet(c10::DispatchKey::Python).raw_repr() |
+                         c10::DispatchKeySet(c10::DispatchKey::NestedTensor).raw_repr();
+    return (t->key_set().raw_repr() & odd) == 0 && t->has_storage();
 }
 
 inline void* data_of(const c10::TensorImpl* t) { return const_cast<c10::TensorImpl*>(t)->mutable_data(); }
@@ -183,6 +188,112 @@ inline bool sums_rows_itself(const rt_tensor_desc& d) {
            narrow(d.m_dtype) && narrow(d.v_dtype) && (d.m_dtype == RT_DT_F16) == (d.v_dtype == RT_DT_F16);
 }
 
+// (new step, its number as a Python int): tensors at the same step share the object
+using Steps = std::vector<std::pair<long long, PyObject*>>;
+
+struct Walk {
+    PyObject *params, *states, *grads, *recorded;   // the last two may be NULL
+    Py_ssize_t n, cap;
+    int dev;
+    long centralize;
+    unsigned long scalars_base, id_base;
+    rt_tensor_desc* rows;
+    uint8_t* status;       // kPython everywhere when the walk begins
+    Py_ssize_t written, left;   // results
+    uint64_t means;
+};
+
+// The walk of gather_group.  False: a Python error is set.  It may throw as well, where torch does not give away a
+// tensor's sizes or memory; either way `status` says which step counts have moved, and those tensors' rows by how much.
+bool walk_group(Walk& a, Steps& steps) {
+    PyObject *const params = a.params, *const states = a.states, *const grads = a.grads, *const recorded = a.recorded;
+    const Py_ssize_t n = a.n, cap = a.cap;
+    const int dev = a.dev;
+    const long centralize = a.centralize;
+    const unsigned long scalars_base = a.scalars_base, id_base = a.id_base;
+    rt_tensor_desc* const rows = a.rows;
+    uint8_t* const status = a.status;
+    Py_ssize_t w = 0, left = 0;
+    uint64_t means = 0;
+    Warm warm;
+    warm.params = params;
+    warm.states = states;
+    warm.grads = grads;
+    warm.n = (size_t)n;
+    for (Py_ssize_t i = 0; i < n; ++i) {
+        warm.ahead_of(i);
+        ++left;
+        PyObject* po = PyList_GET_ITEM(params, i);
+        PyObject* so = PyList_GET_ITEM(states, i);
+        const c10::TensorImpl* const* im = warm.impl[(size_t)i % kRing];
+        const c10::TensorImpl *p = im[0], *g = im[1], *m = im[2], *v = im[3];
+        if (!p || !PyDict_CheckExact(so) || (recorded && PyList_GET_ITEM(recorded, i) != po)) continue;
+        if (!g) {
+            if (grads && PyList_GET_ITEM(grads, i) != Py_None) continue;
+            status[i] = kNoGrad;
+            --left;
+            continue;
+        }
+        if (w >= cap) continue;
+        PyObject* st = entry(so, k_step, h_step);   // (not the one found ahead: the same dict may have had its turn since)
+        if (!m || !v || !st || !PyLong_CheckExact(st)) continue;
+        const int pc = pmv_code(p), mc = pmv_code(m), vc = pmv_code(v), gc = grad_code(g);
+        if (pc < 0 || mc < 0 || vc < 0 || gc < 0) continue;
+        if (!ordinary(g) || !dense_on(p, dev) || !dense_on(g, dev) || !dense_on(m, dev) || !dense_on(v, dev))
+            continue;
+        const int64_t numel = p->numel();
+        if (g->numel() != numel || m->numel() != numel || v->numel() != numel) continue;
+        int overflow = 0;
+        const long long step = PyLong_AsLongLongAndOverflow(st, &overflow);
+        if (overflow || step < 0) continue;
+        const long long new_step = step + 1;  // adamw.py:177
+        size_t si = steps.size();
+        for (size_t k = steps.size(); k-- > 0;)
+            if (steps[k].first == new_step) {
+                si = k;
+                break;
+            }
+        if (si == steps.size()) {
+            PyObject* ns = PyLong_FromLongLong(new_step);
+            if (!ns) return false;
+            steps.emplace_back(new_step, ns);
+        }
+        if (PyDict_SetItem(so, k_step, steps[si].second) != 0) return false;
+        // (what putting the count back takes; with the addresses read before the dict is written the walk measured
+        // 124 ns a tensor instead of 105)
+        rows[w].scalars_idx = (uint32_t)(scalars_base + si);
+        status[i] = kWritten;
+
+        rt_tensor_desc d{};
+        d.p = data_of(p);
+        d.g = data_of(g);
+        d.m = data_of(m);
+        d.v = data_of(v);
+        d.numel = (uint64_t)numel;
+        d.tensor_id = (uint32_t)(id_base + (unsigned long)i);
+        d.step = (uint32_t)((unsigned long long)new_step & 0xFFFFFFFFull);
+        d.scalars_idx = (uint32_t)(scalars_base + si);
+        d.p_dtype = (uint8_t)pc;
+        d.g_dtype = (uint8_t)gc;
+        d.m_dtype = (uint8_t)mc;
+        d.v_dtype = (uint8_t)vc;
+        --left;
+        if (centralize && numel > 0) {
+            const uint64_t count = g->dim() >= 2 ? (uint64_t)g->size(0) : 1;
+            d.row_len = (uint64_t)numel / count;
+            if (centralize != 2 || !sums_rows_itself(d)) {
+                d.row_mean = reinterpret_cast<float*>(means + 1);
+                means += count;
+            }
+        }
+        rows[w++] = d;
+    }
+    a.written = w;
+    a.left = left;
+    a.means = means;
+    return true;
+}
+
 // gather_group(params, states, dev, desc_addr, desc_cap, status_addr, scalars_base, tensor_id_base
 //              [, grads, centralize[, recorded]])
 //   -> (rows_written, [distinct new step values, in order of first use]
@@ -225,108 +336,28 @@ PyObject* gather_group(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         PyErr_SetString(PyExc_ValueError, "params / states length mismatch, NULL buffer, or grads / recorded is not a list of that length");
         return nullptr;
     }
-    // (new step, its number as a Python int): tensors at the same step share the object
-    std::vector<std::pair<long long, PyObject*>> steps;
-    Py_ssize_t w = 0, left = 0;
-    uint64_t means = 0;
-    bool failed = false;
-    Warm warm;
-    warm.params = params;
-    warm.states = states;
-    warm.grads = grads;
-    warm.n = (size_t)n;
-    Py_ssize_t i = 0;
+    Walk a{params, states, grads, recorded, n, cap, (int)dev, centralize, scalars_base, id_base, rows, status, 0, 0, 0};
+    Steps steps;
+    std::memset(status, kPython, (size_t)n);
+    bool ok = false;
     try {
-        for (; i < n; ++i) {
-            warm.ahead_of(i);
-            status[i] = kPython;
-            ++left;
-            PyObject* po = PyList_GET_ITEM(params, i);
-            PyObject* so = PyList_GET_ITEM(states, i);
-            const c10::TensorImpl* const* im = warm.impl[(size_t)i % kRing];
-            const c10::TensorImpl *p = im[0], *g = im[1], *m = im[2], *v = im[3];
-            if (!p || !PyDict_CheckExact(so) || (recorded && PyList_GET_ITEM(recorded, i) != po)) continue;
-            if (!g) {
-                if (grads && PyList_GET_ITEM(grads, i) != Py_None) continue;
-                status[i] = kNoGrad;
-                --left;
-                continue;
-            }
-            if (w >= cap) continue;
-            PyObject* st = entry(so, k_step, h_step);   // (not the one found ahead: the same dict may have had its turn since)
-            if (!m || !v || !st || !PyLong_CheckExact(st)) continue;
-            const int pc = pmv_code(p), mc = pmv_code(m), vc = pmv_code(v), gc = grad_code(g);
-            if (pc < 0 || mc < 0 || vc < 0 || gc < 0) continue;
-            if (!dense_on(p, (int)dev) || !dense_on(g, (int)dev) || !dense_on(m, (int)dev) || !dense_on(v, (int)dev))
-                continue;
-            const int64_t numel = p->numel();
-            if (g->numel() != numel || m->numel() != numel || v->numel() != numel) continue;
-            int overflow = 0;
-            const long long step = PyLong_AsLongLongAndOverflow(st, &overflow);
-            if (overflow || step < 0) continue;
-            const long long new_step = step + 1;  // adamw.py:177
-            size_t si = steps.size();
-            for (size_t k = steps.size(); k-- > 0;)
-                if (steps[k].first == new_step) {
-                    si = k;
-                    break;
-                }
-            if (si == steps.size()) {
-                PyObject* ns = PyLong_FromLongLong(new_step);
-                if (!ns) {
-                    failed = true;
-                    break;
-                }
-                steps.emplace_back(new_step, ns);
-            }
-
-            rt_tensor_desc d{};
-            d.p = data_of(p);
-            d.g = data_of(g);
-            d.m = data_of(m);
-            d.v = data_of(v);
-            d.numel = (uint64_t)numel;
-            d.tensor_id = (uint32_t)(id_base + (unsigned long)i);
-            d.step = (uint32_t)((unsigned long long)new_step & 0xFFFFFFFFull);
-            d.scalars_idx = (uint32_t)(scalars_base + si);
-            d.p_dtype = (uint8_t)pc;
-            d.g_dtype = (uint8_t)gc;
-            d.m_dtype = (uint8_t)mc;
-            d.v_dtype = (uint8_t)vc;
-            uint64_t count = 0;   // rows that need a mean
-            if (centralize && numel > 0) {
-                count = g->dim() >= 2 ? (uint64_t)g->size(0) : 1;
-                d.row_len = (uint64_t)numel / count;
-                if (centralize == 2 && sums_rows_itself(d)) count = 0;
-                else d.row_mean = reinterpret_cast<float*>(means + 1);
-            }
-            // from here on nothing can fail but the dict
-            if (PyDict_SetItem(so, k_step, steps[si].second) != 0) {
-                failed = true;
-                break;
-            }
-            rows[w++] = d;
-            means += count;
-            status[i] = kWritten;
-            --left;
-        }
-    } catch (const std::exception& e) {   // torch does not give away a tensor's sizes or memory
+        ok = walk_group(a, steps);
+    } catch (const std::exception& e) {
         if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
-        failed = true;
     }
     PyObject* out = nullptr;
-    if (!failed) {
+    if (ok) {
         PyObject* lst = PyList_New((Py_ssize_t)steps.size());
         for (size_t k = 0; lst && k < steps.size(); ++k) {
             Py_INCREF(steps[k].second);
             PyList_SET_ITEM(lst, (Py_ssize_t)k, steps[k].second);
         }
-        if (lst) out = nargs >= 10 ? Py_BuildValue("(nNnK)", w, lst, left, (unsigned long long)means) : Py_BuildValue("(nN)", w, lst);
+        if (lst) out = nargs >= 10 ? Py_BuildValue("(nNnK)", a.written, lst, a.left, (unsigned long long)a.means) : Py_BuildValue("(nN)", a.written, lst);
     }
     if (!out) {   // put the step counts back; the error stays set
         PyObject *type, *value, *trace;
         PyErr_Fetch(&type, &value, &trace);
-        for (Py_ssize_t k = 0, r = 0; k < i; ++k) {
+        for (Py_ssize_t k = 0, r = 0; k < n; ++k) {
             if (status[k] != kWritten) continue;
             PyObject* old = PyLong_FromLongLong(steps[rows[r++].scalars_idx - scalars_base].first - 1);
             if (!old || PyDict_SetItem(PyList_GET_ITEM(states, k), k_step, old) != 0) PyErr_Clear();
@@ -422,7 +453,7 @@ bool verify_range(PyObject* params, const uint64_t* expect, Py_ssize_t lo, Py_ss
             if (want != 0) return false;
             continue;
         }
-        if (want == 0 || !g.has_storage() || g.key_set().has(c10::DispatchKey::Python) || g.layout() != at::kStrided || !g.is_contiguous() || g.numel() != p.numel() ||
+        if (want == 0 || !ordinary(g.unsafeGetTensorImpl()) || g.layout() != at::kStrided || !g.is_contiguous() || g.numel() != p.numel() ||
             reinterpret_cast<uint64_t>(g.data_ptr()) != want || (uint64_t)grad_code(g.unsafeGetTensorImpl()) != expect[3 * i + 2])
             return false;
     }

@@ -907,8 +907,8 @@ class _Wrapped(torch.Tensor):
 
 
 def test_gatherer_leaves_unusual_gradients_to_the_caller():
-    """Gradients inside a function transform, of a wrapper class, or nested: left to the caller, who raises as
-    for any of them, and their step count has not moved."""
+    """Gradients inside a function transform, of a wrapper class, or nested: left to the caller, and their step count
+    has not moved.  A state whose memory torch does not give away: an error, and no step count has moved."""
     import subprocess
     import sys
     from ramtorch_amd import _gather as G
@@ -920,23 +920,30 @@ import warnings, numpy as np, torch
 warnings.simplefilter("ignore")
 from ramtorch_amd import _gather as G, functional as F
 from tests.test_host import _Wrapped
-def gather(g, own, centralize):
+def gather(g, own, centralize, ema=None):
     ps = [torch.nn.Parameter(torch.zeros(8), requires_grad=False) for _ in range(3)]
     states = [{"step": 5, "ema": torch.zeros(8), "ema_squared": torch.zeros(8)} for _ in ps]
     given = [torch.ones(8), g, torch.ones(8)]
+    if ema is not None:
+        states[1]["ema"] = ema
     if own:
         for p, x in zip(ps, given):
             p.grad = x
     rows, status = np.zeros(3, F.DESC_DTYPE), np.zeros(3, np.uint8)
-    n, *_ = G.module().gather_group(ps, states, -1, rows.ctypes.data, 3, status.ctypes.data, 0, 0, None if own else given, centralize)
+    try:
+        n, *_ = G.module().gather_group(ps, states, -1, rows.ctypes.data, 3, status.ctypes.data, 0, 0, None if own else given, centralize)
+    except RuntimeError:
+        assert [s["step"] for s in states] == [5, 5, 5]
+        return "error"
     assert n == 2 and [s["step"] for s in states] == [6, 5, 6] and status[1] == G.module().PYTHON
     return "left"
 for centralize in (0, 1):
     torch.vmap(lambda x: (print(gather(x, False, centralize)), x)[1])(torch.zeros(3, 8))
     print(gather(_Wrapped(torch.zeros(8)), True, centralize))
     print(gather(torch.nested.nested_tensor([torch.zeros(3), torch.zeros(5)]), False, centralize))
+    torch.vmap(lambda x: (print(gather(torch.ones(8), True, centralize, ema=x)), x)[1])(torch.zeros(3, 8))
 """
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300, cwd=root)
     assert res.returncode == 0, res.stderr[-2000:]
-    assert res.stdout.split() == ["left"] * 6
+    assert res.stdout.split() == (["left"] * 3 + ["error"]) * 2
