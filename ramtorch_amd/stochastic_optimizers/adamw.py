@@ -21,7 +21,7 @@ from .. import _native as N
 from .. import functional as F
 
 _handles: Dict[int, N.Handle] = {}
-_FREEZE_MIN_TENSORS = 256   # shorter parameter lists are walked faster than a recorded layout is set up
+_GATHER_MIN_TENSORS = 256   # default of AdamW.gather_min_tensors
 
 
 def _handle(device_index: int) -> N.Handle:
@@ -175,7 +175,9 @@ class AdamW(Optimizer):
         self.max_inflight_bytes = 2 << 30  # gradients kept alive for updates still in flight (step_param)
         self.max_inflight_calls = 2       # staging chunks handed to the copy pipeline and not finished yet
         self._poll_seconds = 0.0002       # completion is read from host memory; no runtime call while waiting
-        self.gather_min_tensors = 1       # from this many parameters on, step() gathers descriptors in C++
+        # From this many parameters on, a layout may be recorded (freeze_layout).  step() gathers descriptors in C++ for
+        # sets of any size; a value above the default keeps sets shorter than it in the Python loop.
+        self.gather_min_tensors = _GATHER_MIN_TENSORS
         self._gather_bufs = {}            # device -> descriptor rows the gatherer fills
         self._gather_stat = None
         self._state_lists = {}
@@ -207,7 +209,7 @@ class AdamW(Optimizer):
                             max_grad_norm=None, noise_source="philox", fuse_in_backward=True, host_arrays_ordered=False,
                             fuse_row_means=True,
                             max_inflight_bytes=2 << 30, max_inflight_calls=2, _poll_seconds=0.0002,
-                            gather_min_tensors=1, state_placement="auto", state_pool_min_bytes=1 << 30,
+                            gather_min_tensors=_GATHER_MIN_TENSORS, state_placement="auto", state_pool_min_bytes=1 << 30,
                             assume_static_layout=False)
 
     def __getstate__(self):
@@ -523,7 +525,8 @@ class AdamW(Optimizer):
         # Groups of plain GPU tensors are walked in C++ when the helper is built; it writes
         # their descriptor rows and advances their step counts, and leaves the rest to the loop below.
         gather = None
-        if not extras and not early and sum(len(g["params"]) for g in self.param_groups) >= self.gather_min_tensors:
+        if not extras and not early and (self.gather_min_tensors <= _GATHER_MIN_TENSORS
+                                         or sum(len(g["params"]) for g in self.param_groups) >= self.gather_min_tensors):
             gather = G.module()
         gathered: Dict[int, list] = {}    # dev -> [descriptor buffer, its address, rows used]
         gathered_means: Dict[int, list] = {}   # dev -> [(first row, rows, row means they need)] of centralized groups
@@ -734,8 +737,8 @@ class AdamW(Optimizer):
         sets of thousands of small tensors whose gradients keep their storage from step to step
         (``zero_grad(set_to_none=False)`` or gradients accumulated in place).
 
-        Applies to steps that the C++ gatherer covers completely: one GPU, at least 256
-        parameters, every stepping tensor plain (contiguous, on the GPU), no
+        Applies to steps that the C++ gatherer covers completely: one GPU, at least
+        ``gather_min_tensors`` (256) parameters, every stepping tensor plain (contiguous, on the GPU), no
         ``centralization`` / ``max_grad_norm`` / ``noise_source="reference"`` / ``step_param``.
         Otherwise nothing is recorded and steps run as usual.
 
@@ -779,7 +782,7 @@ class AdamW(Optimizer):
         self._frozen = None
         if (explicit or plain or resident or streamed or len(gathered) != 1 or self.max_grad_norm is not None
                 or any(g["centralization"] != 0 for g in self.param_groups)
-                or sum(len(g["params"]) for g in self.param_groups) < _FREEZE_MIN_TENSORS
+                or sum(len(g["params"]) for g in self.param_groups) < self.gather_min_tensors
                 or G.module() is None or not hasattr(G.module(), "verify_layout")):
             return
         (dev, (buf, _, rows)), = gathered.items()

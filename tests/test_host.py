@@ -947,3 +947,22 @@ for centralize in (0, 1):
     res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300, cwd=root)
     assert res.returncode == 0, res.stderr[-2000:]
     assert res.stdout.split() == (["left"] * 3 + ["error"]) * 2
+
+
+@pytest.mark.parametrize("gather_min_tensors,recorded,walked", [(None, False, True), (1, True, True), (40, True, True),
+                                                                 (41, False, True), (10 ** 9, False, False)])
+def test_which_sets_are_walked_in_cpp_and_recorded(launches, gather_min_tensors, recorded, walked):
+    """Sets of any size are gathered in C++ unless ``gather_min_tensors`` is set above its default and above their
+    size; layouts are recorded from ``gather_min_tensors`` parameters on."""
+    ps = [torch.nn.Parameter(torch.zeros(8, dtype=torch.bfloat16)) for _ in range(40)]
+    opt = ramtorch_amd.AdamW(ps, assume_static_layout=True)
+    if gather_min_tensors is not None:
+        opt.gather_min_tensors = gather_min_tensors
+    for p in ps:
+        p.grad = torch.ones_like(p)
+    for _ in range(3):
+        opt.step()
+    assert [what for what, _ in launches] == ["step" if walked else "streamed"] * 3   # (CPU tensors: streamed ones in the loop)
+    assert (opt._frozen is not None) == recorded and (not recorded or opt._frozen["pending"] == 2)
+    opt.unfreeze_layout()
+    assert [opt.state[p]["step"] for p in ps] == [3] * 40
