@@ -143,7 +143,8 @@ int rt_step_multi(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, const r
  * grad, p) and :204-222 (D2H write-back).  When every host array of the call is
  * pinned (and mapped, and not hipHostMallocNonCoherent) the update kernels read
  * and write it in place over the host link, on a stream of the handle and with
- * 32 workgroups, and nothing is staged.  Otherwise -- an array in ordinary CPU
+ * 32 workgroups, and nothing is staged (tensors of the call that lie on the
+ * device altogether run in a launch of their own, as in rt_step_multi).  Otherwise -- an array in ordinary CPU
  * memory, explicit noise, more than 512 chunks of 8192 elements with debug
  * outputs, in a runtime-typed layout or with centralized rows shorter than 8 --
  * chunks of `chunk_elems` elements are moved H2D / updated / moved D2H on three

@@ -1538,13 +1538,16 @@ static void* mapped_host(const void* host, size_t bytes) {
     return first.devicePointer;
 }
 
-// The descriptors with every host array replaced by its mapped address; false if one has none.
-static bool map_host_arrays(const rt_tensor_desc* descs, uint32_t n, std::vector<rt_tensor_desc>& out, double& bytes_up,
-                            double& bytes_down) {
-    out.assign(descs, descs + n);
+// The descriptors with host arrays, each replaced by its mapped address, and the ones without; false if a host array
+// has no such address.
+static bool map_host_arrays(const rt_tensor_desc* descs, uint32_t n, std::vector<rt_tensor_desc>& over_link,
+                            std::vector<rt_tensor_desc>& resident, double& bytes_up, double& bytes_down) {
+    over_link.clear();
+    resident.clear();
     bytes_up = bytes_down = 0;
-    for (rt_tensor_desc& d : out) {
-        const uint32_t mask = d.host_mask;
+    for (uint32_t i = 0; i < n; ++i) {
+        rt_tensor_desc d = descs[i];
+        const uint32_t mask = d.host_mask & (RT_HOST_P | RT_HOST_G | RT_HOST_M | RT_HOST_V);
         d.host_mask = 0;
         if (d.numel == 0) continue;
         const int es[4] = {dtype_size(d.p_dtype), dtype_size(d.g_dtype), dtype_size(d.m_dtype), dtype_size(d.v_dtype)};
@@ -1558,22 +1561,25 @@ static bool map_host_arrays(const rt_tensor_desc* descs, uint32_t n, std::vector
             if (a != 1) bytes_down += (double)bytes;
         }
         d.p = at[0]; d.g = at[1]; d.m = at[2]; d.v = at[3];
+        (mask ? over_link : resident).push_back(d);
     }
     return true;
 }
 
-// Enqueues one call whose table image (`plan`, h->image) addresses host memory directly.
-static int streamed_in_place(rt_handle* h, const Plan& plan, uint64_t seed, const float* d_clip_coef,
-                             const uint32_t* d_skip, hipStream_t user, bool trace) {
+// Enqueues one call that addresses host memory directly: `image` holds the table images of the tensors over the
+// link (`link`, at its begin) and of the ones that lie on the device altogether (`resident`, at `resident_off`).
+static int streamed_in_place(rt_handle* h, const Plan& link, const Plan& resident, const std::vector<uint8_t>& image,
+                             size_t resident_off, uint64_t seed, const float* d_clip_coef, const uint32_t* d_skip,
+                             hipStream_t user, bool trace) {
     Streamed& st = h->st;
     Streamed::TableRing* tab = nullptr;
-    int rc = streamed_table(h, h->image.data(), plan.bytes, &tab);
+    int rc = streamed_table(h, image.data(), image.size(), &tab);
     if (rc != RT_OK) return rc;
     // the kernels wait for everything queued on the caller's stream, whichever arrays it writes
     HIP_TRY(hipEventRecord(st.start, user));
     HIP_TRY(hipStreamWaitEvent(st.comp, st.start, 0));
     st.pending = true;
-    rc = upload_table(h, *tab, plan.bytes);
+    rc = upload_table(h, *tab, image.size());
     if (rc != RT_OK) return rc;
     if (trace) {   // one row: up and down are one kernel's time
         while (st.tl_events.size() < 4) {
@@ -1583,7 +1589,10 @@ static int streamed_in_place(rt_handle* h, const Plan& plan, uint64_t seed, cons
         }
         for (int k = 0; k < 4; k += 2) HIP_TRY(hipEventRecord(st.tl_events[k], st.comp));
     }
-    rc = enqueue_kernels(plan, (const uint8_t*)tab->dev.ptr, seed, RT_NOISE_PHILOX, d_clip_coef, d_skip, st.comp,
+    rc = enqueue_kernels(resident, (const uint8_t*)tab->dev.ptr + resident_off, seed, RT_NOISE_PHILOX, d_clip_coef,
+                         d_skip, st.comp);
+    if (rc != RT_OK) return rc;
+    rc = enqueue_kernels(link, (const uint8_t*)tab->dev.ptr, seed, RT_NOISE_PHILOX, d_clip_coef, d_skip, st.comp,
                          nullptr, nullptr, /*over_link=*/true);
     if (rc != RT_OK) return rc;
     if (trace)
@@ -1621,19 +1630,29 @@ static int streamed_enqueue_impl(rt_handle* h, const rt_tensor_desc* descs, uint
     if (ticket_out) *ticket_out = st.tickets_issued;  // nothing to wait for beyond what is already issued
     if (n == 0) return RT_OK;
 
-    // ---- everything on the host pinned, and (nearly) every tensor one of the fast kernels': no copies at
+    // ---- everything on the host pinned, and (nearly) every tensor of it one of the fast kernels': no copies at
     //      all.  Explicit noise stages; so do many chunks with debug outputs, of runtime-typed layouts or of
-    //      centralized rows shorter than 8 elements.
+    //      centralized rows shorter than 8 elements.  Tensors that lie on the device altogether are updated by the
+    //      kernels for those: 40 M bf16 elements take 0.11 ms, with the few workgroups that fill the link 0.75 ms.
     if (noise_mode == RT_NOISE_PHILOX) {
-        std::vector<rt_tensor_desc> mapped;
+        std::vector<rt_tensor_desc> over_link, resident;
         double up = 0, down = 0;
-        if (map_host_arrays(descs, n, mapped, up, down)) {
-            Plan plan;
-            build_image(h, mapped.data(), n, scalars, /*want_explicit=*/false, plan, h->image, /*over_link=*/true);
+        if (map_host_arrays(descs, n, over_link, resident, up, down)) {
+            Plan link, rest;
+            std::vector<uint8_t>& image = h->image;
+            build_image(h, over_link.data(), (uint32_t)over_link.size(), scalars, /*want_explicit=*/false, link, image,
+                        /*over_link=*/true);
             uint64_t n_generic = 0;
-            for (const Batch& b : plan.batches) n_generic += b.n_generic;
+            for (const Batch& b : link.batches) n_generic += b.n_generic;
             if (n_generic <= kLinkChunksMax) {
-                rc = streamed_in_place(h, plan, seed, d_clip_coef, d_skip, user, trace);
+                const size_t at = align_up(image.size(), 256);
+                if (!resident.empty()) {
+                    std::vector<uint8_t> second;
+                    build_image(h, resident.data(), (uint32_t)resident.size(), scalars, /*want_explicit=*/false, rest, second);
+                    image.resize(at + second.size());
+                    memcpy(image.data() + at, second.data(), second.size());
+                }
+                rc = streamed_in_place(h, link, rest, image, at, seed, d_clip_coef, d_skip, user, trace);
                 if (rc != RT_OK) return rc;
                 st.bytes_h2d = up;
                 st.bytes_d2h = down;

@@ -512,6 +512,47 @@ def test_pinned_arrays_are_updated_in_place(handle, layout, central, host):
     assert all(nmis(a, b) == 0 for a, b in zip(before, (getattr(s, k) for _, s in pair for k in "pmv")))
 
 
+def test_device_tensors_of_a_streamed_call_get_the_whole_chip(handle):
+    """A list with pinned host arrays and with tensors that lie on the GPU altogether: every bit as from the resident
+    step, and the device tensors run at the rate of device memory (32 workgroups, enough for the link, took
+    5.7 times as long as the resident step where a limit of 3 is asked for)."""
+    lens, n_big = [7, 512, 8197, 40_000], 40_000_003
+    sc = [F.make_scalars(step=4, **HP0)]
+    pair = []
+    for i, n in enumerate(lens):
+        vals = oracle.synth_inputs(n, 900 + i)
+        both = []
+        for where in ("cuda", "host"):
+            p, g, m, v = (dev16(x) if where == "cuda" or (i % 2 and k) else host16(x) for k, x in enumerate(vals))
+            if i == 2:
+                p, g, m, v = (dev16(x) for x in vals)    # one of the list on the GPU altogether
+            both.append(F.Entry(p=p, g=g, m=m, v=v, step=4, scalars_idx=0, tensor_id=i))
+        pair.append(both)
+    big = [torch.full((n_big,), x, dtype=torch.bfloat16, device="cuda") for x in (0.02, 1e-3, 1e-4, 1e-6)]
+    copies = [b.clone() for b in big]
+    pair.append([F.Entry(p=a[0], g=a[1], m=a[2], v=a[3], step=4, scalars_idx=0, tensor_id=9) for a in (big, copies)])
+    F.step_resident(handle, [r for r, _ in pair], sc, seed=8, explicit_noise=False)
+    F.step_streamed(handle, [s for _, s in pair], sc, seed=8, explicit_noise=False, chunk_elems=8192)
+    torch.cuda.synchronize()
+    for i, (r, s) in enumerate(pair):
+        for name in "pmv":
+            assert nmis(getattr(r, name), getattr(s, name)) == 0, (i, name)
+
+    resident, streamed = [], []
+    handle.set_timing(True)
+    for _ in range(5):
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        begin.record()
+        F.step_resident(handle, [pair[-1][0]], sc, seed=8, explicit_noise=False)
+        end.record()
+        torch.cuda.synchronize()
+        resident.append(begin.elapsed_time(end))
+        F.step_streamed(handle, [pair[-1][1]], sc, seed=8, explicit_noise=False, chunk_elems=1 << 26)
+        streamed.append(float(np.ravel(handle.streamed_timeline())[1]))
+    handle.set_timing(False)
+    assert min(streamed) < 3 * min(resident), (streamed, resident)
+
+
 def test_in_place_and_staged_calls_take_turns(handle):
     """Asynchronous calls that alternate between both ways finish in order, and a finished ticket means final
     host memory either way."""
