@@ -948,8 +948,11 @@ int rt_step_multi(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, const r
 // The gradient table of the norm pass: one NormEntry per non-empty gradient.  Chunks of 8192
 // elements are numbered in two sequences -- every whole chunk of the gradients
 // first, then the partial ones, each in tensor order -- and chunk c belongs to workgroup c mod grid.
+// kept: how many whole chunks, from the first on, make up kKeptBytes (or all there are).
 static int build_norm_table(const rt_tensor_desc* descs, uint32_t n, size_t max_entries, std::vector<NormEntry>& tab,
-                            uint64_t& n_whole, uint64_t& n_rest) {
+                            uint64_t& n_whole, uint64_t& n_rest, uint32_t& kept) {
+    uint64_t room = kKeptBytes;
+    kept = 0;
     tab.clear();
     n_whole = n_rest = 0;
     for (uint32_t i = 0; i < n; ++i) {
@@ -977,6 +980,9 @@ static int build_norm_table(const rt_tensor_desc* descs, uint32_t n, size_t max_
         tab.push_back(e);
         n_whole += whole;
         n_rest += chunks - whole;
+        const uint64_t chunk_bytes = (uint64_t)kChunkElems * dtype_size(d.g_dtype), keep = std::min(whole, room / chunk_bytes);
+        kept += (uint32_t)keep;
+        room = keep < whole ? 0 : room - keep * chunk_bytes;
         if (n_whole + n_rest > kMaxGrid) return fail(RT_EUNSUPPORTED, "too many elements in one call");
     }
     return RT_OK;
@@ -991,7 +997,8 @@ int rt_grad_norm(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, float in
     HIP_TRY(hipSetDevice(h->device));
     std::vector<NormEntry>& tab = h->norm_table;
     uint64_t n_whole = 0, n_rest = 0;
-    int rc = build_norm_table(descs, n, SIZE_MAX, tab, n_whole, n_rest);
+    uint32_t kept = 0;
+    int rc = build_norm_table(descs, n, SIZE_MAX, tab, n_whole, n_rest, kept);
     if (rc != RT_OK) return rc;
     rc = dev_reserve(h->norm_partials, kNormPartials * sizeof(double));
     if (rc != RT_OK) return rc;
@@ -1009,7 +1016,7 @@ int rt_grad_norm(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, float in
         if (rc != RT_OK) return rc;
         hipLaunchKernelGGL(grad_sumsq_table_kernel, dim3(grid), dim3(kThreads), 0, stream,
                            (const NormEntry*)slot->dev.ptr, (uint32_t)tab.size(), (uint32_t)n_whole, n_chunks,
-                           inv_loss_scale, (double*)h->norm_partials.ptr);
+                           kept, inv_loss_scale, (double*)h->norm_partials.ptr);
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipEventRecord(slot->done, stream));
         slot->in_flight = true;
@@ -1030,7 +1037,8 @@ int rt_grad_norm_static(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, f
     HIP_TRY(hipSetDevice(h->device));
     std::vector<NormEntry>& tab = h->norm_entries;  // capacity reserved by rt_create
     uint64_t n_whole = 0, n_rest = 0;
-    const int rc = build_norm_table(descs, n, kStaticMaxTensors, tab, n_whole, n_rest);
+    uint32_t kept = 0;
+    const int rc = build_norm_table(descs, n, kStaticMaxTensors, tab, n_whole, n_rest, kept);
     if (rc != RT_OK) return rc;
     double* partials = (double*)h->static_scratch;
     NormEntry* table = (NormEntry*)((uint8_t*)h->static_scratch + kStaticPartialsBytes);
@@ -1058,7 +1066,7 @@ int rt_grad_norm_static(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, f
     }
     if (n_chunks != 0) {
         hipLaunchKernelGGL(grad_sumsq_table_kernel, dim3(grid), dim3(kThreads), 0, stream, (const NormEntry*)table,
-                           (uint32_t)tab.size(), (uint32_t)n_whole, n_chunks, inv_loss_scale, partials);
+                           (uint32_t)tab.size(), (uint32_t)n_whole, n_chunks, kept, inv_loss_scale, partials);
         HIP_TRY(hipGetLastError());
     }
     hipLaunchKernelGGL(grad_norm_finish_kernel, dim3(1), dim3(kThreads), 0, stream, (const double*)partials, grid,

@@ -67,6 +67,12 @@ constexpr uint32_t kFastUnitElems = kThreads * kVec * kFastIters;
 // has drained (17.7 M elements in 160 ragged fp32 tensors: 66 + 10.5 us of kernels, 66 us with pieces).
 constexpr uint32_t kPieceElems = 64 * kVec;  // 512: one 128-bit vector per lane
 
+// How much of the gradients the passes before an update leave in the memory-side cache: the part that the update reads
+// first (see ldg128_keep).  A clipped step's norm and update over bf16 p, m and fp32 g, v, in us with 0 / 256 MB / 512 MB /
+// everything kept: 0.24 GB of gradients 248 / 226 / 225 / 225, 0.87 GB 900 / 865 / 860 / 869, 1.7 GB 1804 / 1772 / 1761 /
+// 1790, 3.5 GB 3633 / 3606 / 3591 / 3648, 7 GB 7381 / 7339 / 7311 / 7414, 32 GB 30.40 / 30.47 / 30.41 / 30.74 ms.
+constexpr uint64_t kKeptBytes = 512ull << 20;
+
 // Sets of scalars that travel as kernel arguments.  They are what changes from step to step while the tensors
 // stay where they are: as part of the table they cost a copy in front of every launch (2.5 us of host time and as much
 // on the GPU).  Four cover two param groups at two step counts; 64 bytes of arguments cost 0.04 us a launch.

@@ -62,11 +62,11 @@ typedef u32x4 u32x4_any __attribute__((aligned(2)));
 __device__ __forceinline__ u32x4 ldg128(uint64_t addr) {
     return __builtin_nontemporal_load((const RT_GLOBAL u32x4_any*)addr);
 }
-// What the next kernel reads again -- gradients, in the passes before the update -- is loaded without the hint:
-// it then stays in the 256 MB memory-side cache (with the hint it does not).  Those passes walk the
-// gradients backwards, so that what the update reads first is what they read last.  A clipped step of 122 M fp32
-// elements (489 MB of gradients) takes 451 us with the hint in the norm pass and 417 us without; 218 M with
-// bf16 gradients 616 and 577 us, with fp32 gradients (872 MB) 917 and 886 us.  Walking backwards with the hint: no change.
+// What the next kernel reads again -- gradients, in the passes before the update -- is loaded without the hint where
+// it can still lie in the 256 MB memory-side cache by then (with the hint it does not).  Those passes walk the
+// gradients backwards, so that what the update reads first is what they read last.  Without the hint a pass itself is
+// slower, whatever else it does (the norm of 0.87 GB 184 us against 130, of 32 GB 5.2 ms against 4.6), so only
+// the part that it reads last, kKeptBytes of it, goes without.
 __device__ __forceinline__ u32x4 ldg128_keep(uint64_t addr) { return *(const RT_GLOBAL u32x4_any*)addr; }
 __device__ __forceinline__ void stg128(uint64_t addr, u32x4 v) {
     __builtin_nontemporal_store(v, (RT_GLOBAL u32x4_any*)addr);
@@ -1371,13 +1371,16 @@ __device__ __forceinline__ float block_sum(float x, float* lds) {
 // Whole chunk: every load is 16 bytes per lane and contiguous across the
 // wave whatever the element type (a sum does not care which lane gets which element), all loads
 // of the chunk are in flight together.
-template <int GDT>
+template <int GDT, bool KEEP>
 __device__ __forceinline__ float chunk_sumsq_full(uint64_t g_addr, uint32_t chunk, float inv_loss_scale) {
     constexpr int kLoads = (int)(kChunkElems * esize<GDT>() / 16 / kThreads);  // 4 (16-bit) or 8 (fp32)
     const uint64_t base = g_addr + (uint64_t)chunk * kChunkElems * esize<GDT>() + (uint64_t)threadIdx.x * 16;
     u32x4 r[kLoads];
 #pragma unroll
-    for (int k = 0; k < kLoads; ++k) r[k] = ldg128_keep(base + (uint64_t)k * (kThreads * 16));
+    for (int k = 0; k < kLoads; ++k) {
+        if constexpr (KEEP) r[k] = ldg128_keep(base + (uint64_t)k * (kThreads * 16));
+        else r[k] = ldg128(base + (uint64_t)k * (kThreads * 16));
+    }
     float acc = 0.0f;
 #pragma unroll
     for (int k = 0; k < kLoads; ++k) {
@@ -1403,10 +1406,10 @@ __device__ __forceinline__ float chunk_sumsq_full(uint64_t g_addr, uint32_t chun
     return acc;
 }
 
-template <int GDT>
+template <int GDT, bool KEEP>
 __device__ __forceinline__ float chunk_sumsq(uint64_t g_addr, uint64_t n, uint32_t chunk, float inv_loss_scale) {
     const uint64_t chunk_base = (uint64_t)chunk * kChunkElems;
-    if (chunk_base + kChunkElems <= n) return chunk_sumsq_full<GDT>(g_addr, chunk, inv_loss_scale);
+    if (chunk_base + kChunkElems <= n) return chunk_sumsq_full<GDT, KEEP>(g_addr, chunk, inv_loss_scale);
     float acc = 0.0f;
 #pragma unroll 1
     for (int it = 0; it < kItersPerChunk; ++it) {
@@ -1425,11 +1428,12 @@ __device__ __forceinline__ float chunk_sumsq(uint64_t g_addr, uint64_t n, uint32
     return acc;
 }
 
+template <bool KEEP>
 __device__ __forceinline__ float chunk_sumsq_dt(int dt, uint64_t g_addr, uint64_t n, uint32_t chunk,
                                                 float inv_loss_scale) {
-    if (dt == RT_DT_BF16) return chunk_sumsq<RT_DT_BF16>(g_addr, n, chunk, inv_loss_scale);
-    if (dt == RT_DT_F32) return chunk_sumsq<RT_DT_F32>(g_addr, n, chunk, inv_loss_scale);
-    return chunk_sumsq<RT_DT_F16>(g_addr, n, chunk, inv_loss_scale);
+    if (dt == RT_DT_BF16) return chunk_sumsq<RT_DT_BF16, KEEP>(g_addr, n, chunk, inv_loss_scale);
+    if (dt == RT_DT_F32) return chunk_sumsq<RT_DT_F32, KEEP>(g_addr, n, chunk, inv_loss_scale);
+    return chunk_sumsq<RT_DT_F16, KEEP>(g_addr, n, chunk, inv_loss_scale);
 }
 
 // ---------------------------------------------------------------------------
@@ -1443,6 +1447,7 @@ __device__ __forceinline__ float chunk_sumsq_dt(int dt, uint64_t g_addr, uint64_
 // A lane keeps its sum in fp64 from chunk to chunk and the workgroup reduces once, at the end, so that the
 // four waves never wait for each other between chunks.  17.7 M fp32 elements in 160 ragged gradients
 // 16.6 -> 15.2 us, 218 M in nine 144.6 -> 141.7 us, against a binary search and a reduction with two barriers per chunk.
+// Bound by memory: 6.4 - 6.9 TB/s beyond the caches.
 // ---------------------------------------------------------------------------
 struct alignas(16) NormEntry {
     uint64_t g;
@@ -1466,24 +1471,32 @@ __global__ __launch_bounds__(kNormEntriesPerWrite) void norm_table_write_kernel(
     if (threadIdx.x < count) table[first + threadIdx.x] = slice.e[threadIdx.x];
 }
 
+template <bool KEEP>
+__device__ __forceinline__ double table_chunk_sumsq(const NormEntry* __restrict__ table, uint32_t n, uint32_t total_whole,
+                                                    uint32_t c, float inv_loss_scale) {
+    constexpr uint32_t kStep = sizeof(NormEntry) / 4;
+    const bool whole = c < total_whole;
+    const uint32_t key = whole ? c : c - total_whole;
+    // the last entry whose first chunk number in this sequence is <= key is the one with chunks: entries
+    // without any share their number with the entry behind them
+    const uint32_t at = find_range<kStep>(whole ? &table->first_whole : &table->first_rest, n, key);
+    const NormEntry e = table[__builtin_amdgcn_readfirstlane(at)];
+    const uint32_t chunk = whole ? key - e.first_whole : e.n_whole + (key - e.first_rest);
+    return (double)chunk_sumsq_dt<KEEP>((int)e.dtype, e.g, e.numel, chunk, inv_loss_scale);
+}
+
 __global__ __launch_bounds__(kThreads) void grad_sumsq_table_kernel(const NormEntry* __restrict__ table, uint32_t n,
                                                                     uint32_t total_whole, uint32_t n_chunks,
-                                                                    float inv_loss_scale,
+                                                                    uint32_t kept, float inv_loss_scale,
                                                                     double* __restrict__ partials) {
-    constexpr uint32_t kStep = sizeof(NormEntry) / 4;
     double total = 0.0;
-    // backwards, see ldg128_keep
-    for (uint32_t left = (n_chunks - blockIdx.x + gridDim.x - 1u) / gridDim.x; left-- > 0u;) {
-        const uint32_t c = blockIdx.x + left * gridDim.x;
-        const bool whole = c < total_whole;
-        const uint32_t key = whole ? c : c - total_whole;
-        // the last entry whose first chunk number in this sequence is <= key is the one with chunks: entries
-        // without any share their number with the entry behind them
-        const uint32_t at = find_range<kStep>(whole ? &table->first_whole : &table->first_rest, n, key);
-        const NormEntry e = table[__builtin_amdgcn_readfirstlane(at)];
-        const uint32_t chunk = whole ? key - e.first_whole : e.n_whole + (key - e.first_rest);
-        total += (double)chunk_sumsq_dt((int)e.dtype, e.g, e.numel, chunk, inv_loss_scale);
-    }
+    // Backwards, and the first `kept` chunks (kKeptBytes) without the hint, see ldg128_keep.  Two loops: of one whose
+    // loads choose between the two the compiler makes loads without.
+    uint32_t left = (n_chunks - blockIdx.x + gridDim.x - 1u) / gridDim.x;
+    while (left > 0u && blockIdx.x + (left - 1u) * gridDim.x >= kept)
+        total += table_chunk_sumsq<false>(table, n, total_whole, blockIdx.x + --left * gridDim.x, inv_loss_scale);
+    while (left > 0u)
+        total += table_chunk_sumsq<true>(table, n, total_whole, blockIdx.x + --left * gridDim.x, inv_loss_scale);
     __shared__ double lds[kThreads / 64];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off, 64);

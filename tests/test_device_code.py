@@ -79,3 +79,12 @@ def test_update_kernels_keep_their_occupancy(device_asm):
         assert m, "kernel metadata not found"
         print("row-wise", short, "vgpr_count", m.group(2))
         assert int(m.group(2)) <= limit, m.group(2)
+
+
+def test_norm_kernel_loads_most_gradients_with_the_nontemporal_hint(device_asm):
+    """Whole chunks are loaded with the hint and, in the part that the update reads first, without: 8 loads for fp32
+    and 4 for each 16-bit type either way.  (From one loop that chose between the two the compiler made loads without.)"""
+    body = re.search(r"^_ZN2rt23grad_sumsq_table_kernel\w+:.*?$(.*?)^\s+s_endpgm", device_asm, flags=re.M | re.S)
+    assert body, "kernel not found"
+    loads = re.findall(r"^\s+global_load_dwordx4 .*$", body.group(1), flags=re.M)
+    assert sum(" nt" in x for x in loads) >= 16 and sum(" nt" not in x for x in loads) >= 16, loads

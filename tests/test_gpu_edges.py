@@ -175,3 +175,19 @@ def test_norm_pass_finds_every_gradient(handle, n):
     want = float(torch.cat([g.float() for g in grads]).double().square().sum()) ** 0.5
     out = F.grad_norm(handle, grads, inv_loss_scale=1.0, max_norm=1.0)
     assert float(out[0]) == pytest.approx(want, rel=32 * 2 ** -24)
+
+
+@pytest.mark.parametrize("sizes", [(100_000_003, 70_000_000, 8192 * 3 + 5, 30_000_001),   # the cut inside the second
+                                   (134_217_728, 8192, 4097), (134_225_920, 20_000, 9)])   # at the first one's end, and one chunk before it
+def test_norm_pass_over_more_than_stays_in_the_cache(handle, sizes):
+    """Gradients on both sides of the 512 MiB that are loaded to stay, fp32 and 16 bit: each chunk counts once, whichever
+    loop takes it.  fp32 sums of at most 32 squares a lane and chunk, in fp64 from chunk to chunk."""
+    gen, want, grads = torch.Generator(device="cuda").manual_seed(sizes[1]), 0.0, []
+    for k, n in enumerate(sizes):
+        g = torch.empty(n, dtype=[torch.float32, torch.bfloat16, torch.float16, torch.float32][k], device="cuda")
+        g.normal_(0, 10.0 ** -k, generator=gen)
+        grads.append(g)
+        want += sum(float(x.double().square().sum()) for x in g.split(1 << 24))
+    for _ in range(2):
+        out = F.grad_norm(handle, grads, inv_loss_scale=1.0, max_norm=1.0)
+        assert float(out[0]) == pytest.approx(want ** 0.5, rel=32 * 2 ** -24)
