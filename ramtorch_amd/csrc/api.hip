@@ -1086,13 +1086,14 @@ int rt_row_means(rt_handle* h, const void* g, int g_dtype, uint64_t rows, uint64
     if ((uintptr_t)g % dtype_size(g_dtype)) return fail(RT_EINVAL, "gradient pointer not aligned to its element size");
     hipStream_t stream = (hipStream_t)stream_;
     HIP_TRY(hipSetDevice(h->device));
+    const uint64_t kept = kKeptBytes / dtype_size(g_dtype) / row_len;
     if (row_len <= kWaveRowMax) {
         const uint32_t grid = (uint32_t)((rows + kThreads / 64 - 1) / (kThreads / 64));
         hipLaunchKernelGGL(row_mean_kernel, dim3(grid), dim3(kThreads), 0, stream, (uint64_t)g, (uint32_t)g_dtype, rows,
-                           (uint32_t)row_len, inv_loss_scale, d_row_mean);
+                           (uint32_t)row_len, kept, inv_loss_scale, d_row_mean);
     } else {
         hipLaunchKernelGGL(row_mean_long_kernel, dim3((uint32_t)rows), dim3(kThreads), 0, stream, (uint64_t)g,
-                           (uint32_t)g_dtype, row_len, inv_loss_scale, d_row_mean);
+                           (uint32_t)g_dtype, row_len, kept, inv_loss_scale, d_row_mean);
     }
     HIP_TRY(hipGetLastError());
     return RT_OK;
@@ -1107,7 +1108,8 @@ int rt_row_means_multi(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, fl
     std::vector<RowMeanEntry>& tab = h->rowmean_table;
     tab.clear();
     std::vector<RowMeanEntry> long_tab;
-    uint64_t rows_short = 0, rows_long = 0;
+    uint64_t rows_short = 0, rows_long = 0, room = kKeptBytes;
+    uint32_t kept_short = 0, kept_long = 0;   // rows, from the first on, that make up kKeptBytes (or all there are)
     for (uint32_t i = 0; i < n; ++i) {
         const rt_tensor_desc& d = descs[i];
         if (d.numel == 0 || !d.row_mean) continue;
@@ -1129,6 +1131,9 @@ int rt_row_means_multi(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, fl
         e.rows = (uint32_t)(d.numel / d.row_len);
         e.pad[0] = e.pad[1] = e.pad[2] = 0;
         (is_long ? long_tab : tab).push_back(e);
+        const uint64_t es = dtype_size(d.g_dtype), keep = std::min<uint64_t>(e.rows, room / es / d.row_len);
+        (is_long ? kept_long : kept_short) += (uint32_t)keep;
+        room = keep < e.rows ? 0 : room - keep * d.row_len * es;
         rows += d.numel / d.row_len;
         if (rows > kMaxGrid) return fail(RT_EUNSUPPORTED, "more than %llu rows in one call", (unsigned long long)kMaxGrid);
     }
@@ -1154,13 +1159,14 @@ int rt_row_means_multi(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, fl
     if (rows_short) {
         const uint32_t grid = (uint32_t)((rows_short + kThreads / 64 - 1) / (kThreads / 64));
         hipLaunchKernelGGL(row_mean_table_kernel, dim3(grid), dim3(kThreads), 0, stream, (const uint32_t*)dev,
-                           (const RowMeanEntry*)(dev + off_rec_s), (uint32_t)ns, (uint32_t)rows_short, inv_loss_scale);
+                           (const RowMeanEntry*)(dev + off_rec_s), (uint32_t)ns, (uint32_t)rows_short, kept_short,
+                           inv_loss_scale);
         HIP_TRY(hipGetLastError());
     }
     if (rows_long) {
         hipLaunchKernelGGL(row_mean_table_long_kernel, dim3((uint32_t)rows_long), dim3(kThreads), 0, stream,
                            (const uint32_t*)(dev + off_first_l), (const RowMeanEntry*)(dev + off_rec_l), (uint32_t)nl,
-                           inv_loss_scale);
+                           kept_long, inv_loss_scale);
         HIP_TRY(hipGetLastError());
     }
     HIP_TRY(hipEventRecord(slot->done, stream));

@@ -1565,10 +1565,12 @@ __device__ __forceinline__ float load_elem(uint64_t base, uint64_t idx) {
 // Sum of row [base, base + row_len) of g by the calling wavefront; the result is in every lane.
 // A row moves as whole vectors, 32 registers of them in flight per lane, and at most 7 single
 // elements at its end.
-// The row is read again, by the update behind this pass or right away by the update that takes its own row
-// means: its lines are loaded the ordinary way and stay in the caches.
-template <int DT>
-__device__ __forceinline__ Raw8<DT> load_raw_cached(uint64_t base, uint64_t i) {
+// KEEP: the row is read again, by the update behind this pass (see ldg128_keep) or right away by the update that takes
+// its own row means: its lines are loaded the ordinary way and stay in the caches.  fp32 rows are always loaded so: a
+// lane's two accesses share a line.
+template <int DT, bool KEEP>
+__device__ __forceinline__ Raw8<DT> load_raw_row(uint64_t base, uint64_t i) {
+    if constexpr (!KEEP && DT != RT_DT_F32) return load_raw<DT>(base, i);
     Raw8<DT> r;
     const uint64_t addr = base + i * esize<DT>();
     r.a = ldg128_keep(addr);
@@ -1576,7 +1578,7 @@ __device__ __forceinline__ Raw8<DT> load_raw_cached(uint64_t base, uint64_t i) {
     return r;
 }
 
-template <int GDT>
+template <int GDT, bool KEEP>
 __device__ __forceinline__ float row_sum_wave(uint64_t g, uint64_t base, uint32_t row_len, float inv_loss_scale) {
     constexpr int kB = GDT == RT_DT_F32 ? kRowVecs / 2 : kRowVecs;   // an fp32 vector of 8 elements is two loads
     const uint32_t lane = threadIdx.x & 63u;
@@ -1587,7 +1589,7 @@ __device__ __forceinline__ float row_sum_wave(uint64_t g, uint64_t base, uint32_
 #pragma unroll
         for (int k = 0; k < kB; ++k) {
             const uint32_t v = v0 + (uint32_t)k * 64u + lane;
-            if (v < n_vec) r[k] = load_raw_cached<GDT>(g, base + (uint64_t)v * kVec);
+            if (v < n_vec) r[k] = load_raw_row<GDT, KEEP>(g, base + (uint64_t)v * kVec);
         }
 #pragma unroll
         for (int k = 0; k < kB; ++k) {
@@ -1601,7 +1603,7 @@ __device__ __forceinline__ float row_sum_wave(uint64_t g, uint64_t base, uint32_
 }
 
 // Sum of one (long) row by the calling workgroup; valid in thread 0.
-template <int GDT>
+template <int GDT, bool KEEP>
 __device__ __forceinline__ float row_sum_block(uint64_t g, uint64_t base, uint64_t row_len, float inv_loss_scale,
                                                float* lds) {
     constexpr int kInFlight = 4;
@@ -1612,7 +1614,7 @@ __device__ __forceinline__ float row_sum_block(uint64_t g, uint64_t base, uint64
         for (int k = 0; k < kInFlight; ++k) {
             const uint64_t e = c0 + ((uint64_t)k * kThreads + threadIdx.x) * kVec;
             if (e < row_len)
-                r[k] = (e + kVec <= row_len) ? load_raw_cached<GDT>(g, base + e)
+                r[k] = (e + kVec <= row_len) ? load_raw_row<GDT, KEEP>(g, base + e)
                                              : load_raw_guarded<GDT>(g, base + e, base + row_len);
         }
 #pragma unroll
@@ -1624,33 +1626,50 @@ __device__ __forceinline__ float row_sum_block(uint64_t g, uint64_t base, uint64
     return block_sum(acc, lds);
 }
 
+template <bool KEEP>
 __device__ __forceinline__ float row_sum_wave_dt(uint32_t dt, uint64_t g, uint64_t base, uint32_t row_len, float inv) {
-    if (dt == RT_DT_BF16) return row_sum_wave<RT_DT_BF16>(g, base, row_len, inv);
-    if (dt == RT_DT_F32) return row_sum_wave<RT_DT_F32>(g, base, row_len, inv);
-    return row_sum_wave<RT_DT_F16>(g, base, row_len, inv);
+    if (dt == RT_DT_BF16) return row_sum_wave<RT_DT_BF16, KEEP>(g, base, row_len, inv);
+    if (dt == RT_DT_F32) return row_sum_wave<RT_DT_F32, KEEP>(g, base, row_len, inv);
+    return row_sum_wave<RT_DT_F16, KEEP>(g, base, row_len, inv);
 }
+template <bool KEEP>
 __device__ __forceinline__ float row_sum_block_dt(uint32_t dt, uint64_t g, uint64_t base, uint64_t row_len, float inv,
                                                   float* lds) {
-    if (dt == RT_DT_BF16) return row_sum_block<RT_DT_BF16>(g, base, row_len, inv, lds);
-    if (dt == RT_DT_F32) return row_sum_block<RT_DT_F32>(g, base, row_len, inv, lds);
-    return row_sum_block<RT_DT_F16>(g, base, row_len, inv, lds);
+    if (dt == RT_DT_BF16) return row_sum_block<RT_DT_BF16, KEEP>(g, base, row_len, inv, lds);
+    if (dt == RT_DT_F32) return row_sum_block<RT_DT_F32, KEEP>(g, base, row_len, inv, lds);
+    return row_sum_block<RT_DT_F16, KEEP>(g, base, row_len, inv, lds);
 }
 
-// One gradient.  Rows of at most kWaveRowMax elements: workgroup b takes rows 4b .. 4b+3, one per wave.
+// Row sums of a pass over whole gradients, by a wavefront and by a workgroup per row.  keep: the row is
+// among the ones that the pass reads last and the update first.
+__device__ __forceinline__ float pass_row_sum_wave(bool keep, uint32_t dt, uint64_t g, uint64_t base, uint32_t row_len,
+                                                   float inv) {
+    if (keep) return row_sum_wave_dt<true>(dt, g, base, row_len, inv);
+    return row_sum_wave_dt<false>(dt, g, base, row_len, inv);
+}
+__device__ __forceinline__ float pass_row_sum_block(bool keep, uint32_t dt, uint64_t g, uint64_t base, uint64_t row_len,
+                                                    float inv, float* lds) {
+    if (keep) return row_sum_block_dt<true>(dt, g, base, row_len, inv, lds);
+    return row_sum_block_dt<false>(dt, g, base, row_len, inv, lds);
+}
+
+// One gradient.  Rows of at most kWaveRowMax elements: workgroup b takes the four rows that end 4b rows before the
+// last, one per wave (backwards, and the first `kept` rows to stay in the cache, see ldg128_keep).
 __global__ __launch_bounds__(kThreads) void row_mean_kernel(uint64_t g, uint32_t dtype, uint64_t rows, uint32_t row_len,
-                                                            float inv_loss_scale, float* __restrict__ out) {
+                                                            uint64_t kept, float inv_loss_scale, float* __restrict__ out) {
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const uint64_t row = (uint64_t)blockIdx.x * (kThreads / 64) + wave;
+    uint64_t row = (uint64_t)blockIdx.x * (kThreads / 64) + wave;
     if (row >= rows) return;
-    const float sum = row_sum_wave_dt(dtype, g, row * row_len, row_len, inv_loss_scale);
+    row = rows - 1u - row;
+    const float sum = pass_row_sum_wave(row < kept, dtype, g, row * row_len, row_len, inv_loss_scale);
     if ((threadIdx.x & 63u) == 0) out[row] = sum / (float)row_len;
 }
 // Longer rows: one workgroup per row.
 __global__ __launch_bounds__(kThreads) void row_mean_long_kernel(uint64_t g, uint32_t dtype, uint64_t row_len,
-                                                                 float inv_loss_scale, float* __restrict__ out) {
+                                                                 uint64_t kept, float inv_loss_scale, float* __restrict__ out) {
     __shared__ float lds[kThreads / 64];
-    const uint64_t row = blockIdx.x;
-    const float sum = row_sum_block_dt(dtype, g, row * row_len, row_len, inv_loss_scale, lds);
+    const uint64_t row = gridDim.x - 1u - blockIdx.x;
+    const float sum = pass_row_sum_block(row < kept, dtype, g, row * row_len, row_len, inv_loss_scale, lds);
     if (threadIdx.x == 0) out[row] = sum / (float)row_len;
 }
 
@@ -1672,7 +1691,8 @@ static_assert(sizeof(RowMeanEntry) == 48, "RowMeanEntry layout");
 // then has nothing in flight while it reduces a row.)
 __global__ __launch_bounds__(kThreads) void row_mean_table_kernel(const uint32_t* __restrict__ first,
                                                                   const RowMeanEntry* __restrict__ table, uint32_t n,
-                                                                  uint32_t rows_total, float inv_loss_scale) {
+                                                                  uint32_t rows_total, uint32_t kept,
+                                                                  float inv_loss_scale) {
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     uint32_t row = blockIdx.x * (kThreads / 64) + wave;
     if (row >= rows_total) return;
@@ -1680,19 +1700,19 @@ __global__ __launch_bounds__(kThreads) void row_mean_table_kernel(const uint32_t
     const uint32_t idx = find_range(first, n, row);   // each wave searches on its own
     const RowMeanEntry e = load_const(&table[idx]);
     const uint64_t r = row - e.first_row;
-    const float sum = row_sum_wave_dt(e.dtype, e.g, r * e.row_len, (uint32_t)e.row_len, inv_loss_scale);
+    const float sum = pass_row_sum_wave(row < kept, e.dtype, e.g, r * e.row_len, (uint32_t)e.row_len, inv_loss_scale);
     if ((threadIdx.x & 63u) == 0) ((RT_GLOBAL float*)e.out)[r] = sum / (float)e.row_len;
 }
 
 __global__ __launch_bounds__(kThreads) void row_mean_table_long_kernel(const uint32_t* __restrict__ first,
                                                                        const RowMeanEntry* __restrict__ table, uint32_t n,
-                                                                       float inv_loss_scale) {
+                                                                       uint32_t kept, float inv_loss_scale) {
     __shared__ float lds[kThreads / 64];
     const uint32_t row = gridDim.x - 1u - blockIdx.x;   // backwards as well
     const uint32_t idx = find_range(first, n, row);
     const RowMeanEntry e = load_const(&table[idx]);
     const uint64_t r = row - e.first_row;
-    const float sum = row_sum_block_dt(e.dtype, e.g, r * e.row_len, e.row_len, inv_loss_scale, lds);
+    const float sum = pass_row_sum_block(row < kept, e.dtype, e.g, r * e.row_len, e.row_len, inv_loss_scale, lds);
     if (threadIdx.x == 0) ((RT_GLOBAL float*)e.out)[r] = sum / (float)e.row_len;
 }
 
@@ -1797,7 +1817,7 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_rowwise_kernel(const Launch
     }
     // (sixteen vectors per lane on the way at once instead of eight -- a lane adds its vectors in ascending
     // order whatever the batch, so no bit changes -- measured the same time on the 8B set)
-    const float sum = row_sum_wave<GDT>(tg, e0, row_len, c.s.inv_loss_scale);
+    const float sum = row_sum_wave<GDT, true>(tg, e0, row_len, c.s.inv_loss_scale);
     const float mc = cen_term(sum / (float)row_len, c.s, c.do_clip, c.coef);
 
     struct In {

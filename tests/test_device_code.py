@@ -81,10 +81,15 @@ def test_update_kernels_keep_their_occupancy(device_asm):
         assert int(m.group(2)) <= limit, m.group(2)
 
 
-def test_norm_kernel_loads_most_gradients_with_the_nontemporal_hint(device_asm):
-    """Whole chunks are loaded with the hint and, in the part that the update reads first, without: 8 loads for fp32
-    and 4 for each 16-bit type either way.  (From one loop that chose between the two the compiler made loads without.)"""
-    body = re.search(r"^_ZN2rt23grad_sumsq_table_kernel\w+:.*?$(.*?)^\s+s_endpgm", device_asm, flags=re.M | re.S)
+@pytest.mark.parametrize("kernel,hinted,plain", [("grad_sumsq_table_kernel", 16, 16), ("row_mean_table_kernel", 16, 16),
+                                                 ("row_mean_table_long_kernel", 8, 8), ("row_mean_kernel", 16, 16),
+                                                 ("row_mean_long_kernel", 8, 8)])
+def test_gradient_passes_load_with_and_without_the_nontemporal_hint(device_asm, kernel, hinted, plain):
+    """The passes in front of an update load gradients with the hint, and without it in the part that the update reads
+    first: for a whole chunk 8 loads of fp32 and 4 of each 16-bit type, for a row 8 (a workgroup's: 4) of each 16-bit type.
+    (Where code chose between the two loads one by one, the compiler made loads without the hint of both.)"""
+    body = re.search(rf"^_ZN2rt{len(kernel)}{kernel}E\w+:.*?$(.*?)^\s+\.section", device_asm, flags=re.M | re.S)
     assert body, "kernel not found"
     loads = re.findall(r"^\s+global_load_dwordx4 .*$", body.group(1), flags=re.M)
-    assert sum(" nt" in x for x in loads) >= 16 and sum(" nt" not in x for x in loads) >= 16, loads
+    nt = sum(" nt" in x for x in loads)
+    assert nt >= hinted and len(loads) - nt >= plain, (nt, len(loads))

@@ -191,3 +191,25 @@ def test_norm_pass_over_more_than_stays_in_the_cache(handle, sizes):
     for _ in range(2):
         out = F.grad_norm(handle, grads, inv_loss_scale=1.0, max_norm=1.0)
         assert float(out[0]) == pytest.approx(want ** 0.5, rel=32 * 2 ** -24)
+
+
+def test_row_means_over_more_than_stays_in_the_cache(handle):
+    """Rows on both sides of the 512 MiB that are loaded to stay, of a wavefront and of a workgroup, many gradients in
+    one launch and one on its own.  A lane adds at most row / 64 elements and the lanes' sums in six steps more."""
+    gen, jobs = torch.Generator(device="cuda").manual_seed(2), []
+    for k, (rows, row, dt) in enumerate([(2001, 33_000, torch.bfloat16), (50_000, 4096, torch.bfloat16), (3, 40_001, torch.float16),
+                                         (9000, 4097, torch.float32), (1111, 77, torch.float16), (3000, 33_001, torch.bfloat16)]):
+        g = torch.empty(rows, row, dtype=dt, device="cuda").normal_(0, 1, generator=gen)
+        jobs.append((F.Entry(p=None, g=g, m=None, v=None, step=1, scalars_idx=0, tensor_id=k), rows, row))
+    F.row_means_multi(handle, jobs, 0.5)
+    assert sum(e.g.numel() * e.g.element_size() for e, *_ in jobs) > 640 << 20
+    single = torch.empty(70_001, 4096, dtype=torch.bfloat16, device="cuda").normal_(0, 1, generator=gen)
+    checks = [(e.g, e.row_mean, row) for e, rows, row in jobs]
+    checks += [(single, F.row_means(handle, single, 70_001, 4096, 0.5), 4096)]
+    long = single.view(-1)[:8000 * 35_001].view(8000, 35_001)
+    checks += [(long, F.row_means(handle, long, 8000, 35_001, 0.5), 35_001)]
+    for g, mean, row in checks:
+        for lo in range(0, len(g), 1024):
+            x = g[lo:lo + 1024].double() * 0.5
+            bound = (row / 64 + 8) * 2 ** -24 * x.abs().mean(1)
+            assert bool(((mean[lo:lo + 1024].double() - x.mean(1)).abs() <= bound).all()), (row, lo)
