@@ -213,3 +213,34 @@ def test_row_means_over_more_than_stays_in_the_cache(handle):
             x = g[lo:lo + 1024].double() * 0.5
             bound = (row / 64 + 8) * 2 ** -24 * x.abs().mean(1)
             assert bool(((mean[lo:lo + 1024].double() - x.mean(1)).abs() <= bound).all()), (row, lo)
+
+
+@pytest.mark.parametrize("mix", ["bf16", "f16", "f16_bf16states"])
+@pytest.mark.parametrize("shifts", [(0, 1, 0, 0), (3, 7, 5, 1), (4, 4, 4, 4)])
+def test_rows_summed_inside_the_update_may_begin_at_any_element(handle, mix, shifts):
+    """The row-wise kernel on views that begin at an element of their own, both instances (rows of up to 4096 elements
+    and longer ones) and the limits of its row lengths: the bits of the same update with row means given, over arrays that
+    begin at a 512-byte boundary, and nothing outside the arrays changes."""
+    codes = {**_MIX, "f16_bf16states": (2, 2, 0, 0)}[mix]
+    entries, reference, wholes = [], [], []
+    for k, (rows, row) in enumerate([(5, 512), (9, 520), (3, 4096), (6, 4104), (2, 14336), (1, 32768)]):
+        n = rows * row
+        arrays = oracle.synth_inputs(n, 600 + k)
+        arrays = [a if c == 0 else oracle.bf16_to_f32(a).astype(np.float16).view(np.uint16) for a, c in zip(arrays, codes)]
+        views = [guarded(a, c, s) for a, c, s in zip(arrays, codes, shifts)]
+        plain = [guarded(a, c, 0)[0] for a, c in zip(arrays, codes)]
+        wholes += [(w, s, n) for (_, w), s in zip(views, shifts)]
+        e = F.Entry(p=views[0][0], g=views[1][0], m=views[2][0], v=views[3][0], step=10, scalars_idx=0, tensor_id=k)
+        assert F.rowwise_ok(e, row)
+        e.row_len = row
+        entries.append(e)
+        reference.append(F.Entry(p=plain[0], g=plain[1], m=plain[2], v=plain[3], step=10, scalars_idx=0, tensor_id=k,
+                                 row_mean=F.row_means(handle, plain[1], rows, row), row_len=row))
+    for lst in (entries, reference):
+        F.step_resident(handle, lst, [F.make_scalars(step=10, centralization=0.7, **HP0)], seed=77, explicit_noise=False)
+    torch.cuda.synchronize()
+    for e, r in zip(entries, reference):
+        for name in "pgmv":
+            np.testing.assert_array_equal(bits(getattr(e, name)), bits(getattr(r, name)), err_msg=f"rows of {e.row_len} {name}")
+    for whole, s, n in wholes:
+        check_guards(whole, s, n)

@@ -2,6 +2,8 @@
 chunked H2D -> update -> D2H.  Results must be bit-identical to the resident
 path and to the oracle, whatever the chunk size.  Run with ``-m gpu``.
 """
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -555,7 +557,8 @@ def test_device_tensors_of_a_streamed_call_get_the_whole_chip(handle):
 
 def test_in_place_and_staged_calls_take_turns(handle):
     """Asynchronous calls that alternate between both ways finish in order, and a finished ticket means final
-    host memory either way."""
+    host memory either way.  (Here an array that is not pinned sends a call through the staging buffers, and such a call
+    first waits until everything before it is done.)"""
     n, state = 700_001, []
     for i in range(6):
         p, g, m, v = oracle.synth_inputs(n, 800 + i)
@@ -569,6 +572,38 @@ def test_in_place_and_staged_calls_take_turns(handle):
     assert handle.streamed_completed() == tickets[-1]
     for i, (p, g, m, v, e) in enumerate(state):
         oracle.step_tensor(p, g, m, v, oracle.scalars_from_hparams(step=2, **HP0), seed=6, step=2, tensor_id=i)
+        for name, t, a in zip("pmv", (e.p, e.m, e.v), (p, m, v)):
+            np.testing.assert_array_equal(bits16(t), a, err_msg=f"{i} {name}")
+
+
+@pytest.mark.parametrize("first", [0, 1])
+def test_staged_and_in_place_calls_are_in_flight_together(handle, first):
+    """Asynchronous calls, all arrays pinned, in turn updated in place and (explicit noise) moved through the staging
+    buffers in a dozen chunks queued up front: none of them waits on the host for the one before, so both
+    kinds share the streams.  Tickets complete in order, and a finished ticket means final host memory."""
+    n, step, calls = 700_001, 2, []
+    for i in range(8):
+        arrays, staged = oracle.synth_inputs(n, 900 + i), (i + first) % 2 == 1
+        noise = oracle.synth_noise(n, 900 + i) if staged else None
+        p, g, m, v = arrays
+        e = F.Entry(p=host16(p), g=dev16(g) if i % 3 else host16(g), m=host16(m), v=host16(v), step=step, scalars_idx=0, tensor_id=i,
+                    noise=None if noise is None else tuple(torch.from_numpy(z.view(np.int16).copy()).cuda() for z in noise))
+        calls.append((arrays, noise, e))
+    sc, sco = [F.make_scalars(step=step, **HP0)], oracle.scalars_from_hparams(step=step, **HP0)
+    torch.cuda.synchronize()
+    tickets = [F.step_streamed(handle, [e], sc, seed=6, explicit_noise=noise is not None, chunk_elems=65_536, wait=False)
+               for _, noise, e in calls]
+    assert tickets == list(range(tickets[0], tickets[0] + 8))
+    done, deadline = 0, time.monotonic() + 20
+    while done < tickets[-1] and time.monotonic() < deadline:
+        now = handle.streamed_completed()
+        assert now >= done
+        if now == done:
+            time.sleep(1e-4)
+        done = now
+    handle.streamed_wait()
+    for i, ((p, g, m, v), noise, e) in enumerate(calls):
+        oracle.step_tensor(p, g, m, v, sco, noise=noise, seed=6, step=step, tensor_id=i)
         for name, t, a in zip("pmv", (e.p, e.m, e.v), (p, m, v)):
             np.testing.assert_array_equal(bits16(t), a, err_msg=f"{i} {name}")
 
