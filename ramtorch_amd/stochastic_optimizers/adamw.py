@@ -167,11 +167,14 @@ class AdamW(Optimizer):
         self.noise_source = noise_source
         self.last_grad_norm: Optional[torch.Tensor] = None  # [norm, clip_coef, found_inf bits, -] on the GPU
         self._skip_check = None           # per device of the last step with max_grad_norm: (event, host copy of the
-                                          # norm record, [(state, step count before)]) -- see _settle_skipped_step
+                                          # norm record, the step counts it advanced) -- see _settle_skipped_step
         self.last_step_skipped = False    # as of the last _settle_skipped_step()
         self.fuse_in_backward = True      # the hook of make_post_accumulate_hook() is live
         self.host_arrays_ordered = False  # step_param: uploads from pinned host p / m / v wait for the current stream
-        self.fuse_row_means = True        # centralization: matrices whose rows fit a wavefront are summed inside the update
+        # Centralization: matrices whose rows fit a wavefront are summed inside the update, whatever their sizes.  In us a step,
+        # inside against a pass before: convolutions of 11.5 / 27.6 M elements 63 / 118 against 48 / 85, transformer layers of
+        # 3.4 / 54 / 218 M 30 / 147 / 569 against 44 / 142 / 554, 8 G elements 18.0 against 20.2 ms.
+        self.fuse_row_means = True
         self.max_inflight_bytes = 2 << 30  # gradients kept alive for updates still in flight (step_param)
         self.max_inflight_calls = 2       # staging chunks handed to the copy pipeline and not finished yet
         self._poll_seconds = 0.0002       # completion is read from host memory; no runtime call while waiting
@@ -531,7 +534,10 @@ class AdamW(Optimizer):
         gathered: Dict[int, list] = {}    # dev -> [descriptor buffer, its address, rows used]
         gathered_means: Dict[int, list] = {}   # dev -> [(first row, rows, row means they need)] of centralized groups
         cen_jobs: Dict[int, list] = {}    # dev -> [(entry, rows, row_len)] of gradients to centralize
-        counted: Dict[int, list] = {}     # dev -> [(state, step count before)] of the tensors under max_grad_norm
+        # dev -> the step counts advanced under max_grad_norm: (state, count before) from the Python loop, (states, status
+        # bytes or None for all, code of the written ones, scalar index of each or None for one step, first such index,
+        # the new steps) from the gatherer
+        counted: Dict[int, list] = {}
         skip_checks = []
 
         for gi, group in enumerate(self.param_groups):
@@ -679,8 +685,8 @@ class AdamW(Optimizer):
         explicit = noise is not None
         work_by_dev = []
         # (a device whose tensors all lack gradients has a descriptor buffer without rows: nothing to launch there)
-        with_rows = {dev for dev, slot in gathered.items() if slot[2]}
-        for dev in sorted(set(plain) | set(resident) | set(streamed) | with_rows):
+        with_rows = [dev for dev, slot in gathered.items() if slot[2]]
+        for dev in sorted({*plain, *resident, *streamed, *with_rows}):
             res, stm = resident.get(dev, []), streamed.get(dev, [])
             lane = plain.get(dev)
             descs = self._plain_descs(dev, lane) if lane is not None else None
