@@ -616,7 +616,8 @@ static int stage_image(rt_handle* h, const Plan& plan, const uint8_t* img, uint6
     }
     // Two regions: the DevScalars sets change with every step, the lists behind them only when the
     // tensors do; what differs from the device copy goes up in one copy.  Sets that travel as kernel
-    // arguments are not uploaded at all, so steps over the same tensors copy nothing.
+    // arguments are not uploaded at all, so steps over the same tensors copy nothing -- while they have at most kSlots
+    // images: three (row means, norm, update) take turns in two slots and are uploaded every time.
     const size_t lists = std::min(plan.off_tensors, plan.bytes);
     const size_t begin = plan.n_sets <= kArgSets ? lists : 0;
     const bool known = s.valid_bytes == plan.bytes && s.valid_from <= begin;
@@ -1007,7 +1008,7 @@ int rt_grad_norm(rt_handle* h, const rt_tensor_desc* descs, uint32_t n, float in
     const uint32_t n_chunks = (uint32_t)(n_whole + n_rest);
     const uint32_t grid = std::min<uint32_t>(kNormPartials, n_chunks);
     if (n_chunks != 0) {
-        // the table goes through a staging slot: the same gradients step after step upload nothing
+        // the table goes through a staging slot: the same gradients step after step upload nothing (see stage_image)
         Plan plan;
         plan.bytes = tab.size() * sizeof(NormEntry);
         h->image.assign((const uint8_t*)tab.data(), (const uint8_t*)tab.data() + plan.bytes);

@@ -1,4 +1,4 @@
-// Host-side helper of AdamW.step for parameter sets with very many tensors: walks one
+// Host-side helper of AdamW.step, for sets of any size: walks one
 // param group and writes the rt_tensor_desc rows of every "plain" tensor (param, gradient
 // and both states contiguous on one GPU, supported dtypes) straight into a caller-owned
 // buffer, advancing state["step"] as adamw.py:177 does.  It does, per tensor, what the Python

@@ -865,9 +865,9 @@ __global__ __launch_bounds__(kThreads) void sr_adamw_link_kernel(const LaunchArg
 }
 
 // ---------------------------------------------------------------------------
-// Generic kernel: the last (partial) chunk of a tensor, debug outputs, gradient
-// centralization.  Full vectors still move as 128-bit accesses; everything else
-// element by element under an index guard.
+// Generic kernel: debug outputs, centralized rows shorter than 8 elements (over the host link: centralized layouts
+// with an fp32 array), and what explicit-noise tensors have beside whole units.  Full vectors still move as
+// 128-bit accesses; everything else element by element under an index guard.
 // ---------------------------------------------------------------------------
 template <int PDT, int GDT, int MDT, int VDT, int NOISE>
 __global__ __launch_bounds__(kThreads) void sr_adamw_generic_kernel(const LaunchArgs a) {

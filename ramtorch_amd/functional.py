@@ -280,6 +280,7 @@ class GatheredMeans:
         self.buf, self.addr, self.rows, self.segments, self.place, self.means = buf, addr, rows, segments, place, None
 
     def __len__(self) -> int:
+        """How many gradients need means from the pass."""
         return int(np.count_nonzero(self.buf["row_mean"][:self.rows]))
 
     def allocate(self, device: int) -> None:
