@@ -1447,7 +1447,7 @@ __device__ __forceinline__ float chunk_sumsq_dt(int dt, uint64_t g_addr, uint64_
 // A lane keeps its sum in fp64 from chunk to chunk and the workgroup reduces once, at the end, so that the
 // four waves never wait for each other between chunks.  17.7 M fp32 elements in 160 ragged gradients
 // 16.6 -> 15.2 us, 218 M in nine 144.6 -> 141.7 us, against a binary search and a reduction with two barriers per chunk.
-// Bound by memory: 6.4 - 6.9 TB/s beyond the caches.
+// Bound by memory: 0.87 GB in 139 us (6.3 TB/s), 32 GB in 4.79 ms (6.7 TB/s).
 // ---------------------------------------------------------------------------
 struct alignas(16) NormEntry {
     uint64_t g;
